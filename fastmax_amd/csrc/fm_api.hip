@@ -1001,7 +1001,8 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
   {
     constexpr int RT = S::RT_KV, NW = S::NW_KV, BM = 32 * RT * NW, BNK = S::BN_KV;
     static_assert(256 % BM == 0 && 256 % BNK == 0, "blocks and stages do not straddle the chunks of the linear mode");
-    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + NW);
+    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + (NW + 3) / 4 * 4) +
+                        (S::KLO ? (size_t)NW * (DP / dense::Policy<DP, T>::KF) * 64 * sizeof(fm_u4) : 0);
     auto kern = dense::dense_dkdv_kernel<DP, T, RT, BNK, NW>;
     FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
     const int nb = (pl.nk + BM - 1) / BM;

@@ -424,3 +424,23 @@ def test_strided_views_with_many_heads_take_the_linear_mode(built, monkeypatch):
     g2 = _ops.backward(qd, kd, vd, o2, den2, god, qk_scale=sc2, qk_argmax=arg2, **kw)
     for name, a, b2 in zip(("o", "dq", "dk", "dv"), got, (o2,) + tuple(g2)):
         assert_close(name, a.float(), b2.float(), 3e-2, atol=1e-6)
+
+
+@pytest.mark.parametrize("d", [32, 36, 64])
+@pytest.mark.parametrize("n", [31, 256, 289])
+@pytest.mark.parametrize("mask", [False, True])
+def test_fp32_contractions_keep_24_bits(ops, d, n, mask):
+    """fp32 contractions run on parts of 3 x 8 bits.  With positive values and weights nothing cancels, so the
+    outputs are as good as their roundings: about sqrt(6 n / 16) of 2^-24 each in the sums (11 at n = 289) on top
+    of a few in the weights.  A product of parts left out would show as 2^-18 or more (64 of these units)."""
+    q, k, v, go = (t.abs() for t in O.seeded_inputs((2, n, d), seed=n + d))
+    v, go = v + 0.1, go + 0.1
+    kw = dict(mask=mask, normalize=True, p=2)
+    print("24 bits", d, n, mask, flush=True)
+    qd, kd, vd, god = (t.cuda() for t in (q, k, v, go))
+    o, den, sc, arg = ops.forward(qd, kd, vd, **kw)
+    dv = ops.backward(qd, kd, vd, o, den, god, qk_scale=sc, qk_argmax=arg, **kw)[2]
+    ro, _, _, rdv = O.dense_truth(q.double(), k.double(), v.double(), go.double(), **kw)
+    for name, got, ref in (("o", o, ro), ("dv", dv, rdv)):
+        err = ((got.cpu().double() - ref.double()).norm() / ref.double().norm()).item()
+        assert err < 16 * 2.0 ** -24, f"{name}: {err / 2.0 ** -24:.1f} units of 2^-24"
