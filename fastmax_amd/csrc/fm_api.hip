@@ -14,6 +14,7 @@
 #include "fastmax_amd.h"
 #include "fm_apply.h"
 #include "fm_backward.h"
+#include "fm_cut.h"
 #include "fm_decode.h"
 #include "fm_dense.h"
 #include "fm_forward.h"
@@ -107,6 +108,7 @@ struct Plan {
   bool lin;            // dense kernels in linear mode (p = 1, long sequences): chunk states of (dp + 1) rows in
                        // the workspace, lslots of them per head, one per lchunk positions
   int lchunk, lslots, ldp;
+  bool cut;            // fp32, d = 64, p = 2: state products on the bf16 instruction with cut operands (fm_cut.h)
   bool split;          // causal p = 1 with few heads: the chunks of a head are built side by side as partial
                        // states and a prefix pass over the chunks makes the causal states of them
   size_t scratch_bytes;   // per head: where the fp32 partial states of a split build go when the
@@ -150,6 +152,10 @@ int linear_min_heads(const fastmax_desc* ds) {
   return ds->dtype == FASTMAX_BF16 ? FM_LINEAR_MIN_HEADS_BF16 : FM_LINEAR_MIN_HEADS;
 }
 bool use_linear_scan(const fastmax_desc* ds, const Plan& pl);
+
+#ifndef FM_CUT_MIN_BLOCKS
+#define FM_CUT_MIN_BLOCKS 256
+#endif
 
 // Dense score tiles cost 2 n d flop per token under the mask (4 n d without it), the moment form about
 // 2.1 d^3 (p = 2) whatever n is: below these key counts the dense kernels are the faster ones (measured,
@@ -209,7 +215,7 @@ Plan make_plan(const fastmax_desc* ds, int pass, bool plain = true, bool allow_d
     // no states: the workspace holds the per-head scalars only (and c_i, normalisation partials)
     pl.rtw = pl.gsplit = pl.nslots = pl.nparts = 1;
     pl.zlen = pl.chunk = 0;
-    pl.scan = pl.rowpass = pl.split = false;
+    pl.scan = pl.rowpass = pl.split = pl.cut = false;
     pl.scratch_bytes = pl.per_head_bytes = 0;
     pl.state_floats = 0;
     size_t fx = align256((size_t)2 * pl.bh * sizeof(float)) + align256((size_t)2 * pl.bh * sizeof(int));
@@ -284,6 +290,9 @@ Plan make_plan(const fastmax_desc* ds, int pass, bool plain = true, bool allow_d
   pl.scratch_bytes = (pl.split && ds->dtype == FASTMAX_BF16)
                          ? (size_t)pl.nslots * state_floats_for(pl.d, pl.p2) * sizeof(float) : 0;
   pl.per_head_bytes += pl.scratch_bytes;
+  // (one block of eight waves per CU and 256 positions: with fewer blocks than CUs the smaller blocks of the fp32 kernels
+  // spread a head over twice as many)
+  pl.cut = pl.p2 && pl.d == 64 && ds->dtype == FASTMAX_F32 && (int64_t)pl.bh * ((pl.n + cut::TB - 1) / cut::TB) >= FM_CUT_MIN_BLOCKS;
   pl.rowpass = !pl.p2 && !pl.masked && pl.d == 64 && pl.ratio == 1 && pl.n >= 32 && pl.plain && pl.nq == pl.nk;
   return pl;
 }
@@ -472,6 +481,8 @@ constexpr bool kBf16Mfma = false;
 template <>
 constexpr bool kBf16Mfma<bf16_t> = true;
 
+int allow_lds(const void* kernel, size_t bytes);
+
 // State of (X, Y, extra) over n positions of `heads` heads (X.h0 is the first of them).
 template <int D, class T>
 int launch_build(const Plan& pl, int heads, int n, const Rows<const T>& X, const Rows<const T>& Y,
@@ -494,11 +505,21 @@ int launch_build(const Plan& pl, int heads, int n, const Rows<const T>& X, const
     return launch_status("build_kernel (chunks side by side)");
   }
   const dim3 grid(pl.gsplit, heads, pl.nparts);
+  // (a head is three blocks of eight waves here and six of four in the fp32 kernel: with fewer blocks than CUs the
+  // latter walk the sequence on twice as many CUs)
+  bool cut_build = false;
+  if constexpr (D == 64 && !kBf16Mfma<T>) cut_build = pl.cut && 3 * pl.bhkv * pl.nparts >= FM_CUT_MIN_BLOCKS;   // (whatever the head batch)
 #define FM_BUILD(RTW)                                                                            \
   build_kernel<D, T, RTW, kBf16Mfma<T>><<<grid, 256, 0, stream>>>(X, Y, xscale, yden, ew, state, \
                                                     n, pl.chunk, pl.nslots, pl.masked, reverse, \
                                                     pl.p2, pl.zlen)
-  if (pl.rtw == 1) {
+  if (cut_build) {
+    if constexpr (D == 64 && !kBf16Mfma<T>) {
+      FM_TRY(allow_lds(reinterpret_cast<const void*>(cut::cut_build_kernel), cut::BUILD_LDS));
+      cut::cut_build_kernel<<<dim3(3, heads, pl.nparts), cut::NT, cut::BUILD_LDS, stream>>>(
+          X, Y, xscale, yden, ew, state, n, pl.chunk, pl.nslots, pl.masked, reverse, pl.zlen);
+    }
+  } else if (pl.rtw == 1) {
     FM_BUILD(1);
   } else if constexpr (D == 64) {
     FM_BUILD(3);
@@ -541,6 +562,27 @@ inline void finish_state_both(const Plan& pl, int heads, float* state, hipStream
   if (pl.nparts > 1)
     state_accumulate_kernel<<<dim3((unsigned)((ss / 4 + 255) / 256), heads), 256, 0, stream>>>(
         state, (int64_t)pl.nslots * ss, state, pl.nslots, pl.nparts, ss, 0);
+}
+
+// The tiles of every query's own chunk, added to the state products that the kernels of fm_cut.h left in the outputs.
+template <int DP, class T>
+int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v, T* o,
+                     float* den, int64_t den_stride, const float* scale, float* kstate, hipStream_t stream, int add = 0);
+template <int DP, class T>
+int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v,
+                      const T* o, const float* den, int64_t den_stride, const T* go, T* dq, T* dk, T* dv,
+                      const float* scale, float* cvec_w, float* rpart, float* kstate, float* qstate, int* nbq_out,
+                      int* nbk_out, hipStream_t stream, int add = 0);
+Plan own_chunk_plan(const Plan& pl) {
+  Plan cp = pl;
+  cp.lin = false;
+  cp.lchunk = pl.chunk;
+  cp.lslots = pl.nslots;
+  return cp;
+}
+// 256-token blocks of the kernels of fm_cut.h for query-side rows
+int cut_blocks_q(const Plan& pl) {
+  return pl.masked ? (pl.nk + cut::TB - 1) / cut::TB - pl.off / cut::TB : (pl.nq + cut::TB - 1) / cut::TB;
 }
 
 template <int D, class T>
@@ -629,6 +671,15 @@ int forward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const 
         apply_kernel_bf<D, 0><<<agrid, 256, 0, stream>>>(
             qr, kr, vr, scale + h0, scale + bh + kv0, kNoScalars, state, pl.nslots, orow, dn, nown, pl.chunk,
             pl.masked, pl.p2, ds->a0, ds->a1, pl.p2 ? ds->a2 : 0.f, 1, ratio);
+      } else if (D == 64 && pl.cut) {
+        if constexpr (D == 64) {
+          if (!pl.masked || pl.nslots > 1) {
+            auto kern = cut::cut_apply_kernel<0>;
+            FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), cut::APPLY_LDS));
+            kern<<<dim3(cut_blocks_q(pl), heads), cut::NT, cut::APPLY_LDS, stream>>>(
+                qr, scale + h0, state, pl.nslots, orow, dn, nown, pl.chunk, pl.masked, ds->a0, ds->a1, ds->a2, 1, ratio);
+          }
+        }
       } else {
         apply_kernel<D, T, 0><<<agrid, 256, 0, stream>>>(
             qr, kr, vr, scale + h0, scale + bh + kv0, kNoScalars, state, pl.nslots, orow, dn, nown, pl.chunk,
@@ -636,6 +687,10 @@ int forward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const 
       }
     }
     FM_TRY(launch_status("fwd_apply_kernel"));
+  }
+  if constexpr (D == 64 && !kBf16Mfma<T>) {
+    if (pl.cut && pl.masked)
+      return dense_forward_dp<D, T>(ds, own_chunk_plan(pl), L, q, k, v, o, den, den_stride, scale, nullptr, stream, 1);
   }
   return FASTMAX_OK;
 }
@@ -738,6 +793,7 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
   // positions the own rows of the query-side / key-side kernels run over, and where the query-side
   // rows start (the queries sit at positions off .. nk-1 under the mask)
   const int nown_q = pl.masked ? nk : nq, nown_k = nk, off = pl.off;
+  const int nbq_cut = cut_blocks_q(pl);
   for (int h0 = 0; h0 < bh; h0 += hb) {
     const int heads = bh - h0 < hb ? bh - h0 : hb;
     const int kv0 = h0 / ratio;                // first key/value head of the batch
@@ -826,6 +882,13 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
         grad_kernel_bf<D, 0><<<grid, 256, 0, stream>>>(
             qr, gr, dn, cv, kr, vr, kNoScalars, scale + h0, scale + bh + kv0, stS, pl.nslots, dqr,
             rpart + (int64_t)h0 * pl.nblk_q, nown_q, pl.chunk, pl.masked, pl.p2, ds->a1, a2, 1, ratio);
+      } else if (D == 64 && pl.cut) {
+        if constexpr (D == 64) {
+          if (!pl.masked || pl.nslots > 1)
+            cut::cut_grad_kernel<0><<<dim3(nbq_cut, heads), cut::NT, 0, stream>>>(
+                qr, gr, dn, cv, scale + h0, stS, pl.nslots, dqr, rpart + (int64_t)h0 * nbq_cut, nown_q, pl.chunk, pl.masked,
+                ds->a1, a2, 1, ratio);
+        }
       } else {
         grad_kernel<D, T, 0><<<grid, 256, 0, stream>>>(
             qr, gr, dn, cv, kr, vr, kNoScalars, scale + h0, scale + bh + kv0, stS, pl.nslots, dqr,
@@ -834,12 +897,20 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
     }
     FM_TRY(launch_status("grad_kernel (dq)"));
     const dim3 kgrid(pl.nblk_k, heads);
+    const dim3 ckgrid((nk + cut::TB - 1) / cut::TB, heads);
     {
       ScopedKernel sk(FASTMAX_K_BWD_DK, stream);
       if constexpr (kBf16Mfma<T>) {
         grad_kernel_bf<D, 1><<<kgrid, 256, 0, stream>>>(
             kr, vr, kNoScalars, cv, qr, gr, dn, scale + bh + kv0, scale + h0, stR, pl.nslots, dk_q,
             rpart_k + (int64_t)h0 * pl.nblk_k, nown_k, pl.chunk, pl.masked, pl.p2, ds->a1, a2, ratio, 1);
+      } else if (D == 64 && pl.cut) {
+        if constexpr (D == 64) {
+          if (!pl.masked || pl.nslots > 1)
+            cut::cut_grad_kernel<1><<<ckgrid, cut::NT, 0, stream>>>(
+                kr, vr, kNoScalars, cv, scale + bh + kv0, stR, pl.nslots, dk_q,
+                rpart + (int64_t)bh * nbq_cut + (int64_t)h0 * ckgrid.x, nown_k, pl.chunk, pl.masked, ds->a1, a2, ratio, 1);
+        }
       } else {
         grad_kernel<D, T, 1><<<kgrid, 256, 0, stream>>>(
             kr, vr, kNoScalars, cv, qr, gr, dn, scale + bh + kv0, scale + h0, stR, pl.nslots, dk_q,
@@ -853,6 +924,16 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
         apply_kernel_bf<D, 1><<<kgrid, 256, 0, stream>>>(
             kr, qr, gr, scale + bh + kv0, scale + h0, dn, stR, pl.nslots, dv_q, RowScalarsOut{nullptr, 0, 0}, nown_k,
             pl.chunk, pl.masked, pl.p2, ds->a0, ds->a1, a2, ratio, 1);
+      } else if (D == 64 && pl.cut) {
+        if constexpr (D == 64) {
+          if (!pl.masked || pl.nslots > 1) {
+            auto kern = cut::cut_apply_kernel<1>;
+            FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), cut::APPLY_LDS));
+            kern<<<ckgrid, cut::NT, cut::APPLY_LDS, stream>>>(kr, scale + bh + kv0, stR, pl.nslots, dv_q,
+                                                              RowScalarsOut{nullptr, 0, 0}, nown_k, pl.chunk, pl.masked,
+                                                              ds->a0, ds->a1, a2, ratio, 1);
+          }
+        }
       } else {
         apply_kernel<D, T, 1><<<kgrid, 256, 0, stream>>>(
             kr, qr, gr, scale + bh + kv0, scale + h0, dn, stR, pl.nslots, dv_q, RowScalarsOut{nullptr, 0, 0}, nown_k,
@@ -860,13 +941,25 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
       }
     }
     FM_TRY(launch_status("apply_kernel (dv)"));
-    if (ratio > 1) {
+    if (ratio > 1 && !(pl.cut && pl.masked && pl.nslots < 2)) {
       const int64_t per_head = (int64_t)nk * D;
       const dim3 sgrid((unsigned)((per_head / 4 + 255) / 256), heads / ratio);
       group_sum_kernel<T><<<sgrid, 256, 0, stream>>>(dk_tmp, mk_rows(dk, L.dk, kv0), nk, D, ratio);
       group_sum_kernel<T><<<sgrid, 256, 0, stream>>>(dv_tmp, mk_rows(dv, L.dv, kv0), nk, D, ratio);
       FM_TRY(launch_status("group_sum_kernel"));
     }
+  }
+  // normalisation partials per query head and per key/value head
+  int nbq = pl.nblk_q, nbk = pl.nblk_k * ratio;
+  if (pl.cut) {
+    nbq = nbq_cut;
+    nbk = (nk + cut::TB - 1) / cut::TB * ratio;
+    if constexpr (D == 64 && !kBf16Mfma<T>) {
+      if (pl.masked)
+        FM_TRY((dense_backward_dp<D, T>(ds, own_chunk_plan(pl), L, q, k, v, o, den, den_stride, go, dq, dk, dv, scale, cvec,
+                                        rpart, nullptr, nullptr, &nbq, &nbk, stream, 1)));
+    }
+    rpart_k = rpart + (int64_t)bh * nbq;
   }
   if (ds->normalize && pl.rowpass) {
     // one partial per row block of the dq pass; sum_j dk_hat_j . k_hat_j is the same number
@@ -879,8 +972,8 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
   } else if (ds->normalize) {
     ScopedKernel sk(FASTMAX_K_NORM_FIX, stream);
     norm_fix_kernel<T><<<bh + bhkv, D, 0, stream>>>(
-        NormFixSide<T>{mk_rows(dq, L.dq), mk_rows(q, L.q), scale, arg, rpart, bh, pl.nblk_q, nq},
-        NormFixSide<T>{mk_rows(dk, L.dk), mk_rows(k, L.k), scale + bh, arg + bh, rpart_k, bhkv, pl.nblk_k * ratio, nk}, D,
+        NormFixSide<T>{mk_rows(dq, L.dq), mk_rows(q, L.q), scale, arg, rpart, bh, nbq, nq},
+        NormFixSide<T>{mk_rows(dk, L.dk), mk_rows(k, L.k), scale + bh, arg + bh, rpart_k, bhkv, nbk, nk}, D,
         ds->lim);
     FM_TRY(launch_status("norm_fix_kernel"));
   }
@@ -925,7 +1018,7 @@ int dense_lin_states(const fastmax_desc* ds, const Plan& pl, const Layout& L, co
 
 template <int DP, class T>
 int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v, T* o,
-                     float* den, int64_t den_stride, const float* scale, float* kstate, hipStream_t stream) {
+                     float* den, int64_t den_stride, const float* scale, float* kstate, hipStream_t stream, int add) {
   using S = dense::Shape<DP, T>;
   constexpr int RT = S::RT_FWD, BN = S::BN, NW = S::NW_FWD, BM = 32 * RT * NW;
   static_assert(256 % BM == 0 && 256 % BN == 0, "blocks and stages do not straddle the chunks of the linear mode");
@@ -941,7 +1034,7 @@ int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, co
                                                scale + pl.bh, mk_rows(o, L.o, 0, pl.off),
                                                mk_scalars(den, pl.nq, den_stride, 0, pl.off), npos, pl.nk, ds->d,
                                                pl.masked, ds->a0, ds->a1, pl.p2 ? ds->a2 : 0.f, pl.ratio,
-                                               pl.lin ? kstate : nullptr, pl.lchunk, pl.lslots);
+                                               pl.lin ? kstate : nullptr, pl.lchunk, pl.lslots, add);
   return launch_status("dense_fwd_kernel");
 }
 
@@ -964,11 +1057,13 @@ template <int DP, class T>
 int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v,
                       const T* o, const float* den, int64_t den_stride, const T* go, T* dq, T* dk, T* dv,
                       const float* scale, float* cvec_w, float* rpart, float* kstate, float* qstate, int* nbq_out,
-                      int* nbk_out, hipStream_t stream) {
+                      int* nbk_out, hipStream_t stream, int add) {
   // c_i = grad_out_i . out_i / den_i: the dq kernel forms it from rows it holds anyway and leaves it in cvec for the
   // dk / dv kernel -- except in the linear mode, whose query-side states need it before any of them runs
-  const bool prep_in_dq = !pl.lin;
-  if (!prep_in_dq) FM_TRY((launch_bwd_prep<T>(pl, L, go, o, den, den_stride, cvec_w, stream)));
+  // (add: the states of the other chunks needed it, too)
+  const bool prep_in_dq = !pl.lin && !add;
+  const int lchunk = pl.lchunk, lslots = pl.lslots;
+  if (pl.lin) FM_TRY((launch_bwd_prep<T>(pl, L, go, o, den, den_stride, cvec_w, stream)));
   const float* cvec = cvec_w;
   using S = dense::Shape<DP, T>;
   constexpr int BN = S::BN;
@@ -986,7 +1081,7 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
   {
     constexpr int RT = S::RT_DQ, NW = S::NW_DQ, BM = 32 * RT * NW;
     static_assert(256 % BM == 0, "blocks do not straddle the chunks of the linear mode");
-    const size_t smem = dense::Lds<DP, T, BN>::bytes(2, 1, NW);
+    const size_t smem = dense::Lds<DP, T, BN>::bytes(2, 1, 2 * NW);
     auto kern = dense::dense_dq_kernel<DP, T, RT, BN, NW>;
     FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
     const int nb = (npos + BM - 1) / BM - pl.off / BM;
@@ -994,15 +1089,15 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
     ScopedKernel sk(FASTMAX_K_BWD_DQ, stream);
     kern<<<dim3(pl.bh, nb), 64 * NW, smem, stream>>>(qr, gr, dn, cv, kr, vr, scale, scale + pl.bh, mk_rows(dq, L.dq, 0, pl.off), rq,
                                                  npos, pl.nk, ds->d, pl.masked, pl.p2 && a2 != 0.f, ds->a1, a2, pl.ratio,
-                                                 ksl, pl.lchunk, pl.lslots, mk_rows(o, L.o, 0, pl.off),
-                                                 prep_in_dq ? mk_scalars<float>(cvec_w, pl.nq, 1, 0, pl.off) : RowScalarsOut{nullptr, 0, 0});
+                                                 ksl, lchunk, lslots, mk_rows(o, L.o, 0, pl.off),
+                                                 prep_in_dq ? mk_scalars<float>(cvec_w, pl.nq, 1, 0, pl.off) : RowScalarsOut{nullptr, 0, 0}, add);
     FM_TRY(launch_status("dense_dq_kernel"));
   }
   {
     constexpr int RT = S::RT_KV, NW = S::NW_KV, BM = 32 * RT * NW, BNK = S::BN_KV;
     static_assert(256 % BM == 0 && 256 % BNK == 0, "blocks and stages do not straddle the chunks of the linear mode");
-    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + (NW + 3) / 4 * 4) +
-                        (S::KLO ? (size_t)NW * (DP / dense::Policy<DP, T>::KF) * 64 * sizeof(fm_u4) : 0);
+    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + 2 * ((NW + 3) / 4 * 4)) +
+                        (S::KLO ? (size_t)NW * (DP / dense::Policy<DP, T>::KF + 1) * 64 * sizeof(fm_u4) : 0);
     auto kern = dense::dense_dkdv_kernel<DP, T, RT, BNK, NW>;
     FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
     const int nb = (pl.nk + BM - 1) / BM;
@@ -1011,7 +1106,7 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
     ScopedKernel sk(FASTMAX_K_BWD_DK, stream);
     kern<<<dim3(pl.bhkv, nb), 64 * NW, smem, stream>>>(kr, vr, qr, gr, dn, cv, scale, scale + pl.bh, mk_rows(dk, L.dk),
                                                    mk_rows(dv, L.dv), rk, npos, pl.nk, ds->d, pl.masked, ds->a0, ds->a1,
-                                                   a2, pl.ratio, qsl, pl.lchunk, pl.lslots);
+                                                   a2, pl.ratio, qsl, lchunk, lslots, add);
     FM_TRY(launch_status("dense_dkdv_kernel"));
   }
   return FASTMAX_OK;
