@@ -147,7 +147,7 @@ struct Mma<float> {
 // Six v_mfma_f32_32x32x16_bf16 take ~200 cycles where eight v_mfma_f32_32x32x2f32 take 512.  The parts of streamed
 // rows are formed once per block on their way into LDS (three planes per row), those of own rows once per
 // wave; only the weights are cut up per tile.
-// Measured (forward + backward, fp32, causal, 512 heads x 1000 x 32): 1403 us with the fp32 instruction, 1037 so;
+// Measured (forward + backward, fp32, causal, 512 heads x 1000 x 32): 1403 us with the fp32 instruction, 1047 so;
 // forward only, unmasked, 512 heads x 1000 x 64: 1164 and 794.  The error against 64 bits falls by 10 to 30 %.
 struct SplitFrag {
   fm_u4 p[3];
