@@ -444,3 +444,10 @@ def test_fp32_contractions_keep_24_bits(ops, d, n, mask):
     for name, got, ref in (("o", o, ro), ("dv", dv, rdv)):
         err = ((got.cpu().double() - ref.double()).norm() / ref.double().norm()).item()
         assert err < 16 * 2.0 ** -24, f"{name}: {err / 2.0 ** -24:.1f} units of 2^-24"
+
+
+@pytest.mark.parametrize("d", [32, 48, 64])
+@pytest.mark.parametrize("mask", [False, True])
+def test_many_heads_fp32(ops, d, mask):
+    # (enough 256-row blocks to fill the chip: the eight-wave form of the kernels; the tests above run the four-wave one)
+    run_case(ops, (130, 289, d), seed=d, mask=mask, normalize=True, p=2)
