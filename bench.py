@@ -177,17 +177,6 @@ def dense_linear_mode(cfg: dict) -> bool:
     return cfg["p"] == 1 and cfg["N"] > (1024 if cfg["mask"] else 512)
 
 
-def runs_on_cut_operands(cfg: dict, bh: int, dense: bool) -> bool:
-    """Whether an fp32 workload's contractions run on the bf16 matrix instruction with operands cut into three parts
-    (dense kernels up to 64 channels; moment kernels at d = 64, p = 2 with enough heads: fm_api.hip::make_plan).  The
-    executed counts stay those of the fp32 contractions; their peak is then a sixth of the bf16 one."""
-    if cfg["dtype"] != "f32":
-        return False
-    if dense:
-        return cfg["D"] <= 64
-    return cfg["D"] == 64 and cfg["p"] == 2 and bh * -(-cfg["N"] // 256) >= 256
-
-
 def executed_dense_flops(cfg: dict, bh: int) -> dict:
     """Flops of the matrix instructions the dense score-tile kernels issue (fm_dense.h): per pair of a
     32-row own tile and a 32-row streamed tile one score contraction over the padded head dimension and one
@@ -412,8 +401,6 @@ def measure(name: str, args, full: bool) -> dict:
     fl = algorithmic_flops(D, cfg["p"])
     token_heads = bh * N
     peak = PEAK_TFLOPS[cfg["dtype"]]
-    if runs_on_cut_operands(cfg, bh, dense):
-        peak = PEAK_TFLOPS["bf16"] / 6   # six bf16 products stand for one fp32 product
     kernels = {}
     for i, kname in enumerate(_cabi.KERNEL_NAMES):
         if kt.launches[i]:
@@ -466,8 +453,7 @@ def measure(name: str, args, full: bool) -> dict:
     dom = max(algo, key=lambda kn: kernels.get(kn, {}).get("ms_per_step", 0.0))
     dom_ms = kernels[dom]["ms_per_step"]
     launches = kernels[dom]["launches_per_step"]
-    # fp32 inputs run every contraction on v_mfma_f32_32x32x2f32 or, with cut operands, as six bf16 products on
-    # v_mfma_f32_32x32x16_bf16, which bf16 inputs run on anyway.
+    # fp32 inputs run every contraction on v_mfma_f32_32x32x2f32, bf16 inputs on v_mfma_f32_32x32x16_bf16.
     # frac is the executed rate over the peak (at most 1, and what SQ_VALU_MFMA_BUSY_CYCLES over the kernel's
     # duration shows); algorithmic_frac prices the same time with the reference-form count and can exceed 1.
     roofline = None

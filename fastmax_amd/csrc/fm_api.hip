@@ -14,7 +14,6 @@
 #include "fastmax_amd.h"
 #include "fm_apply.h"
 #include "fm_backward.h"
-#include "fm_cut.h"
 #include "fm_decode.h"
 #include "fm_dense.h"
 #include "fm_forward.h"
@@ -108,7 +107,6 @@ struct Plan {
   bool lin;            // dense kernels in linear mode (p = 1, long sequences): chunk states of (dp + 1) rows in
                        // the workspace, lslots of them per head, one per lchunk positions
   int lchunk, lslots, ldp;
-  bool cut;            // fp32, d = 64, p = 2: state products on the bf16 instruction with cut operands (fm_cut.h)
   bool split;          // causal p = 1 with few heads: the chunks of a head are built side by side as partial
                        // states and a prefix pass over the chunks makes the causal states of them
   size_t scratch_bytes;   // per head: where the fp32 partial states of a split build go when the
@@ -152,10 +150,6 @@ int linear_min_heads(const fastmax_desc* ds) {
   return ds->dtype == FASTMAX_BF16 ? FM_LINEAR_MIN_HEADS_BF16 : FM_LINEAR_MIN_HEADS;
 }
 bool use_linear_scan(const fastmax_desc* ds, const Plan& pl);
-
-#ifndef FM_CUT_MIN_BLOCKS
-#define FM_CUT_MIN_BLOCKS 256
-#endif
 
 // Dense score tiles cost 2 n d flop per token under the mask (4 n d without it), the moment form about
 // 2.1 d^3 (p = 2) whatever n is: below these key counts the dense kernels are the faster ones (measured,
@@ -215,7 +209,7 @@ Plan make_plan(const fastmax_desc* ds, int pass, bool plain = true, bool allow_d
     // no states: the workspace holds the per-head scalars only (and c_i, normalisation partials)
     pl.rtw = pl.gsplit = pl.nslots = pl.nparts = 1;
     pl.zlen = pl.chunk = 0;
-    pl.scan = pl.rowpass = pl.split = pl.cut = false;
+    pl.scan = pl.rowpass = pl.split = false;
     pl.scratch_bytes = pl.per_head_bytes = 0;
     pl.state_floats = 0;
     size_t fx = align256((size_t)2 * pl.bh * sizeof(float)) + align256((size_t)2 * pl.bh * sizeof(int));
@@ -290,9 +284,6 @@ Plan make_plan(const fastmax_desc* ds, int pass, bool plain = true, bool allow_d
   pl.scratch_bytes = (pl.split && ds->dtype == FASTMAX_BF16)
                          ? (size_t)pl.nslots * state_floats_for(pl.d, pl.p2) * sizeof(float) : 0;
   pl.per_head_bytes += pl.scratch_bytes;
-  // (one block of eight waves per CU and 256 positions: with fewer blocks than CUs the smaller blocks of the fp32 kernels
-  // spread a head over twice as many)
-  pl.cut = pl.p2 && pl.d == 64 && ds->dtype == FASTMAX_F32 && (int64_t)pl.bh * ((pl.n + cut::TB - 1) / cut::TB) >= FM_CUT_MIN_BLOCKS;
   pl.rowpass = !pl.p2 && !pl.masked && pl.d == 64 && pl.ratio == 1 && pl.n >= 32 && pl.plain && pl.nq == pl.nk;
   return pl;
 }
@@ -481,8 +472,6 @@ constexpr bool kBf16Mfma = false;
 template <>
 constexpr bool kBf16Mfma<bf16_t> = true;
 
-int allow_lds(const void* kernel, size_t bytes);
-
 // State of (X, Y, extra) over n positions of `heads` heads (X.h0 is the first of them).
 template <int D, class T>
 int launch_build(const Plan& pl, int heads, int n, const Rows<const T>& X, const Rows<const T>& Y,
@@ -505,21 +494,11 @@ int launch_build(const Plan& pl, int heads, int n, const Rows<const T>& X, const
     return launch_status("build_kernel (chunks side by side)");
   }
   const dim3 grid(pl.gsplit, heads, pl.nparts);
-  // (a head is three blocks of eight waves here and six of four in the fp32 kernel: with fewer blocks than CUs the
-  // latter walk the sequence on twice as many CUs)
-  bool cut_build = false;
-  if constexpr (D == 64 && !kBf16Mfma<T>) cut_build = pl.cut && 3 * pl.bhkv * pl.nparts >= FM_CUT_MIN_BLOCKS;   // (whatever the head batch)
 #define FM_BUILD(RTW)                                                                            \
   build_kernel<D, T, RTW, kBf16Mfma<T>><<<grid, 256, 0, stream>>>(X, Y, xscale, yden, ew, state, \
                                                     n, pl.chunk, pl.nslots, pl.masked, reverse, \
                                                     pl.p2, pl.zlen)
-  if (cut_build) {
-    if constexpr (D == 64 && !kBf16Mfma<T>) {
-      FM_TRY(allow_lds(reinterpret_cast<const void*>(cut::cut_build_kernel), cut::BUILD_LDS));
-      cut::cut_build_kernel<<<dim3(3, heads, pl.nparts), cut::NT, cut::BUILD_LDS, stream>>>(
-          X, Y, xscale, yden, ew, state, n, pl.chunk, pl.nslots, pl.masked, reverse, pl.zlen);
-    }
-  } else if (pl.rtw == 1) {
+  if (pl.rtw == 1) {
     FM_BUILD(1);
   } else if constexpr (D == 64) {
     FM_BUILD(3);
@@ -562,27 +541,6 @@ inline void finish_state_both(const Plan& pl, int heads, float* state, hipStream
   if (pl.nparts > 1)
     state_accumulate_kernel<<<dim3((unsigned)((ss / 4 + 255) / 256), heads), 256, 0, stream>>>(
         state, (int64_t)pl.nslots * ss, state, pl.nslots, pl.nparts, ss, 0);
-}
-
-// The tiles of every query's own chunk, added to the state products that the kernels of fm_cut.h left in the outputs.
-template <int DP, class T>
-int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v, T* o,
-                     float* den, int64_t den_stride, const float* scale, float* kstate, hipStream_t stream, int add = 0);
-template <int DP, class T>
-int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v,
-                      const T* o, const float* den, int64_t den_stride, const T* go, T* dq, T* dk, T* dv,
-                      const float* scale, float* cvec_w, float* rpart, float* kstate, float* qstate, int* nbq_out,
-                      int* nbk_out, hipStream_t stream, int add = 0);
-Plan own_chunk_plan(const Plan& pl) {
-  Plan cp = pl;
-  cp.lin = false;
-  cp.lchunk = pl.chunk;
-  cp.lslots = pl.nslots;
-  return cp;
-}
-// 256-token blocks of the kernels of fm_cut.h for query-side rows
-int cut_blocks_q(const Plan& pl) {
-  return pl.masked ? (pl.nk + cut::TB - 1) / cut::TB - pl.off / cut::TB : (pl.nq + cut::TB - 1) / cut::TB;
 }
 
 template <int D, class T>
@@ -671,15 +629,6 @@ int forward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const 
         apply_kernel_bf<D, 0><<<agrid, 256, 0, stream>>>(
             qr, kr, vr, scale + h0, scale + bh + kv0, kNoScalars, state, pl.nslots, orow, dn, nown, pl.chunk,
             pl.masked, pl.p2, ds->a0, ds->a1, pl.p2 ? ds->a2 : 0.f, 1, ratio);
-      } else if (D == 64 && pl.cut) {
-        if constexpr (D == 64) {
-          if (!pl.masked || pl.nslots > 1) {
-            auto kern = cut::cut_apply_kernel<0>;
-            FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), cut::APPLY_LDS));
-            kern<<<dim3(cut_blocks_q(pl), heads), cut::NT, cut::APPLY_LDS, stream>>>(
-                qr, scale + h0, state, pl.nslots, orow, dn, nown, pl.chunk, pl.masked, ds->a0, ds->a1, ds->a2, 1, ratio);
-          }
-        }
       } else {
         apply_kernel<D, T, 0><<<agrid, 256, 0, stream>>>(
             qr, kr, vr, scale + h0, scale + bh + kv0, kNoScalars, state, pl.nslots, orow, dn, nown, pl.chunk,
@@ -687,10 +636,6 @@ int forward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const 
       }
     }
     FM_TRY(launch_status("fwd_apply_kernel"));
-  }
-  if constexpr (D == 64 && !kBf16Mfma<T>) {
-    if (pl.cut && pl.masked)
-      return dense_forward_dp<D, T>(ds, own_chunk_plan(pl), L, q, k, v, o, den, den_stride, scale, nullptr, stream, 1);
   }
   return FASTMAX_OK;
 }
@@ -793,7 +738,6 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
   // positions the own rows of the query-side / key-side kernels run over, and where the query-side
   // rows start (the queries sit at positions off .. nk-1 under the mask)
   const int nown_q = pl.masked ? nk : nq, nown_k = nk, off = pl.off;
-  const int nbq_cut = cut_blocks_q(pl);
   for (int h0 = 0; h0 < bh; h0 += hb) {
     const int heads = bh - h0 < hb ? bh - h0 : hb;
     const int kv0 = h0 / ratio;                // first key/value head of the batch
@@ -882,13 +826,6 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
         grad_kernel_bf<D, 0><<<grid, 256, 0, stream>>>(
             qr, gr, dn, cv, kr, vr, kNoScalars, scale + h0, scale + bh + kv0, stS, pl.nslots, dqr,
             rpart + (int64_t)h0 * pl.nblk_q, nown_q, pl.chunk, pl.masked, pl.p2, ds->a1, a2, 1, ratio);
-      } else if (D == 64 && pl.cut) {
-        if constexpr (D == 64) {
-          if (!pl.masked || pl.nslots > 1)
-            cut::cut_grad_kernel<0><<<dim3(nbq_cut, heads), cut::NT, 0, stream>>>(
-                qr, gr, dn, cv, scale + h0, stS, pl.nslots, dqr, rpart + (int64_t)h0 * nbq_cut, nown_q, pl.chunk, pl.masked,
-                ds->a1, a2, 1, ratio);
-        }
       } else {
         grad_kernel<D, T, 0><<<grid, 256, 0, stream>>>(
             qr, gr, dn, cv, kr, vr, kNoScalars, scale + h0, scale + bh + kv0, stS, pl.nslots, dqr,
@@ -897,20 +834,12 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
     }
     FM_TRY(launch_status("grad_kernel (dq)"));
     const dim3 kgrid(pl.nblk_k, heads);
-    const dim3 ckgrid((nk + cut::TB - 1) / cut::TB, heads);
     {
       ScopedKernel sk(FASTMAX_K_BWD_DK, stream);
       if constexpr (kBf16Mfma<T>) {
         grad_kernel_bf<D, 1><<<kgrid, 256, 0, stream>>>(
             kr, vr, kNoScalars, cv, qr, gr, dn, scale + bh + kv0, scale + h0, stR, pl.nslots, dk_q,
             rpart_k + (int64_t)h0 * pl.nblk_k, nown_k, pl.chunk, pl.masked, pl.p2, ds->a1, a2, ratio, 1);
-      } else if (D == 64 && pl.cut) {
-        if constexpr (D == 64) {
-          if (!pl.masked || pl.nslots > 1)
-            cut::cut_grad_kernel<1><<<ckgrid, cut::NT, 0, stream>>>(
-                kr, vr, kNoScalars, cv, scale + bh + kv0, stR, pl.nslots, dk_q,
-                rpart + (int64_t)bh * nbq_cut + (int64_t)h0 * ckgrid.x, nown_k, pl.chunk, pl.masked, ds->a1, a2, ratio, 1);
-        }
       } else {
         grad_kernel<D, T, 1><<<kgrid, 256, 0, stream>>>(
             kr, vr, kNoScalars, cv, qr, gr, dn, scale + bh + kv0, scale + h0, stR, pl.nslots, dk_q,
@@ -924,16 +853,6 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
         apply_kernel_bf<D, 1><<<kgrid, 256, 0, stream>>>(
             kr, qr, gr, scale + bh + kv0, scale + h0, dn, stR, pl.nslots, dv_q, RowScalarsOut{nullptr, 0, 0}, nown_k,
             pl.chunk, pl.masked, pl.p2, ds->a0, ds->a1, a2, ratio, 1);
-      } else if (D == 64 && pl.cut) {
-        if constexpr (D == 64) {
-          if (!pl.masked || pl.nslots > 1) {
-            auto kern = cut::cut_apply_kernel<1>;
-            FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), cut::APPLY_LDS));
-            kern<<<ckgrid, cut::NT, cut::APPLY_LDS, stream>>>(kr, scale + bh + kv0, stR, pl.nslots, dv_q,
-                                                              RowScalarsOut{nullptr, 0, 0}, nown_k, pl.chunk, pl.masked,
-                                                              ds->a0, ds->a1, a2, ratio, 1);
-          }
-        }
       } else {
         apply_kernel<D, T, 1><<<kgrid, 256, 0, stream>>>(
             kr, qr, gr, scale + bh + kv0, scale + h0, dn, stR, pl.nslots, dv_q, RowScalarsOut{nullptr, 0, 0}, nown_k,
@@ -941,25 +860,13 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
       }
     }
     FM_TRY(launch_status("apply_kernel (dv)"));
-    if (ratio > 1 && !(pl.cut && pl.masked && pl.nslots < 2)) {
+    if (ratio > 1) {
       const int64_t per_head = (int64_t)nk * D;
       const dim3 sgrid((unsigned)((per_head / 4 + 255) / 256), heads / ratio);
       group_sum_kernel<T><<<sgrid, 256, 0, stream>>>(dk_tmp, mk_rows(dk, L.dk, kv0), nk, D, ratio);
       group_sum_kernel<T><<<sgrid, 256, 0, stream>>>(dv_tmp, mk_rows(dv, L.dv, kv0), nk, D, ratio);
       FM_TRY(launch_status("group_sum_kernel"));
     }
-  }
-  // normalisation partials per query head and per key/value head
-  int nbq = pl.nblk_q, nbk = pl.nblk_k * ratio;
-  if (pl.cut) {
-    nbq = nbq_cut;
-    nbk = (nk + cut::TB - 1) / cut::TB * ratio;
-    if constexpr (D == 64 && !kBf16Mfma<T>) {
-      if (pl.masked)
-        FM_TRY((dense_backward_dp<D, T>(ds, own_chunk_plan(pl), L, q, k, v, o, den, den_stride, go, dq, dk, dv, scale, cvec,
-                                        rpart, nullptr, nullptr, &nbq, &nbk, stream, 1)));
-    }
-    rpart_k = rpart + (int64_t)bh * nbq;
   }
   if (ds->normalize && pl.rowpass) {
     // one partial per row block of the dq pass; sum_j dk_hat_j . k_hat_j is the same number
@@ -972,8 +879,8 @@ int backward_impl(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
   } else if (ds->normalize) {
     ScopedKernel sk(FASTMAX_K_NORM_FIX, stream);
     norm_fix_kernel<T><<<bh + bhkv, D, 0, stream>>>(
-        NormFixSide<T>{mk_rows(dq, L.dq), mk_rows(q, L.q), scale, arg, rpart, bh, nbq, nq},
-        NormFixSide<T>{mk_rows(dk, L.dk), mk_rows(k, L.k), scale + bh, arg + bh, rpart_k, bhkv, nbk, nk}, D,
+        NormFixSide<T>{mk_rows(dq, L.dq), mk_rows(q, L.q), scale, arg, rpart, bh, pl.nblk_q, nq},
+        NormFixSide<T>{mk_rows(dk, L.dk), mk_rows(k, L.k), scale + bh, arg + bh, rpart_k, bhkv, pl.nblk_k * ratio, nk}, D,
         ds->lim);
     FM_TRY(launch_status("norm_fix_kernel"));
   }
@@ -1016,23 +923,16 @@ int dense_lin_states(const fastmax_desc* ds, const Plan& pl, const Layout& L, co
   return launch_status("dense_state_kernel");
 }
 
-// Whether the dense kernels on cut operands run blocks of four waves instead of eight: while the eight-wave blocks leave
-// CUs idle, four-wave ones spread a head over twice as many (a wave then has its SIMD to itself).
-// Measured, fp32 forward + backward, causal, eight against four waves: 8 heads x 400 x 32 102.5 -> 87.8 us, 8 x 2500 x 64
-// 805 -> 698, 32 x 1000 x 64 350 -> 314; where the eight-wave blocks fill the chip they share a stage among more waves.
-bool small_blocks(int heads, int rows) { return (int64_t)heads * ((rows + 255) / 256) < 256; }
-
 template <int DP, class T>
 int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v, T* o,
-                     float* den, int64_t den_stride, const float* scale, float* kstate, hipStream_t stream, int add) {
+                     float* den, int64_t den_stride, const float* scale, float* kstate, hipStream_t stream) {
   using S = dense::Shape<DP, T>;
-  const int npos = pl.masked ? pl.nk : pl.nq;
-  auto launch = [&](auto nwtag) -> int {
-  constexpr int RT = S::RT_FWD, BN = S::BN, NW = decltype(nwtag)::value, BM = 32 * RT * NW;
+  constexpr int RT = S::RT_FWD, BN = S::BN, NW = S::NW_FWD, BM = 32 * RT * NW;
   static_assert(256 % BM == 0 && 256 % BN == 0, "blocks and stages do not straddle the chunks of the linear mode");
   const size_t smem = dense::Lds<DP, T, BN>::bytes(1, 1, BM);
   auto kern = dense::dense_fwd_kernel<DP, T, RT, BN, NW>;
   FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
+  const int npos = pl.masked ? pl.nk : pl.nq;
   const int nb = (npos + BM - 1) / BM - pl.off / BM;
   if (pl.lin)
     FM_TRY((dense_lin_states<DP, T>(ds, pl, L, q, k, v, nullptr, nullptr, 0, nullptr, scale, true, kstate, nullptr, stream)));
@@ -1041,13 +941,8 @@ int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, co
                                                scale + pl.bh, mk_rows(o, L.o, 0, pl.off),
                                                mk_scalars(den, pl.nq, den_stride, 0, pl.off), npos, pl.nk, ds->d,
                                                pl.masked, ds->a0, ds->a1, pl.p2 ? ds->a2 : 0.f, pl.ratio,
-                                               pl.lin ? kstate : nullptr, pl.lchunk, pl.lslots, add);
+                                               pl.lin ? kstate : nullptr, pl.lchunk, pl.lslots);
   return launch_status("dense_fwd_kernel");
-  };
-  if constexpr (S::SPLIT) {
-    if (small_blocks(pl.bh, npos)) return launch(std::integral_constant<int, 4>{});
-  }
-  return launch(std::integral_constant<int, S::NW_FWD>{});
 }
 
 template <class T>
@@ -1069,13 +964,11 @@ template <int DP, class T>
 int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v,
                       const T* o, const float* den, int64_t den_stride, const T* go, T* dq, T* dk, T* dv,
                       const float* scale, float* cvec_w, float* rpart, float* kstate, float* qstate, int* nbq_out,
-                      int* nbk_out, hipStream_t stream, int add) {
+                      int* nbk_out, hipStream_t stream) {
   // c_i = grad_out_i . out_i / den_i: the dq kernel forms it from rows it holds anyway and leaves it in cvec for the
   // dk / dv kernel -- except in the linear mode, whose query-side states need it before any of them runs
-  // (add: the states of the other chunks needed it, too)
-  const bool prep_in_dq = !pl.lin && !add;
-  const int lchunk = pl.lchunk, lslots = pl.lslots;
-  if (pl.lin) FM_TRY((launch_bwd_prep<T>(pl, L, go, o, den, den_stride, cvec_w, stream)));
+  const bool prep_in_dq = !pl.lin;
+  if (!prep_in_dq) FM_TRY((launch_bwd_prep<T>(pl, L, go, o, den, den_stride, cvec_w, stream)));
   const float* cvec = cvec_w;
   using S = dense::Shape<DP, T>;
   constexpr int BN = S::BN;
@@ -1090,10 +983,10 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
     FM_TRY((dense_lin_states<DP, T>(ds, pl, L, q, k, v, go, den, den_stride, cvec, scale, false, kstate, qstate, stream)));
   const float* ksl = pl.lin ? kstate : nullptr;
   const float* qsl = pl.lin ? qstate : nullptr;
-  auto launch_dq = [&](auto nwtag) -> int {
-    constexpr int RT = S::RT_DQ, NW = decltype(nwtag)::value, BM = 32 * RT * NW;
+  {
+    constexpr int RT = S::RT_DQ, NW = S::NW_DQ, BM = 32 * RT * NW;
     static_assert(256 % BM == 0, "blocks do not straddle the chunks of the linear mode");
-    const size_t smem = dense::Lds<DP, T, BN>::bytes(2, 1, 2 * NW);
+    const size_t smem = dense::Lds<DP, T, BN>::bytes(2, 1, NW);
     auto kern = dense::dense_dq_kernel<DP, T, RT, BN, NW>;
     FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
     const int nb = (npos + BM - 1) / BM - pl.off / BM;
@@ -1101,15 +994,15 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
     ScopedKernel sk(FASTMAX_K_BWD_DQ, stream);
     kern<<<dim3(pl.bh, nb), 64 * NW, smem, stream>>>(qr, gr, dn, cv, kr, vr, scale, scale + pl.bh, mk_rows(dq, L.dq, 0, pl.off), rq,
                                                  npos, pl.nk, ds->d, pl.masked, pl.p2 && a2 != 0.f, ds->a1, a2, pl.ratio,
-                                                 ksl, lchunk, lslots, mk_rows(o, L.o, 0, pl.off),
-                                                 prep_in_dq ? mk_scalars<float>(cvec_w, pl.nq, 1, 0, pl.off) : RowScalarsOut{nullptr, 0, 0}, add);
-    return launch_status("dense_dq_kernel");
-  };
-  auto launch_dkdv = [&](auto nwtag) -> int {
-    constexpr int RT = S::RT_KV, NW = decltype(nwtag)::value, BM = 32 * RT * NW, BNK = S::BN_KV;
+                                                 ksl, pl.lchunk, pl.lslots, mk_rows(o, L.o, 0, pl.off),
+                                                 prep_in_dq ? mk_scalars<float>(cvec_w, pl.nq, 1, 0, pl.off) : RowScalarsOut{nullptr, 0, 0});
+    FM_TRY(launch_status("dense_dq_kernel"));
+  }
+  {
+    constexpr int RT = S::RT_KV, NW = S::NW_KV, BM = 32 * RT * NW, BNK = S::BN_KV;
     static_assert(256 % BM == 0 && 256 % BNK == 0, "blocks and stages do not straddle the chunks of the linear mode");
-    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + 2 * ((NW + 3) / 4 * 4)) +
-                        (S::KLO ? (size_t)NW * (DP / dense::Policy<DP, T>::KF + 1) * 64 * sizeof(fm_u4) : 0);
+    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + (NW + 3) / 4 * 4) +
+                        (S::KLO ? (size_t)NW * (DP / dense::Policy<DP, T>::KF) * 64 * sizeof(fm_u4) : 0);
     auto kern = dense::dense_dkdv_kernel<DP, T, RT, BNK, NW>;
     FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
     const int nb = (pl.nk + BM - 1) / BM;
@@ -1118,20 +1011,9 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
     ScopedKernel sk(FASTMAX_K_BWD_DK, stream);
     kern<<<dim3(pl.bhkv, nb), 64 * NW, smem, stream>>>(kr, vr, qr, gr, dn, cv, scale, scale + pl.bh, mk_rows(dk, L.dk),
                                                    mk_rows(dv, L.dv), rk, npos, pl.nk, ds->d, pl.masked, ds->a0, ds->a1,
-                                                   a2, pl.ratio, qsl, lchunk, lslots, add);
-    return launch_status("dense_dkdv_kernel");
-  };
-  bool small_q = false, small_k = false;
-  if constexpr (S::SPLIT) {
-    small_q = small_blocks(pl.bh, npos);
-    small_k = small_blocks(pl.bhkv, pl.nk);
-    if (small_q) FM_TRY(launch_dq(std::integral_constant<int, 4>{}));
+                                                   a2, pl.ratio, qsl, pl.lchunk, pl.lslots);
+    FM_TRY(launch_status("dense_dkdv_kernel"));
   }
-  if (!small_q) FM_TRY(launch_dq(std::integral_constant<int, S::NW_DQ>{}));
-  if constexpr (S::SPLIT) {
-    if (small_k) FM_TRY(launch_dkdv(std::integral_constant<int, 4>{}));
-  }
-  if (!small_k) FM_TRY(launch_dkdv(std::integral_constant<int, S::NW_KV>{}));
   return FASTMAX_OK;
 }
 

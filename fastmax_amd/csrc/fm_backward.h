@@ -73,16 +73,15 @@ __global__ void norm_fix_kernel(NormFixSide<T> a, NormFixSide<T> b, int d, float
   const int row = sd.arg[head];
   if (row < 0 || row >= sd.n) return;
   // the block's threads share the partials (fixed order per thread and in the tree: the same sum every run)
-  // (in 64 bits: the sum's rounding would land in one row of the gradient)
-  __shared__ double red[128];
-  double r = 0;
+  __shared__ float red[128];
+  float r = 0.f;
   for (int bl = c; bl < sd.nblk; bl += blockDim.x) r += sd.rpart[(int64_t)head * sd.nblk + bl];
   red[c] = r;
   __syncthreads();
-  r = 0;
+  r = 0.f;
   for (int t = 0; t < (int)blockDim.x; ++t) r += red[t];
   const float s = sd.scale[head];
-  const float fac = (float)r * s * s / (lim * lim);
+  const float fac = r * s * s / (lim * lim);
   const HeadRows<T> dh = sd.dx.head(head);
   const HeadRows<const T> xh = sd.x.head(head);
   T* dst = dh.row(row) + c;

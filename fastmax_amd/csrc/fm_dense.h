@@ -159,19 +159,14 @@ struct MmaSplit {
   static __device__ __forceinline__ f16v mma1(const fm_u4& a, const fm_u4& b, const f16v& c) {
     return FM_MFMA_BF16(__builtin_bit_cast(bf8v, a), __builtin_bit_cast(bf8v, b), c);
   }
-  // the five products below the first: where a result is about to cancel they are all added up before the first
-  // products, so that only one rounding per step is of the result's own size
-  static __device__ __forceinline__ f16v mma_small(const Frag& a, const Frag& b, f16v c) {
+  static __device__ __forceinline__ f16v mma(const Frag& a, const Frag& b, f16v c) {
     c = mma1(a.p[2], b.p[0], c);
     c = mma1(a.p[0], b.p[2], c);
     c = mma1(a.p[1], b.p[1], c);
     c = mma1(a.p[1], b.p[0], c);
-    return mma1(a.p[0], b.p[1], c);
+    c = mma1(a.p[0], b.p[1], c);
+    return mma1(a.p[0], b.p[0], c);
   }
-  static __device__ __forceinline__ f16v mma(const Frag& a, const Frag& b, const f16v& c) {
-    return mma1(a.p[0], b.p[0], mma_small(a, b, c));
-  }
-  static __device__ __forceinline__ fm_u4 load_first(const Elt* p) { return *reinterpret_cast<const fm_u4*>(p); }
   // the three parts of a pair of floats, packed
   static __device__ __forceinline__ void cut(float x, float y, uint32_t (&w)[3]) {
     w[0] = pack_bf2(x, y);
@@ -193,31 +188,6 @@ struct MmaSplit {
     }
     return f;
   }
-  // The same for values that are formed in registers (weights, features): what a part leaves is one dot product of
-  // the packed pair instead of an unpacking and a subtraction.  A value that is not finite makes its pair not a number,
-  // which ends in the same row of the result either way.
-  static __device__ __forceinline__ Frag make_own(const float (&x)[8]) {
-    // the pairs (-1, 0) and (0, -1), in registers: as a constant the compiler writes the first as the inline -1.0, which
-    // the instruction reads as the fp32 pattern, i.e. as the second
-    uint32_t LO, HI;
-    asm("s_mov_b32 %0, 0xbf80" : "=s"(LO));
-    asm("s_mov_b32 %0, 0xbf800000" : "=s"(HI));
-    Frag f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float a = x[2 * e], b = x[2 * e + 1];
-      uint32_t w = pack_bf2(a, b);
-      f.p[0][e] = w;
-      a = fm_dot2_bf16(w, LO, a);
-      b = fm_dot2_bf16(w, HI, b);
-      w = pack_bf2(a, b);
-      f.p[1][e] = w;
-      a = fm_dot2_bf16(w, LO, a);
-      b = fm_dot2_bf16(w, HI, b);
-      f.p[2][e] = pack_bf2(a, b);
-    }
-    return f;
-  }
   static __device__ __forceinline__ void values(const Frag& f, float (&o)[8]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -225,11 +195,10 @@ struct MmaSplit {
       o[2 * e + 1] = (bf_hi(f.p[2][e]) + bf_hi(f.p[1][e])) + bf_hi(f.p[0][e]);
     }
   }
-  // (OWN = false: the kernel has no two scalar registers left)
-  template <int F, bool OWN = true>
+  template <int F>
   static __device__ __forceinline__ Frag from_acc(const f16v& a) {
     const float x[8] = {a[8 * F], a[8 * F + 1], a[8 * F + 2], a[8 * F + 3], a[8 * F + 4], a[8 * F + 5], a[8 * F + 6], a[8 * F + 7]};
-    return OWN ? make_own(x) : make(x);
+    return make(x);
   }
   template <int F>
   static __device__ __forceinline__ float fsum(const f16v& a, const Frag&, float acc) {
@@ -283,15 +252,15 @@ using Policy = typename PolicyOf<DP, T>::type;
 // an all-zero accumulator tile (the C operand of a contraction's first step)
 constexpr f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-// sum over the NW waves of a block; red is NW values in LDS; the result is valid in every thread
-template <int NW, class S>
-__device__ __forceinline__ S block_sum(S v, S* red, int tid) {
+// sum over the NW waves of a block; red is NW floats of LDS; the result is valid in every thread
+template <int NW>
+__device__ __forceinline__ float block_sum(float v, float* red, int tid) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   __syncthreads();
   if ((tid & 63) == 0) red[tid >> 6] = v;
   __syncthreads();
-  S t = 0;
+  float t = 0.f;
 #pragma unroll
   for (int w = 0; w < NW; ++w) t += red[w];
   return t;
@@ -405,26 +374,17 @@ __device__ __forceinline__ float load_g_frags_and_c(const HeadRows<const T>& gr,
       const int ch = M::KF * m + M::EPL * hh + EPP * u;
       const bool ok = live && ch < d;
       const uint4 tg = *reinterpret_cast<const uint4*>(grow + (ok ? ch : 0));
-      float g[EPP];
+      const uint4 to = *reinterpret_cast<const uint4*>(orw + (ok ? ch : 0));
+      float g[EPP], y[EPP];
       Mma<T>::unpack(tg, g);
+      Mma<T>::unpack(to, y);
 #pragma unroll
-      for (int e = 0; e < EPP; ++e) x[EPP * u + e] = ok ? g[e] * rden : 0.f;
+      for (int e = 0; e < EPP; ++e) {
+        dot += ok ? g[e] * y[e] : 0.f;
+        x[EPP * u + e] = ok ? g[e] * rden : 0.f;
+      }
     }
     f[m] = M::make(x);
-  }
-  // (the lane halves take alternating 16-byte pieces whatever the fragments' layout: c of the first rows nearly cancels
-  // with g . v, and its last bits stay what they are)
-#pragma unroll
-  for (int m = 0; m < DP / (2 * EPP); ++m) {
-    const int ch = 2 * EPP * m + EPP * hh;
-    const bool ok = live && ch < d;
-    const uint4 tg = *reinterpret_cast<const uint4*>(grow + (ok ? ch : 0));
-    const uint4 to = *reinterpret_cast<const uint4*>(orw + (ok ? ch : 0));
-    float g[EPP], y[EPP];
-    Mma<T>::unpack(tg, g);
-    Mma<T>::unpack(to, y);
-#pragma unroll
-    for (int e = 0; e < EPP; ++e) dot += ok ? g[e] * y[e] : 0.f;
   }
   return (dot + __shfl_xor(dot, 32, 64)) * rden;
 }
@@ -462,13 +422,8 @@ struct Shape {
   static constexpr int NW_FWD = ((BF && DP == 64) || SPLIT) ? 8 : 4;
   static constexpr int NW_DQ = ((BF && DP == 64) || SPLIT) ? 8 : 4;
   static constexpr int NW_KV = ((BF && DP == 64) || SPLIT) ? 8 : 4;
-  // what the normaliser's chain rule sums a block's gradients in (with fp32 tensors the sum's own rounding would be
-  // the largest error left in the one row that receives it)
-  using Sum = typename std::conditional<SPLIT, double, float>::type;
-  // the dk / dv kernel keeps the last parts of its own key fragments in LDS (registers that 64 channels lack)
+  // the dk / dv kernel keeps the last parts of its own key fragments in LDS (16 registers that 64 channels lack)
   static constexpr bool KLO = SPLIT && DP == 64;
-  // the kernels can add to sums that cut_apply_kernel / cut_grad_kernel left in the outputs (all of the 64 channels are there)
-  static constexpr bool ADD = SPLIT && DP == 64;
   static constexpr int RT_FWD = 1;
   static constexpr int RT_DQ = 1;
   static constexpr int RT_KV = 1;
@@ -727,7 +682,7 @@ template <int DP, class T, int RT, int BN, int NW>
 __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_kernel(
     Rows<const T> Q, Rows<const T> K, Rows<const T> V, const float* __restrict__ qscale,
     const float* __restrict__ kscale, Rows<T> O, RowScalarsOut den, int npos, int nk, int d, int masked, float a0,
-    float a1, float a2, int ratio, const float* __restrict__ lstate, int lchunk, int lslots, int add) {
+    float a1, float a2, int ratio, const float* __restrict__ lstate, int lchunk, int lslots) {
   using M = Policy<DP, T>;
   using Elt = typename M::Elt;
   using Frag = typename M::Frag;
@@ -759,9 +714,8 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
   const int kend = masked ? (tok0 + BM < nk ? tok0 + BM : nk) : nk;
   const int nst = (kend + BN - 1) / BN;
   // linear mode: the keys before the block's chunk (unmasked: all keys) come as a state
-  const bool walk = lstate || (Shape<DP, T>::ADD && add);   // (add: what the keys before the chunk give is in the output already)
-  const int lc = (walk && masked) ? tok0 / lchunk : 0;
-  const int st0 = walk ? (masked ? lc * (lchunk / BN) : nst) : 0;
+  const int lc = (lstate && masked) ? tok0 / lchunk : 0;
+  const int st0 = lstate ? (masked ? lc * (lchunk / BN) : nst) : 0;
   TileRegs<DP, T, BN, NT, M> kt, vt;
   auto stage_load = [&](int st) {
     kt.load(Kh, st * BN, nk, d, tid);
@@ -832,7 +786,6 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
       for (int cb = 0; cb < CB; ++cb) vb[f][cb] = M::load(vl + (cb * 32 + i) * PT + t32 * 32 + KF * f + EPL * hh, BN);
     // scores, transposed: rows = keys trow(r, hh), lanes = own queries
     f16v sc[RT];
-    const bool first = Shape<DP, T>::SPLIT && masked && kb == 0 && rel == 0;
 #pragma unroll
     for (int m0 = 0; m0 < NF; m0 += HC) {   // (HC operand fragments are read ahead of the instructions that use them)
       Frag ka[HC];
@@ -842,27 +795,6 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
       for (int m = 0; m < HC; ++m)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) sc[rt] = M::mma(ka[m], qf[rt][m0 + m], m0 + m == 0 ? kZero16 : sc[rt]);
-    }
-    if constexpr (Shape<DP, T>::SPLIT) {
-      // (the first query's output in the bits that the fp32 instruction gives: see the dq kernel)
-      if (first) {
-        FM_KEEP_BRANCH();
-        const T* qrow = Qh.base + (unsigned)max(i < npos ? i : npos - 1, Qh.lo) * Qh.pitch;
-        const T* krow = Kh.base + (unsigned)(i < nk ? i : nk - 1) * Kh.pitch;
-        const float fq = add ? qscale[head] : kq, fk = add ? kscale[hkv] : 1.0f;
-        f16v t = kZero16;
-#pragma unroll 1
-        for (int g = 0; g < DP / 8; ++g) {
-          const int ch = add ? hh * (DP / 2) + 4 * g : 8 * g + 4 * hh;
-          const float4 k4 = *reinterpret_cast<const float4*>(krow + (ch < d ? ch : 0)), q4 = *reinterpret_cast<const float4*>(qrow + (ch < d ? ch : 0));
-          const float f = ch < d ? fq : 0.f;
-          t = FM_MFMA(k4.x * fk, q4.x * f, t);
-          t = FM_MFMA(k4.y * fk, q4.y * f, t);
-          t = FM_MFMA(k4.z * fk, q4.z * f, t);
-          t = FM_MFMA(k4.w * fk, q4.w * f, t);
-        }
-        sc[0] = t;
-      }
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -921,31 +853,14 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
     __syncthreads();
   }
 
-  const HeadRows<T> Oh = O.head(head);
-  float* denh = den.head(head);
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    float tot = dn[rt] + __shfl_xor(dn[rt], 32, 64);
-    if constexpr (Shape<DP, T>::ADD) {
-      if (add && lc > 0) {   // numerators and denominators of the keys before the chunk (all requested before the first store)
-        const int own = tok0 + (w * RT + rt) * 32 + i;
-        tot += denh[(int64_t)max(own < npos ? own : npos - 1, Qh.lo) * den.stride];
-        float prev[CB][16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int pos = tok0 + (w * RT + rt) * 32 + trow(r, hh), ps = max(pos < npos ? pos : npos - 1, Qh.lo);
-#pragma unroll
-          for (int cb = 0; cb < CB; ++cb) prev[cb][r] = to_f32(Oh.base[(unsigned)ps * Oh.pitch + (unsigned)(cb * 32 + i)]);
-        }
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[rt][cb][r] += prev[cb][r];
-      }
-    }
+    const float tot = dn[rt] + __shfl_xor(dn[rt], 32, 64);
     if (hh == 0) denl[(w * RT + rt) * 32 + i] = tot;
   }
   __syncthreads();
+  const HeadRows<T> Oh = O.head(head);
+  float* denh = den.head(head);
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -973,7 +888,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
     Rows<const T> Q, Rows<const T> GO, RowScalars den, RowScalars cvec, Rows<const T> K, Rows<const T> V,
     const float* __restrict__ qscale, const float* __restrict__ kscale, Rows<T> DQ, float* __restrict__ rpart,
     int npos, int nk, int d, int masked, int p2, float a1, float a2, int ratio, const float* __restrict__ lstate,
-    int lchunk, int lslots, Rows<const T> OUTF, RowScalarsOut cprep, int add) {
+    int lchunk, int lslots, Rows<const T> OUTF, RowScalarsOut cprep) {
   using M = Policy<DP, T>;
   using Elt = typename M::Elt;
   using Frag = typename M::Frag;
@@ -987,8 +902,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
   Elt* Kl = reinterpret_cast<Elt*>(dense_smem);   // [2][BN][PR]
   Elt* Vl = Kl + 2 * L::RM;                       // [2][BN][PR]
   Elt* Kt = Vl + 2 * L::RM;                       // [2][DP][PT]
-  using Sum = typename Shape<DP, T>::Sum;
-  Sum* red = reinterpret_cast<Sum*>(Kt + 2 * L::TR);   // [NW]
+  float* red = reinterpret_cast<float*>(Kt + 2 * L::TR);   // [NW]
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, hh = l >> 5;
   const int nb = gridDim.y, bx = blockIdx.y;   // (heads, row blocks), as in the forward kernel
@@ -1025,9 +939,8 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
 
   const int kend = masked ? (tok0 + BM < nk ? tok0 + BM : nk) : nk;
   const int nst = (kend + BN - 1) / BN;
-  const bool walk = lstate || (Shape<DP, T>::ADD && add);
-  const int lc = (walk && masked) ? tok0 / lchunk : 0;   // (linear mode and add, as in the forward kernel)
-  const int st0 = walk ? (masked ? lc * (lchunk / BN) : nst) : 0;
+  const int lc = (lstate && masked) ? tok0 / lchunk : 0;   // (linear mode, as in the forward kernel)
+  const int st0 = lstate ? (masked ? lc * (lchunk / BN) : nst) : 0;
   TileRegs<DP, T, BN, NT, M> kt, vt;
   auto stage_load = [&](int st) {
     kt.load(Kh, st * BN, nk, d, tid);
@@ -1078,7 +991,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
 
   // (rel as in the forward kernel: own tile rt has the key tile on its diagonal when rel == 32 rt and
   // wholly after its queries when rel > 32 rt)
-  auto tile = [&](int t32, int kb, int rel, const Elt* kl, const Elt* vl, const Elt* ktl) __attribute__((always_inline)) {
+  auto tile = [&](int t32, int rel, const Elt* kl, const Elt* vl, const Elt* ktl) __attribute__((always_inline)) {
     // transposed tiles (rows = keys, lanes = own queries): f'(s) and g . v - c
     f16v sc[RT], pt[RT];
 #pragma unroll
@@ -1086,7 +999,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         sc[rt][r] = a1;
-        pt[rt][r] = Shape<DP, T>::SPLIT ? 0.f : -cown[rt];
+        pt[rt][r] = -cown[rt];
       }
 #pragma unroll
     for (int m0 = 0; m0 < NF; m0 += HC) {
@@ -1100,53 +1013,14 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
       for (int m = 0; m < HC; ++m)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-          if constexpr (Shape<DP, T>::SPLIT) pt[rt] = M::mma_small(va[m], gf[rt][m0 + m], pt[rt]);
-          else pt[rt] = M::mma(va[m], gf[rt][m0 + m], pt[rt]);
+          pt[rt] = M::mma(va[m], gf[rt][m0 + m], pt[rt]);
           if (p2) sc[rt] = M::mma(ka[m], qf[rt][m0 + m], sc[rt]);
         }
-    }
-    if constexpr (Shape<DP, T>::SPLIT) {   // (g . v and c are nearly equal in the first rows)
-#pragma unroll
-      for (int m = 0; m < NF; ++m)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          pt[rt] = M::mma1(M::load_first(vl + (t32 * 32 + i) * PR + KF * m + EPL * hh), gf[rt][m].p[0], pt[rt]);
-    }
-    float csub[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) csub[rt] = cown[rt];
-    if constexpr (Shape<DP, T>::SPLIT) {
-      // The first query sees one key and its gradient is zero: what comes out is the rounding of g . v - c alone, which
-      // after a long sequence shows against the gradients of the others.  This one tile of a head stays on the fp32
-      // instruction, its channels in the order of the fp32 kernels, so that this rounding does not change.
-      if (masked && kb == 0 && rel == 0) {
-        FM_KEEP_BRANCH();
-        const int ps = max(i < npos ? i : npos - 1, Qh.lo);
-        const float rden = (i < npos && i >= Qh.lo) ? 1.0f / denh[(int64_t)ps * den.stride] : 0.f;
-        const T* grow = Gh.base + (unsigned)ps * Gh.pitch;
-        const T* vrow = Vh.base + (unsigned)(i < nk ? i : nk - 1) * Vh.pitch;
-        f16v t;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) t[r] = add ? 0.f : -cown[0];
-#pragma unroll 1
-        for (int g = 0; g < DP / 8; ++g) {
-          const int ch = add ? hh * (DP / 2) + 4 * g : 8 * g + 4 * hh;
-          const float on = ch < d ? 1.0f : 0.f;
-          const float4 v4 = *reinterpret_cast<const float4*>(vrow + (ch < d ? ch : 0)), g4 = *reinterpret_cast<const float4*>(grow + (ch < d ? ch : 0));
-          const float gs = on * rden;
-          t = FM_MFMA(v4.x, g4.x * gs, t);
-          t = FM_MFMA(v4.y, g4.y * gs, t);
-          t = FM_MFMA(v4.z, g4.z * gs, t);
-          t = FM_MFMA(v4.w, g4.w * gs, t);
-        }
-        pt[0] = t;
-        if (!add) csub[0] = 0.f;
-      }
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) pt[rt][r] = sc[rt][r] * (Shape<DP, T>::SPLIT ? pt[rt][r] - csub[rt] : pt[rt][r]);
+      for (int r = 0; r < 16; ++r) pt[rt][r] = sc[rt][r] * pt[rt][r];
       if (masked && rel >= 32 * rt) {   // (wave-uniform) a key may not lie after the query
         FM_KEEP_BRANCH();
         const int lim = rel > 32 * rt ? -1 : i;
@@ -1185,7 +1059,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
       const int kb = st * BN + t32 * 32;
       if (kb >= kend) continue;
       if (masked && kb > q00 + 32 * (RT - 1)) continue;   // after every own query
-      tile(t32, kb, kb - q00, kl, vl, ktl);
+      tile(t32, kb - q00, kl, vl, ktl);
     }
     if (st + 1 < nst) stage_store(buf ^ 1);
     __syncthreads();
@@ -1193,24 +1067,12 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
 
   // dq = qs ks acc (the keys went in unscaled); sum of dqh . qh = qs ks sum acc . q
   const HeadRows<T> Dh = DQ.head(head);
-  Sum rs = 0;
+  float rs = 0.f;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     // (the q elements are all requested before the first store: a load that had to stay behind a store that
     // may alias it would cost one memory round trip per element)
-    float qv[CB][16], prev[CB][16];
-    const bool plus = Shape<DP, T>::ADD && add && lc > 0;
-    if constexpr (Shape<DP, T>::ADD) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int pos = tok0 + (w * RT + rt) * 32 + trow(r, hh), ps = max(pos < npos ? pos : npos - 1, Qh.lo);
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) {
-          prev[cb][r] = 0.f;
-          if (plus) prev[cb][r] = to_f32(Dh.base[(unsigned)ps * Dh.pitch + (unsigned)(cb * 32 + i)]);
-        }
-      }
-    }
+    float qv[CB][16];
     if (rpart) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -1229,10 +1091,9 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
         for (int cb = 0; cb < CB; ++cb) {
           const int c = cb * 32 + i;
           if (c < d) {
-            float v = acc[rt][cb][r] * kq;
-            if constexpr (Shape<DP, T>::ADD) v += prev[cb][r];
+            const float v = acc[rt][cb][r] * kq;
             Dh.base[(unsigned)pos * Dh.pitch + (unsigned)c] = from_f32<T>(v);
-            if (rpart) rs += (Sum)v * (Sum)qv[cb][r];
+            if (rpart) rs += v * qv[cb][r];
           }
         }
       }
@@ -1240,7 +1101,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
   }
   if (rpart) {
     rs = block_sum<NW>(rs, red, tid);
-    if (tid == 0) rpart[(int64_t)head * nb + bx] = (float)rs;
+    if (tid == 0) rpart[(int64_t)head * nb + bx] = rs;
   }
 }
 
@@ -1255,7 +1116,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
     Rows<const T> K, Rows<const T> V, Rows<const T> Q, Rows<const T> GO, RowScalars den, RowScalars cvec,
     const float* __restrict__ qscale, const float* __restrict__ kscale, Rows<T> DK, Rows<T> DV,
     float* __restrict__ rpart, int npos, int nk, int d, int masked, float a0, float a1, float a2, int ratio,
-    const float* __restrict__ lstate, int lchunk, int lslots, int add) {
+    const float* __restrict__ lstate, int lchunk, int lslots) {
   using M = Policy<DP, T>;
   using Elt = typename M::Elt;
   using Frag = typename M::Frag;
@@ -1271,14 +1132,13 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
   Elt* Qt = Gl + 2 * L::RM;                       // [2][DP][PT]
   Elt* Gt = Qt + 2 * L::TR;                       // [2][DP][PT]
   float* Cl = reinterpret_cast<float*>(Gt + 2 * L::TR);   // [2][BN]: -c of the streamed queries
-  using Sum = typename Shape<DP, T>::Sum;
-  Sum* red = reinterpret_cast<Sum*>(Cl + 2 * BN);   // [NW]
-  fm_u4* kl2 = reinterpret_cast<fm_u4*>(red + (NW + 3) / 4 * 4);   // (KLO) [NW][NF + 1][64]: the last parts of the key fragments and of one value fragment
+  float* red = Cl + 2 * BN;                       // [NW]
+  fm_u4* kl2 = reinterpret_cast<fm_u4*>(red + (NW + 3) / 4 * 4);   // (KLO) [NW][NF][64]: the last parts of the key fragments
   constexpr bool KLO = Shape<DP, T>::KLO;
   static_assert(!KLO || RT == 1, "one own tile per wave");
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, hh = l >> 5;
-  kl2 += w * (NF + 1) * 64 + l;
+  kl2 += w * NF * 64 + l;
   const int nb = gridDim.y, bx = blockIdx.y;   // (key/value heads, key blocks)
   const int hkv = blockIdx.x;
   const int tok0 = bx * BM;   // (under the mask the first key blocks see the most queries: already first)
@@ -1295,18 +1155,10 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
   if constexpr (KLO) {   // (read back by the lane that wrote them: no barrier)
 #pragma unroll
     for (int m = 0; m < NF; ++m) kl2[m * 64] = kf[0][m].p[2];
-    kl2[NF * 64] = vf[0][0].p[2];
   }
   auto key_frag = [&](int rt, int m) __attribute__((always_inline)) {
     Frag f = kf[rt][m];
     if constexpr (KLO) f.p[2] = kl2[m * 64];
-    return f;
-  };
-  auto value_frag = [&](int rt, int m) __attribute__((always_inline)) {
-    Frag f = vf[rt][m];
-    if constexpr (KLO) {
-      if (m == 0) f.p[2] = kl2[NF * 64];
-    }
     return f;
   };
   f16v dk[RT][CB], dv[RT][CB];
@@ -1332,11 +1184,10 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
     const float c2 = a2 * qs * qs, c1 = a1 * qs, b2 = 2.0f * a2 * qs * qs;
     const int lo = Qh.lo;
     // linear mode: the queries after the block's chunk (unmasked: all queries) come as a state
-    const bool walk = lstate || (Shape<DP, T>::ADD && add);   // (add: what the queries after the chunk give is in the outputs already)
-    const int lc = (walk && masked) ? tok0 / lchunk : 0;
-    const int qend = (walk && masked && (lc + 1) * lchunk < npos) ? (lc + 1) * lchunk : npos;
+    const int lc = (lstate && masked) ? tok0 / lchunk : 0;
+    const int qend = (lstate && masked && (lc + 1) * lchunk < npos) ? (lc + 1) * lchunk : npos;
     const int nst = (qend + BN - 1) / BN;
-    const int st0 = walk && !masked ? nst : masked ? (tok0 > lo ? tok0 : lo) / BN : 0;
+    const int st0 = lstate && !masked ? nst : masked ? (tok0 > lo ? tok0 : lo) / BN : 0;
     auto stage_load = [&](int st) {
       qt.load(Qh, st * BN, npos, d, tid);
       gt.load(Gh, st * BN, npos, d, tid, denh, den.stride);
@@ -1388,14 +1239,11 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
-          Frag kx[NF], vx[NF];
+          Frag kx[NF];
 #pragma unroll
-          for (int m = 0; m < NF; ++m) {
-            kx[m] = key_frag(rt, m);
-            vx[m] = value_frag(rt, m);
-          }
+          for (int m = 0; m < NF; ++m) kx[m] = key_frag(rt, m);
           dv[rt][cb] = lin_own_times<DP, T>(kx, Rt + (cb * 32 + i) * PS + EPL * hh, dv[rt][cb]);
-          dk[rt][cb] = lin_own_times<DP, T>(vx, Rn + (cb * 32 + i) * PS + EPL * hh, dk[rt][cb]);
+          dk[rt][cb] = lin_own_times<DP, T>(vf[rt], Rn + (cb * 32 + i) * PS + EPL * hh, dk[rt][cb]);
         }
       __syncthreads();
     }
@@ -1411,7 +1259,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
       f16v sc[RT], pt[RT];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float4 c4 = Shape<DP, T>::SPLIT ? make_float4(0.f, 0.f, 0.f, 0.f) : *reinterpret_cast<const float4*>(cl + t32 * 32 + 8 * j + 4 * hh);
+        const float4 c4 = *reinterpret_cast<const float4*>(cl + t32 * 32 + 8 * j + 4 * hh);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           pt[rt][4 * j] = c4.x; pt[rt][4 * j + 1] = c4.y; pt[rt][4 * j + 2] = c4.z; pt[rt][4 * j + 3] = c4.w;
@@ -1430,26 +1278,9 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt) {
             sc[rt] = M::mma(qa[m], key_frag(rt, m0 + m), m0 + m == 0 ? kZero16 : sc[rt]);
-            if constexpr (Shape<DP, T>::SPLIT) pt[rt] = M::mma_small(ga[m], value_frag(rt, m0 + m), pt[rt]);
-            else pt[rt] = M::mma(ga[m], vf[rt][m0 + m], pt[rt]);
+            pt[rt] = M::mma(ga[m], vf[rt][m0 + m], pt[rt]);
           }
         if (Shape<DP, T>::SPLIT && DP == 64) __builtin_amdgcn_sched_barrier(0);   // (register pressure)
-      }
-      if constexpr (Shape<DP, T>::SPLIT) {   // (as in the dq kernel)
-#pragma unroll
-        for (int m = 0; m < NF; ++m)
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt)
-            pt[rt] = M::mma1(M::load_first(gl + (t32 * 32 + i) * PR + KF * m + EPL * hh), vf[rt][m].p[0], pt[rt]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float4 c4 = *reinterpret_cast<const float4*>(cl + t32 * 32 + 8 * j + 4 * hh);
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt) {
-            pt[rt][4 * j] += c4.x; pt[rt][4 * j + 1] += c4.y; pt[rt][4 * j + 2] += c4.z; pt[rt][4 * j + 3] += c4.w;
-          }
-        }
-        if (DP == 64) __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
@@ -1473,12 +1304,12 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
         if constexpr (Shape<DP, T>::SPLIT) {   // (one operand at a time: a split fragment takes twelve registers)
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt) {
-            const Frag fa = M::template from_acc<F, DP != 64>(sc[rt]);
+            const Frag fa = M::template from_acc<F>(sc[rt]);
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb)
               dv[rt][cb] = M::mma(fa, M::load(gtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh, BN), dv[rt][cb]);
             if (DP == 64) __builtin_amdgcn_sched_barrier(0);
-            const Frag wa = M::template from_acc<F, DP != 64>(pt[rt]);
+            const Frag wa = M::template from_acc<F>(pt[rt]);
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb)
               dk[rt][cb] = M::mma(wa, M::load(qtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh, BN), dk[rt][cb]);
@@ -1529,26 +1360,10 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
 
   // dk = ks dkh (dkh = the accumulated sum); sum of dkh . kh = ks sum acc . k
   const HeadRows<T> DKh = DK.head(hkv), DVh = DV.head(hkv);
-  Sum rs = 0;
+  float rs = 0.f;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     float kv[CB][16];   // (requested before the first store, as in the dq kernel)
-    float pk[CB][16], pv[CB][16];
-    if constexpr (Shape<DP, T>::ADD) {
-      const bool plus = add && tok0 / lchunk + 1 < lslots;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int pos = tok0 + (w * RT + rt) * 32 + trow(r, hh), ps = pos < nk ? pos : nk - 1;
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) {
-          pk[cb][r] = pv[cb][r] = 0.f;
-          if (plus) {
-            pk[cb][r] = to_f32(DKh.base[(unsigned)ps * DKh.pitch + (unsigned)(cb * 32 + i)]);
-            pv[cb][r] = to_f32(DVh.base[(unsigned)ps * DVh.pitch + (unsigned)(cb * 32 + i)]);
-          }
-        }
-      }
-    }
     if (rpart) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
@@ -1567,14 +1382,10 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
         for (int cb = 0; cb < CB; ++cb) {
           const int c = cb * 32 + i;
           if (c < d) {
-            float v = (dk[rt][cb][r] + dkc[cb]) * ks, vv = dv[rt][cb][r] + dvc[cb];
-            if constexpr (Shape<DP, T>::ADD) {
-              v += pk[cb][r];
-              vv += pv[cb][r];
-            }
+            const float v = (dk[rt][cb][r] + dkc[cb]) * ks;
             DKh.base[(unsigned)pos * DKh.pitch + (unsigned)c] = from_f32<T>(v);
-            DVh.base[(unsigned)pos * DVh.pitch + (unsigned)c] = from_f32<T>(vv);
-            if (rpart) rs += (Sum)v * (Sum)kv[cb][r];
+            DVh.base[(unsigned)pos * DVh.pitch + (unsigned)c] = from_f32<T>(dv[rt][cb][r] + dvc[cb]);
+            if (rpart) rs += v * kv[cb][r];
           }
         }
       }
@@ -1582,7 +1393,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
   }
   if (rpart) {
     rs = block_sum<NW>(rs, red, tid);
-    if (tid == 0) rpart[(int64_t)hkv * nb + bx] = (float)rs;
+    if (tid == 0) rpart[(int64_t)hkv * nb + bx] = rs;
   }
 }
 

@@ -1,5 +1,4 @@
-"""The fp32 moment kernels whose products run on cut operands (fastmax_amd/csrc/fm_cut.h): taken at d = 64, p = 2 once
-the heads fill the chip (heads x 256-position blocks >= 256; the state build: 3 x key/value heads >= 256).  Against
+"""The fp32 moment kernels at d = 64, p = 2 with enough heads to fill the chip (heads x 256-position blocks >= 256).  Against
 the fp64 closed form on the CPU, and against the dense kernels for what the closed form would be slow at.
 
 Tolerance: sums of n terms of about equal size round about sqrt(n) times 2^-24 of their size, n <= 1100 here, so 33
@@ -34,7 +33,7 @@ def check(got, want):
         assert_close(name, g, w, TOL)
 
 
-# (256 heads: one block each, no states at all; 128: two; 86: three; 52: five, below the build's threshold)
+# (256 heads: one block each, no states at all; 128: two; 86: three; 52: five)
 @pytest.mark.parametrize("bh,n", [(256, 40), (128, 257), (128, 512), (86, 513), (86, 769), (52, 1100)])
 @pytest.mark.parametrize("mask", [True, False])
 @pytest.mark.parametrize("normalize", [True, False])
@@ -43,7 +42,7 @@ def test_against_the_closed_form(ops, bh, n, mask, normalize):
     kw = dict(mask=mask, normalize=normalize, p=2, a0=0.7, a1=0.9, a2=0.4)
     if not normalize:
         q, k = 0.05 * q, 0.05 * k
-    print("cut states", bh, n, mask, normalize, flush=True)
+    print("many heads", bh, n, mask, normalize, flush=True)
     check(run(ops, q, k, v, go, **kw), O.dense_truth(q, k, v, go, **kw))
 
 
@@ -54,7 +53,7 @@ def test_grouped_heads_and_key_prefix(ops, bh, bhkv, nq, nk, mask):
     q, _, _, go = O.seeded_inputs((bh, nq, 64), seed=nq)
     _, k, v, _ = O.seeded_inputs((bhkv, nk, 64), seed=nk + 1)
     kw = dict(mask=mask, normalize=True, p=2)
-    print("cut states, groups", bh, bhkv, nq, nk, mask, flush=True)
+    print("many heads, groups", bh, bhkv, nq, nk, mask, flush=True)
     ratio = bh // bhkv
     o, dq, dk, dv = O.dense_truth(q, k.repeat_interleave(ratio, 0), v.repeat_interleave(ratio, 0), go, **kw)
     fold = lambda t: t.reshape(bhkv, ratio, nk, 64).sum(1)
@@ -66,7 +65,7 @@ def test_grouped_heads_and_key_prefix(ops, bh, bhkv, nq, nk, mask):
 def test_long_sequences_match_the_dense_kernels(ops, mask, monkeypatch):
     q, k, v, go = O.seeded_inputs((90, 2500, 64), seed=9)
     kw = dict(mask=mask, normalize=True, p=2)
-    print("cut states, long", mask, flush=True)
+    print("many heads, long", mask, flush=True)
     got = run(ops, q, k, v, go, **kw)
     monkeypatch.setenv("FASTMAX_PATH", "dense")
     check(got, run(ops, q, k, v, go, **kw))

@@ -1,0 +1,54 @@
+"""The bits of a training pass, pinned.  Gradients are differences: the first query's is nothing but the rounding of
+g . v - c, the arg-max row takes the rounding of a sum over the whole head, and in such rows fp32 rounding alone is 3e-5 to
+9e-5 of the gradient's rms (measured against 64 bits at 3000 to 16384 tokens).  A kernel that rounds differently is as
+good, but its gradients differ by that much from those of the same program a version ago, so a change of rounding is
+something to decide on, not something to happen: it shows here.
+
+Each row: kernel family, element type, heads, key/value heads, queries, keys, head dimension, mask, order; CRC-32 of the
+bytes of o, dq, dk, dv as gfx950 gives them (ROCm 7.2 hipcc; another compiler may contract or order differently)."""
+import zlib
+
+import pytest
+import torch
+
+from oracle import fastmax_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+MOMENTS = [
+    ("moments", "f32", 128, 128, 520, 520, 64, 1, 2, 200777920, 802387202, 2765038939, 3385367498),
+    ("moments", "f32", 128, 128, 520, 520, 64, 0, 2, 526870643, 1122425630, 2901645568, 2259476806),
+    ("moments", "f32", 172, 86, 300, 600, 64, 1, 2, 2694013926, 81666216, 1380445969, 1293252578),
+    ("moments", "f32", 256, 256, 40, 40, 64, 1, 2, 1858529247, 2990756625, 2149414697, 2616252404),
+    ("moments", "f32", 8, 8, 700, 700, 64, 1, 2, 2083562931, 448657361, 2276979092, 2301417775),
+    ("moments", "f32", 64, 64, 400, 400, 32, 1, 2, 495721487, 2824348809, 995860850, 1128627567),
+    ("moments", "f32", 64, 64, 400, 400, 32, 0, 2, 1216645763, 1943281166, 2462374411, 865680604),
+    ("moments", "f32", 64, 64, 400, 400, 64, 1, 1, 1251168654, 104178095, 3604507057, 2427487636),
+    ("moments", "f32", 64, 64, 400, 400, 64, 0, 1, 1247771956, 2822855131, 124388546, 3172592618),
+    ("moments", "bf16", 64, 64, 900, 900, 64, 1, 2, 2346293350, 2923846821, 4221794454, 1999848270),
+    ("moments", "bf16", 320, 320, 500, 500, 32, 0, 1, 3933300047, 2347415458, 3481478665, 3430664968),
+    ("moments", "bf16", 320, 320, 500, 500, 32, 1, 2, 2396040744, 37566798, 401717903, 1915638753),
+]
+
+
+def training_pass(case, save_states):
+    from fastmax_amd import ops
+
+    dtype, bh, bhkv, nq, nk, d, mask, p = case[1:9]
+    q, _, _, go = O.seeded_inputs((bh, nq, d), seed=nq + d)
+    _, k, v, _ = O.seeded_inputs((bhkv, nk, d), seed=nk + d + 1)
+    q, k, v, go = (t.to(torch.float32 if dtype == "f32" else torch.bfloat16).cuda() for t in (q, k, v, go))
+    kw = dict(mask=bool(mask), normalize=True, p=p)
+    o, den, sc, arg, *saved = ops.forward(q, k, v, save_states=save_states, **kw)
+    return (o,) + ops.backward(q, k, v, o, den, go, qk_scale=sc, qk_argmax=arg, saved_states=saved[0] if saved else None, **kw)
+
+
+@pytest.mark.parametrize("save_states", [True, False])
+@pytest.mark.parametrize("case", MOMENTS, ids=lambda c: "-".join(map(str, c[:9])))
+def test_training_pass_keeps_its_bits(built, monkeypatch, case, save_states):
+    monkeypatch.setenv("FASTMAX_PATH", case[0])
+    print("pinned bits", case[:9], save_states, flush=True)
+    got = training_pass(case, save_states)
+    crc = [zlib.crc32(t.contiguous().view(torch.uint8).cpu().numpy().tobytes()) for t in got]
+    differ = [name for name, a, b in zip(("o", "dq", "dk", "dv"), crc, case[9:]) if a != b]
+    assert not differ, f"other bits than before: {differ}"
