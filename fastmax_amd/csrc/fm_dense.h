@@ -310,19 +310,23 @@ struct TileRegs {
       }
     }
   }
-  // over the row divisor
-  __device__ __forceinline__ void store_divided(Elt* rm, int pr, Elt* tr, int pt, int tid) const {
+  // over the row divisor and times a constant each: srm for the row-major copy, str for the transposed one
+  __device__ __forceinline__ void store_scaled(Elt* rm, int pr, float srm, Elt* tr, int pt, float str, int tid) const {
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
       const int idx = tid + u * NT;
       if (idx < TOTAL) {
         const int row = idx % R, pc = idx / R;
-        float x[EPP];
+        float x[EPP], y[EPP];
         Mma<T>::unpack(raw[u], x);
-        const float inv = 1.0f / rf[u];
+        const float inv = 1.0f / rf[u], f1 = inv * srm, f2 = inv * str;
 #pragma unroll
-        for (int e = 0; e < EPP; ++e) x[e] *= inv;
-        M::put(rm ? rm + row * pr + pc * EPP : nullptr, tr ? tr + pc * EPP * pt + M::tpos(row) : nullptr, DP, pt, R, Mma<T>::pack(x));
+        for (int e = 0; e < EPP; ++e) {
+          y[e] = x[e] * f2;
+          x[e] *= f1;
+        }
+        if (rm) M::put(rm + row * pr + pc * EPP, nullptr, DP, 0, 0, Mma<T>::pack(x));
+        if (tr) M::put(nullptr, tr + pc * EPP * pt + M::tpos(row), 0, pt, R, Mma<T>::pack(y));
       }
     }
   }
@@ -604,7 +608,7 @@ __global__ __launch_bounds__(256) void dense_state_kernel(StateSide<T> sa, State
   for (int tb = t0; tb < t1; tb += BN) {
     __syncthreads();   // the previous stage has been read
     xt.store(nullptr, 0, Xt, PT, tid);
-    if (ydh) yt.store_divided(nullptr, 0, Yt, PT, tid);
+    if (ydh) yt.store_scaled(nullptr, 0, 1.0f, Yt, PT, 1.0f, tid);
     else yt.store(nullptr, 0, Yt, PT, tid);
     if (tid < BN) {
       const float e = ev * em;
@@ -1109,7 +1113,8 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
 // dk and dv.  grid = (key/value heads, key blocks of 128 RT positions); the own rows are keys, the
 // streamed rows the queries at or after them (all of them when unmasked) of every query head of the
 // group in turn.  Score tiles have rows = queries, lanes = own keys.  The streamed g rows go to LDS
-// over den, row-major and transposed (the B operand of dv).  rpart[kvhead * gridDim.y + block] = sum dkh . kh.
+// twice: times qs / den row-major (so that W comes out times qs, the factor of qh in dkh = sum W qh) and
+// times 1 / den transposed (the B operand of dv).  rpart[kvhead * gridDim.y + block] = sum dkh . kh.
 // ---------------------------------------------------------------------------------------
 template <int DP, class T, int RT, int BN, int NW>
 __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_kernel(
@@ -1131,7 +1136,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
   Elt* Gl = Ql + 2 * L::RM;                       // [2][BN][PR]
   Elt* Qt = Gl + 2 * L::RM;                       // [2][DP][PT]
   Elt* Gt = Qt + 2 * L::TR;                       // [2][DP][PT]
-  float* Cl = reinterpret_cast<float*>(Gt + 2 * L::TR);   // [2][BN]: -c of the streamed queries
+  float* Cl = reinterpret_cast<float*>(Gt + 2 * L::TR);   // [2][BN]: -qs c of the streamed queries
   float* red = Cl + 2 * BN;                       // [NW]
   fm_u4* kl2 = reinterpret_cast<fm_u4*>(red + (NW + 3) / 4 * 4);   // (KLO) [NW][NF][64]: the last parts of the key fragments
   constexpr bool KLO = Shape<DP, T>::KLO;
@@ -1180,8 +1185,8 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
     const float* denh = den.head(head);
     const float* ch = cvec.head(head);
     const float qs = qscale[head];
-    // f and qs f' of s = qs sr, where sr = q . kh is what the score tile holds (qs: dkh = sum W qh with plain q rows)
-    const float c2 = a2 * qs * qs, c1 = a1 * qs, b2 = 2.0f * a2 * qs * qs;
+    // f and f' of s = qs sr, where sr = q . kh is what the score tile holds
+    const float c2 = a2 * qs * qs, c1 = a1 * qs, b2 = 2.0f * a2 * qs;
     const int lo = Qh.lo;
     // linear mode: the queries after the block's chunk (unmasked: all queries) come as a state
     const int lc = (lstate && masked) ? tok0 / lchunk : 0;
@@ -1199,8 +1204,8 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
     };
     auto stage_store = [&](int buf) {
       qt.store(Ql + buf * L::RM, PR, Qt + buf * L::TR, PT, tid);
-      gt.store_divided(Gl + buf * L::RM, PR, Gt + buf * L::TR, PT, tid);
-      if (tid < BN) Cl[buf * BN + tid] = -creg * cmask;   // (-c: the tile's start value)
+      gt.store_scaled(Gl + buf * L::RM, PR, qs, Gt + buf * L::TR, PT, 1.0f, tid);
+      if (tid < BN) Cl[buf * BN + tid] = -creg * qs * cmask;   // (-qs c: the tile's start value)
     };
     // (requested before the state is -- one memory latency, not two -- where the registers are there: with fp32
     // fragments of 96 or 128 channels the state's own loads would be left with one register set and a wait each)
@@ -1255,7 +1260,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
     // rel == 32 rt and wholly before its keys when rel < 32 rt (its weights are then zeroed).
     auto tile = [&](int t32, int rel, const Elt* ql, const Elt* gl, const Elt* qtl, const Elt* gtl, const float* cl)
                     __attribute__((always_inline)) {
-      // tiles with rows = queries trow(r, hh), lanes = own keys: sr and g . v - c
+      // tiles with rows = queries trow(r, hh), lanes = own keys: sr and qs (g . v - c)
       f16v sc[RT], pt[RT];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1288,7 +1293,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
         for (int r = 0; r < 16; ++r) {
           const float s = sc[rt][r];
           sc[rt][r] = a0 + s * (c1 + c2 * s);
-          pt[rt][r] = (c1 + b2 * s) * pt[rt][r];
+          pt[rt][r] = (a1 + b2 * s) * pt[rt][r];
         }
         if (masked && rel <= 32 * rt) {   // (wave-uniform) a query may not lie before the key
           FM_KEEP_BRANCH();

@@ -30,6 +30,18 @@ MOMENTS = [
     ("moments", "bf16", 320, 320, 500, 500, 32, 1, 2, 2396040744, 37566798, 401717903, 1915638753),
 ]
 
+DENSE = [
+    ("dense", "bf16", 32, 8, 700, 700, 32, 1, 2, 1289423321, 2679920318, 2637797534, 2530214756),
+    ("dense", "bf16", 48, 48, 300, 300, 64, 1, 2, 1306426386, 1655945515, 1254625497, 3904682697),
+    ("dense", "bf16", 8, 8, 300, 300, 64, 0, 2, 2743260352, 1757138209, 1846273263, 3183953474),
+    ("dense", "bf16", 8, 8, 130, 400, 128, 1, 2, 3485140235, 171599824, 1488258650, 1329825502),
+    ("dense", "bf16", 8, 8, 300, 300, 96, 0, 2, 1576406631, 4144665317, 3626594233, 2899928602),
+    ("dense", "bf16", 8, 4, 1300, 1300, 64, 1, 1, 954993621, 3463860692, 2190427819, 3557732916),
+    ("dense", "f32", 8, 8, 300, 300, 128, 1, 2, 4091383673, 2457249628, 1079922644, 362090554),
+    ("dense", "f32", 8, 2, 300, 300, 96, 0, 2, 1021814443, 3537306125, 680700910, 1153882343),
+    ("dense", "f32", 4, 4, 1300, 1300, 96, 1, 1, 1231972123, 537493458, 1011557046, 1921822793),
+]
+
 
 def training_pass(case, save_states):
     from fastmax_amd import ops
@@ -44,7 +56,7 @@ def training_pass(case, save_states):
 
 
 @pytest.mark.parametrize("save_states", [True, False])
-@pytest.mark.parametrize("case", MOMENTS, ids=lambda c: "-".join(map(str, c[:9])))
+@pytest.mark.parametrize("case", MOMENTS + DENSE, ids=lambda c: "-".join(map(str, c[:9])))
 def test_training_pass_keeps_its_bits(built, monkeypatch, case, save_states):
     monkeypatch.setenv("FASTMAX_PATH", case[0])
     print("pinned bits", case[:9], save_states, flush=True)
