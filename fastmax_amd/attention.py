@@ -104,7 +104,7 @@ class FASTMultiHeadAttention_Function(torch.autograd.Function):
         need_grad = any(t.requires_grad for t in (q, k, v))
         save = need_grad and _states_fit(q3, k3, bool(mask), int(p))
         o, den, scale, arg, saved = ext.forward_ex(q3, k3, v3, bool(mask), bool(normalize), float(temperature),
-                                                   float(a0), float(a1), float(a2), float(lim), int(p), save)
+                                                   float(a0), float(a1), float(a2), float(lim), int(p), save, need_grad)
         noise = None
         out = o
         if dropout and dropout > 0.0:

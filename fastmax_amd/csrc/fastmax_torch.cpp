@@ -68,10 +68,11 @@ fastmax_stream_t current_stream(const torch::Tensor& t) {
 }
 
 // (o, den, qk_scale, qk_argmax, saved_states); o is (bh, n, d).  save_states keeps the prefix
-// states for backward_ex (a uint8 tensor; empty when not asked for)
+// states for backward_ex (a uint8 tensor; empty when not asked for).  backward_follows = false: no
+// gradients will be asked for (FASTMAX_NO_BACKWARD)
 std::vector<torch::Tensor> forward_ex(torch::Tensor q, torch::Tensor k, torch::Tensor v, bool mask,
                                       bool normalize, double temperature, double a0, double a1,
-                                      double a2, double lim, int64_t p, bool save_states) {
+                                      double a2, double lim, int64_t p, bool save_states, bool backward_follows) {
   CHECK_INPUT(q);
   CHECK_INPUT(k);
   CHECK_INPUT(v);
@@ -101,7 +102,8 @@ std::vector<torch::Tensor> forward_ex(torch::Tensor q, torch::Tensor k, torch::T
   raise_on(fastmax_forward_saving(&ds, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), ds.d,
                                   den.data_ptr<float>(), 1, scale.data_ptr<float>(), arg.data_ptr<int32_t>(),
                                   ws.data_ptr(), wsb, save_states ? saved.data_ptr() : nullptr,
-                                  (size_t)saved.numel(), current_stream(q)));
+                                  save_states || backward_follows ? (size_t)saved.numel() : FASTMAX_NO_BACKWARD,
+                                  current_stream(q)));
   return {o, den, scale, arg, saved};
 }
 
@@ -189,7 +191,7 @@ fastmax_desc make_desc5(const torch::Tensor& q, const torch::Tensor& k, bool mas
 // token-major (B, T, G, R, D) memory.
 std::vector<torch::Tensor> forward_strided(torch::Tensor q, torch::Tensor k, torch::Tensor v, bool mask,
                                            bool normalize, double temperature, double a0, double a1,
-                                           double a2, double lim, int64_t p, bool save_states) {
+                                           double a2, double lim, int64_t p, bool save_states, bool backward_follows) {
   CHECK_GPU(q);
   CHECK_GPU(k);
   CHECK_GPU(v);
@@ -224,7 +226,8 @@ std::vector<torch::Tensor> forward_strided(torch::Tensor q, torch::Tensor k, tor
   raise_on(fastmax_forward_strided(&ds, &lay, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                    den.data_ptr<float>(), 1, scale.data_ptr<float>(), arg.data_ptr<int32_t>(),
                                    ws.data_ptr(), wsb, save_states ? saved.data_ptr() : nullptr,
-                                   (size_t)saved.numel(), current_stream(q)));
+                                   save_states || backward_follows ? (size_t)saved.numel() : FASTMAX_NO_BACKWARD,
+                                   current_stream(q)));
   return {o, den, scale, arg, saved};
 }
 
@@ -385,9 +388,17 @@ PYBIND11_MODULE(fastmax_cuda, m) {
   m.def("saved_state_bytes", &saved_state_bytes, "size of the prefix states forward_ex can keep");
   m.def("backwardpass", &backwardpass, "backwardpass");
   m.def("forward_ex", &forward_ex, "forward returning (o, den, qk_scale, qk_argmax, saved_states)");
+  m.def("forward_ex", [](torch::Tensor q, torch::Tensor k, torch::Tensor v, bool mask, bool normalize, double temperature, double a0,
+                         double a1, double a2, double lim, int64_t p, bool save_states) {
+    return forward_ex(q, k, v, mask, normalize, temperature, a0, a1, a2, lim, p, save_states, true);
+  });
   m.def("backward_ex", &backward_ex, "backward through the normalisation, returns [dq, dk, dv]");
   m.def("saved_state_bytes_strided", &saved_state_bytes_strided, "the same for strided (B, G, R, T, D) / (B, G, T, D) views");
   m.def("forward_strided", &forward_strided, "forward on strided (B, G, R, T, D) / (B, G, T, D) views");
+  m.def("forward_strided", [](torch::Tensor q, torch::Tensor k, torch::Tensor v, bool mask, bool normalize, double temperature,
+                              double a0, double a1, double a2, double lim, int64_t p, bool save_states) {
+    return forward_strided(q, k, v, mask, normalize, temperature, a0, a1, a2, lim, p, save_states, true);
+  });
   m.def("backward_strided", &backward_strided, "backward on strided views, writes dq, dk, dv in place");
   m.def("version", []() { return std::string(fastmax_version()); });
 }

@@ -14,6 +14,7 @@
 #include "fastmax_amd.h"
 #include "fm_apply.h"
 #include "fm_backward.h"
+#include "fm_cut.h"
 #include "fm_decode.h"
 #include "fm_dense.h"
 #include "fm_forward.h"
@@ -945,12 +946,40 @@ int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, co
   return launch_status("dense_fwd_kernel");
 }
 
+// Forward pass on cut operands (fm_cut.h).  Blocks of four waves instead of eight while the eight-wave blocks leave CUs idle.
+template <int DP>
+int cut_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const float* q, const float* k, const float* v, float* o,
+                float* den, int64_t den_stride, const float* scale, hipStream_t stream) {
+  const int npos = pl.masked ? pl.nk : pl.nq;
+  auto launch = [&](auto nwtag) -> int {
+    constexpr int NW = decltype(nwtag)::value, BM = 32 * NW;
+    constexpr size_t smem = cut::Lds<DP>::bytes(BM);
+    static_assert(smem <= 64 * 1024, "fits the LDS a kernel gets by default");
+    const int nb = (npos + BM - 1) / BM - pl.off / BM;
+    ScopedKernel sk(FASTMAX_K_FWD_APPLY, stream);
+    cut::cut_fwd_kernel<DP, NW><<<dim3(pl.bh, nb), 64 * NW, smem, stream>>>(
+        mk_rows(q, L.q, 0, pl.off), mk_rows(k, L.k), mk_rows(v, L.v), scale, scale + pl.bh, mk_rows(o, L.o, 0, pl.off),
+        mk_scalars(den, pl.nq, den_stride, 0, pl.off), npos, pl.nk, ds->d, pl.masked, ds->a0, ds->a1, pl.p2 ? ds->a2 : 0.f, pl.ratio);
+    return launch_status("cut_fwd_kernel");
+  };
+  if ((int64_t)pl.bh * ((npos + 255) / 256) < 256) return launch(std::integral_constant<int, 4>{});
+  return launch(std::integral_constant<int, 8>{});
+}
+
 template <class T>
 int dense_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v, T* o,
-                  float* den, int64_t den_stride, float* scale_out, int32_t* arg_out, char* ws, hipStream_t stream) {
+                  float* den, int64_t den_stride, float* scale_out, int32_t* arg_out, char* ws, bool backward_follows,
+                  hipStream_t stream) {
   float* scale = scale_out ? scale_out : reinterpret_cast<float*>(ws);
   int* arg = arg_out ? arg_out : reinterpret_cast<int*>(ws + align256((size_t)2 * pl.bh * sizeof(float)));
   FM_TRY(compute_scales<T>(ds, L, q, k, scale, arg, stream));
+  if constexpr (std::is_same<T, float>::value) {
+    // (96 and 128 channels: two stages of cut rows do not fit the LDS two blocks share; the linear mode of p = 1 spends
+    // its time on states, not on tiles)
+    if (!backward_follows && ds->d <= 64 && !pl.lin)
+      return ds->d <= 32 ? cut_forward<32>(ds, pl, L, q, k, v, o, den, den_stride, scale, stream)
+                         : cut_forward<64>(ds, pl, L, q, k, v, o, den, den_stride, scale, stream);
+  }
   float* kstate = reinterpret_cast<float*>(ws + align256((size_t)2 * pl.bh * sizeof(float)) + align256((size_t)2 * pl.bh * sizeof(int)));
 #define FM_DENSE_FWD(DP) return dense_forward_dp<DP, T>(ds, pl, L, q, k, v, o, den, den_stride, scale, kstate, stream)
   if (ds->d <= 32) FM_DENSE_FWD(32);
@@ -1001,8 +1030,7 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
   {
     constexpr int RT = S::RT_KV, NW = S::NW_KV, BM = 32 * RT * NW, BNK = S::BN_KV;
     static_assert(256 % BM == 0 && 256 % BNK == 0, "blocks and stages do not straddle the chunks of the linear mode");
-    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + (NW + 3) / 4 * 4) +
-                        (S::KLO ? (size_t)NW * (DP / dense::Policy<DP, T>::KF) * 64 * sizeof(fm_u4) : 0);
+    const size_t smem = dense::Lds<DP, T, BNK>::bytes(2, 2, 2 * BNK + NW);
     auto kern = dense::dense_dkdv_kernel<DP, T, RT, BNK, NW>;
     FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
     const int nb = (pl.nk + BM - 1) / BM;
@@ -1281,11 +1309,12 @@ static int forward_entry(const fastmax_desc* desc, const fastmax_layout* layout,
   char* ws = static_cast<char*>(workspace);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (pl.dense) {
+    const bool backward_follows = saved_states || saved_bytes != FASTMAX_NO_BACKWARD;
     if (desc->dtype == FASTMAX_F32)
       return dense_forward<float>(desc, pl, L, (const float*)q, (const float*)k, (const float*)v, (float*)o, den,
-                                  den_stride, qk_scale, qk_argmax, ws, st);
+                                  den_stride, qk_scale, qk_argmax, ws, backward_follows, st);
     return dense_forward<bf16_t>(desc, pl, L, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)o, den,
-                                 den_stride, qk_scale, qk_argmax, ws, st);
+                                 den_stride, qk_scale, qk_argmax, ws, backward_follows, st);
   }
 #define FM_FWD(DD, TT)                                                                             \
   return forward_impl<DD, TT>(desc, pl, L, (const TT*)q, (const TT*)k, (const TT*)v, (TT*)o, den, \

@@ -43,7 +43,7 @@ struct Mma<bf16_t> {
   static constexpr int EPL = 8;    // elements per lane and fragment
   static constexpr int KF = 16;    // contraction length of a fragment step
   static constexpr int PAD = 8;    // row padding of LDS tiles (elements): 16 bytes, conflict-free 128-bit rows
-  static constexpr int PLANES = 1; // elements of an LDS row per element of the tensor row
+  static __device__ __forceinline__ Frag zero() { return Frag{0u, 0u, 0u, 0u}; }
   static __device__ __forceinline__ f16v mma(const Frag& a, const Frag& b, const f16v& c) {
     return FM_MFMA_BF16(__builtin_bit_cast(bf8v, a), __builtin_bit_cast(bf8v, b), c);
   }
@@ -60,8 +60,7 @@ struct Mma<bf16_t> {
     return (x & ~15) | (((x >> 2) & 1) << 3) | (((x >> 3) & 1) << 2) | (x & 3);
   }
   // acc + the sum of the fragment's elements, as rounded
-  template <int F>
-  static __device__ __forceinline__ float fsum(const f16v&, const Frag& w, float acc) {
+  static __device__ __forceinline__ float fsum(const Frag& w, float acc) {
     acc = fm_dot2_bf16(w.x, 0x3f803f80u, acc);
     acc = fm_dot2_bf16(w.y, 0x3f803f80u, acc);
     acc = fm_dot2_bf16(w.z, 0x3f803f80u, acc);
@@ -78,20 +77,7 @@ struct Mma<bf16_t> {
     const uint32_t w = e < 2 ? r.x : e < 4 ? r.y : e < 6 ? r.z : r.w;
     return (Elt)((e & 1) ? (w >> 16) : w);
   }
-  static __device__ __forceinline__ Frag load(const Elt* p, int) { return *reinterpret_cast<const Frag*>(p); }
-  static __device__ __forceinline__ Frag make(const float (&x)[8]) { return __builtin_bit_cast(Frag, pack(x)); }
-  static __device__ __forceinline__ void values(const Frag& f, float (&o)[8]) { unpack(__builtin_bit_cast(uint4, f), o); }
-  // a 16-byte piece of a tensor row into an LDS row / down an LDS column of pitch pt (plane: see MmaSplit)
-  static __device__ __forceinline__ void put(Elt* row, Elt* col, int, int pt, int, const uint4& raw) {
-    if (row) *reinterpret_cast<uint4*>(row) = raw;
-    if (col) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) col[e * pt] = elt(raw, e);
-    }
-  }
-  static __device__ __forceinline__ void put4(Elt* p, int, const float4& v) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf2(v.x, v.y), pack_bf2(v.z, v.w));
-  }
+  static __device__ __forceinline__ Elt to_elt(float v) { return (Elt)pack_bf2(v, 0.f); }
 };
 
 template <>
@@ -101,7 +87,7 @@ struct Mma<float> {
   static constexpr int EPL = 4;
   static constexpr int KF = 8;
   static constexpr int PAD = 4;
-  static constexpr int PLANES = 1;
+  static __device__ __forceinline__ Frag zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
   static __device__ __forceinline__ f16v mma(const Frag& a, const Frag& b, f16v c) {
     c = FM_MFMA(a.x, b.x, c);
     c = FM_MFMA(a.y, b.y, c);
@@ -114,8 +100,7 @@ struct Mma<float> {
     return make_float4(a[4 * F], a[4 * F + 1], a[4 * F + 2], a[4 * F + 3]);
   }
   static __device__ __forceinline__ int tpos(int x) { return x; }
-  template <int F>
-  static __device__ __forceinline__ float fsum(const f16v&, const Frag& w, float acc) { return acc + ((w.x + w.y) + (w.z + w.w)); }
+  static __device__ __forceinline__ float fsum(const Frag& w, float acc) { return acc + ((w.x + w.y) + (w.z + w.w)); }
   static __device__ __forceinline__ void unpack(const uint4& r, float (&o)[4]) {
     o[0] = __uint_as_float(r.x); o[1] = __uint_as_float(r.y); o[2] = __uint_as_float(r.z); o[3] = __uint_as_float(r.w);
   }
@@ -125,123 +110,8 @@ struct Mma<float> {
   static __device__ __forceinline__ Elt elt(const uint4& r, int e) {
     return __uint_as_float(e == 0 ? r.x : e == 1 ? r.y : e == 2 ? r.z : r.w);
   }
-  static __device__ __forceinline__ Frag load(const Elt* p, int) { return *reinterpret_cast<const Frag*>(p); }
-  static __device__ __forceinline__ Frag make(const float (&x)[4]) { return make_float4(x[0], x[1], x[2], x[3]); }
-  static __device__ __forceinline__ void values(const Frag& f, float (&o)[4]) { unpack(__builtin_bit_cast(uint4, f), o); }
-  static __device__ __forceinline__ void put(Elt* row, Elt* col, int, int pt, int, const uint4& raw) {
-    if (row) *reinterpret_cast<uint4*>(row) = raw;
-    if (col) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) col[e * pt] = elt(raw, e);
-    }
-  }
-  static __device__ __forceinline__ void put4(Elt* p, int, const float4& v) { *reinterpret_cast<float4*>(p) = v; }
+  static __device__ __forceinline__ Elt to_elt(float v) { return v; }
 };
-
-// fp32 contractions on the bf16 matrix instruction.  Every operand is cut into three bf16 parts, each the
-// nearest bf16 value of what the parts before it leave: 3 x 8 significand bits and the signs of the parts hold
-// all 24 bits of the float.  Of the nine products of parts the six of order 2^-18 and above are formed
-// (accumulated in fp32, smallest first); what is left out is below 2^-26 of a product, a quarter of what rounding
-// that product to fp32 costs, and a step of 16 products rounds the accumulator six times instead of sixteen.
-// A non-finite operand gives a non-finite result (infinite minus infinite parts: not a number).
-// Six v_mfma_f32_32x32x16_bf16 take ~200 cycles where eight v_mfma_f32_32x32x2f32 take 512.  The parts of streamed
-// rows are formed once per block on their way into LDS (three planes per row), those of own rows once per
-// wave; only the weights are cut up per tile.
-// Measured (forward + backward, fp32, causal, 512 heads x 1000 x 32): 1403 us with the fp32 instruction, 1047 so;
-// forward only, unmasked, 512 heads x 1000 x 64: 1164 and 794.  The error against 64 bits falls by 10 to 30 %.
-struct SplitFrag {
-  fm_u4 p[3];
-};
-struct MmaSplit {
-  using Elt = uint16_t;
-  using Frag = SplitFrag;
-  static constexpr int EPL = 8, KF = 16, PAD = 8, PLANES = 3;
-  static __device__ __forceinline__ f16v mma1(const fm_u4& a, const fm_u4& b, const f16v& c) {
-    return FM_MFMA_BF16(__builtin_bit_cast(bf8v, a), __builtin_bit_cast(bf8v, b), c);
-  }
-  static __device__ __forceinline__ f16v mma(const Frag& a, const Frag& b, f16v c) {
-    c = mma1(a.p[2], b.p[0], c);
-    c = mma1(a.p[0], b.p[2], c);
-    c = mma1(a.p[1], b.p[1], c);
-    c = mma1(a.p[1], b.p[0], c);
-    c = mma1(a.p[0], b.p[1], c);
-    return mma1(a.p[0], b.p[0], c);
-  }
-  // the three parts of a pair of floats, packed
-  static __device__ __forceinline__ void cut(float x, float y, uint32_t (&w)[3]) {
-    w[0] = pack_bf2(x, y);
-    x -= bf_lo(w[0]);
-    y -= bf_hi(w[0]);
-    w[1] = pack_bf2(x, y);
-    x -= bf_lo(w[1]);
-    y -= bf_hi(w[1]);
-    w[2] = pack_bf2(x, y);
-  }
-  static __device__ __forceinline__ Frag make(const float (&x)[8]) {
-    Frag f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint32_t w[3];
-      cut(x[2 * e], x[2 * e + 1], w);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) f.p[k][e] = w[k];
-    }
-    return f;
-  }
-  static __device__ __forceinline__ void values(const Frag& f, float (&o)[8]) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o[2 * e] = (bf_lo(f.p[2][e]) + bf_lo(f.p[1][e])) + bf_lo(f.p[0][e]);
-      o[2 * e + 1] = (bf_hi(f.p[2][e]) + bf_hi(f.p[1][e])) + bf_hi(f.p[0][e]);
-    }
-  }
-  template <int F>
-  static __device__ __forceinline__ Frag from_acc(const f16v& a) {
-    const float x[8] = {a[8 * F], a[8 * F + 1], a[8 * F + 2], a[8 * F + 3], a[8 * F + 4], a[8 * F + 5], a[8 * F + 6], a[8 * F + 7]};
-    return make(x);
-  }
-  template <int F>
-  static __device__ __forceinline__ float fsum(const f16v& a, const Frag&, float acc) {
-    return acc + (((a[8 * F] + a[8 * F + 1]) + (a[8 * F + 2] + a[8 * F + 3])) +
-                  ((a[8 * F + 4] + a[8 * F + 5]) + (a[8 * F + 6] + a[8 * F + 7])));
-  }
-  static __device__ __forceinline__ int tpos(int x) { return Mma<bf16_t>::tpos(x); }
-  // an LDS row holds its three planes one after another, `plane` elements apart
-  static __device__ __forceinline__ Frag load(const Elt* p, int plane) {
-    Frag f;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) f.p[k] = *reinterpret_cast<const fm_u4*>(p + k * plane);
-    return f;
-  }
-  static __device__ __forceinline__ void put(Elt* row, Elt* col, int rplane, int pt, int cplane, const uint4& raw) {
-    uint32_t a[3], b[3];
-    cut(__uint_as_float(raw.x), __uint_as_float(raw.y), a);
-    cut(__uint_as_float(raw.z), __uint_as_float(raw.w), b);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      if (row) *reinterpret_cast<uint2*>(row + k * rplane) = make_uint2(a[k], b[k]);
-      if (col) {
-        Elt* c = col + k * cplane;
-        c[0] = (Elt)a[k];
-        c[pt] = (Elt)(a[k] >> 16);
-        c[2 * pt] = (Elt)b[k];
-        c[3 * pt] = (Elt)(b[k] >> 16);
-      }
-    }
-  }
-  static __device__ __forceinline__ void put4(Elt* p, int plane, const float4& v) {
-    put(p, nullptr, plane, 0, 0, make_uint4(__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)));
-  }
-};
-
-// The policy of the forward, dq and dk / dv kernels.  (fp32 with 96 or 128 channels: two stages of split rows in both
-// layouts do not fit the 160 KB of LDS, so those stay on the fp32 instruction.)
-template <int DP, class T>
-struct PolicyOf {
-  using type = typename std::conditional<std::is_same<T, float>::value && DP <= 64, MmaSplit, Mma<T>>::type;
-};
-template <int DP, class T>
-using Policy = typename PolicyOf<DP, T>::type;
 
 // The per-element mask tests of a score tile sit in blocks that only the diagonal and the ragged last tiles
 // enter (a wave-uniform condition).  Left alone the compiler turns such a block into selects that every tile
@@ -269,11 +139,17 @@ __device__ __forceinline__ float block_sum(float v, float* red, int tid) {
 __device__ __forceinline__ float to_f32_elt(float v) { return v; }
 __device__ __forceinline__ float to_f32_elt(uint16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
 
+template <class T>
+__device__ __forceinline__ typename Mma<T>::Frag lds_frag(const typename Mma<T>::Elt* p) {
+  return *reinterpret_cast<const typename Mma<T>::Frag*>(p);
+}
+
 // R rows x DP channels of one head on their way global -> registers -> LDS, by the NT threads of a block.
 // Consecutive threads take consecutive rows (16 bytes of a row each), which makes both the row-major
 // and the transposed LDS writes conflict-free.  Rows outside [lo, pend) and channels past d are zero.
-template <int DP, class T, int R, int NT, class M>
+template <int DP, class T, int R, int NT>
 struct TileRegs {
+  using M = Mma<T>;
   using Elt = typename M::Elt;
   static constexpr int EPP = 16 / (int)sizeof(T);   // elements per 16-byte piece
   static constexpr int PPR = DP / EPP;
@@ -306,7 +182,12 @@ struct TileRegs {
       const int idx = tid + u * NT;
       if (idx < TOTAL) {
         const int row = idx % R, pc = idx / R;
-        M::put(rm ? rm + row * pr + pc * EPP : nullptr, tr ? tr + pc * EPP * pt + M::tpos(row) : nullptr, DP, pt, R, raw[u]);
+        if (rm) *reinterpret_cast<uint4*>(rm + row * pr + pc * EPP) = raw[u];
+        if (tr) {
+          Elt* t0 = tr + pc * EPP * pt + M::tpos(row);
+#pragma unroll
+          for (int e = 0; e < EPP; ++e) t0[e * pt] = M::elt(raw[u], e);
+        }
       }
     }
   }
@@ -318,15 +199,20 @@ struct TileRegs {
       if (idx < TOTAL) {
         const int row = idx % R, pc = idx / R;
         float x[EPP], y[EPP];
-        Mma<T>::unpack(raw[u], x);
+        M::unpack(raw[u], x);
         const float inv = 1.0f / rf[u], f1 = inv * srm, f2 = inv * str;
 #pragma unroll
         for (int e = 0; e < EPP; ++e) {
           y[e] = x[e] * f2;
           x[e] *= f1;
         }
-        if (rm) M::put(rm + row * pr + pc * EPP, nullptr, DP, 0, 0, Mma<T>::pack(x));
-        if (tr) M::put(nullptr, tr + pc * EPP * pt + M::tpos(row), 0, pt, R, Mma<T>::pack(y));
+        if (rm) *reinterpret_cast<uint4*>(rm + row * pr + pc * EPP) = M::pack(x);
+        if (tr) {
+          const uint4 yt = M::pack(y);
+          Elt* t0 = tr + pc * EPP * pt + M::tpos(row);
+#pragma unroll
+          for (int e = 0; e < EPP; ++e) t0[e * pt] = M::elt(yt, e);
+        }
       }
     }
   }
@@ -334,37 +220,33 @@ struct TileRegs {
 
 // The fragments of one own row (position pos of the head), times `scale`: fragment m holds channels
 // KF m + EPL hh .. + EPL - 1.  A row outside [lo, pend) gives zeros, and so do channels past d.
-template <int DP, class T, class M>
+template <int DP, class T>
 __device__ __forceinline__ void load_own_frags(const HeadRows<const T>& hr, int pos, int pend, int d, int hh, float scale,
-                                               typename M::Frag (&f)[DP / M::KF]) {
-  constexpr int EPP = 16 / (int)sizeof(T), NP = M::EPL / EPP;   // 16-byte pieces of the row per fragment
+                                               typename Mma<T>::Frag (&f)[DP / Mma<T>::KF]) {
+  using M = Mma<T>;
   const bool live = pos >= hr.lo && pos < pend;
   const int ps = max(pos < pend ? pos : pend - 1, hr.lo);
   const T* row = hr.base + (unsigned)ps * hr.pitch;
 #pragma unroll
   for (int m = 0; m < DP / M::KF; ++m) {
+    const int ch = M::KF * m + M::EPL * hh;
+    const bool ok = live && ch < d;
+    const uint4 t = *reinterpret_cast<const uint4*>(row + (ok ? ch : 0));
     float x[M::EPL];
+    M::unpack(t, x);
 #pragma unroll
-    for (int u = 0; u < NP; ++u) {
-      const int ch = M::KF * m + M::EPL * hh + EPP * u;
-      const bool ok = live && ch < d;
-      const uint4 t = *reinterpret_cast<const uint4*>(row + (ok ? ch : 0));
-      float y[EPP];
-      Mma<T>::unpack(t, y);
-#pragma unroll
-      for (int e = 0; e < EPP; ++e) x[EPP * u + e] = ok ? y[e] * scale : 0.f;
-    }
-    f[m] = M::make(x);
+    for (int e = 0; e < M::EPL; ++e) x[e] = ok ? x[e] * scale : 0.f;
+    f[m] = __builtin_bit_cast(typename M::Frag, M::pack(x));
   }
 }
 
 // The own-row fragments of g = grad_out / den for position pos, and c = grad_out . out / den of that row (the lane
 // half's channels summed with the other half's): what a separate pass over grad_out and out would leave in memory.
-template <int DP, class T, class M>
+template <int DP, class T>
 __device__ __forceinline__ float load_g_frags_and_c(const HeadRows<const T>& gr, const HeadRows<const T>& orow, int pos,
                                                     int pend, int d, int hh, float rden,
-                                                    typename M::Frag (&f)[DP / M::KF]) {
-  constexpr int EPP = 16 / (int)sizeof(T), NP = M::EPL / EPP;
+                                                    typename Mma<T>::Frag (&f)[DP / Mma<T>::KF]) {
+  using M = Mma<T>;
   const bool live = pos >= gr.lo && pos < pend;
   const int ps = max(pos < pend ? pos : pend - 1, gr.lo);
   const T* grow = gr.base + (unsigned)ps * gr.pitch;
@@ -372,23 +254,19 @@ __device__ __forceinline__ float load_g_frags_and_c(const HeadRows<const T>& gr,
   float dot = 0.f;
 #pragma unroll
   for (int m = 0; m < DP / M::KF; ++m) {
-    float x[M::EPL];
+    const int ch = M::KF * m + M::EPL * hh;
+    const bool ok = live && ch < d;
+    const uint4 tg = *reinterpret_cast<const uint4*>(grow + (ok ? ch : 0));
+    const uint4 to = *reinterpret_cast<const uint4*>(orw + (ok ? ch : 0));
+    float x[M::EPL], y[M::EPL];
+    M::unpack(tg, x);
+    M::unpack(to, y);
 #pragma unroll
-    for (int u = 0; u < NP; ++u) {
-      const int ch = M::KF * m + M::EPL * hh + EPP * u;
-      const bool ok = live && ch < d;
-      const uint4 tg = *reinterpret_cast<const uint4*>(grow + (ok ? ch : 0));
-      const uint4 to = *reinterpret_cast<const uint4*>(orw + (ok ? ch : 0));
-      float g[EPP], y[EPP];
-      Mma<T>::unpack(tg, g);
-      Mma<T>::unpack(to, y);
-#pragma unroll
-      for (int e = 0; e < EPP; ++e) {
-        dot += ok ? g[e] * y[e] : 0.f;
-        x[EPP * u + e] = ok ? g[e] * rden : 0.f;
-      }
+    for (int e = 0; e < M::EPL; ++e) {
+      dot += ok ? x[e] * y[e] : 0.f;
+      x[e] = ok ? x[e] * rden : 0.f;
     }
-    f[m] = M::make(x);
+    f[m] = __builtin_bit_cast(typename M::Frag, M::pack(x));
   }
   return (dot + __shfl_xor(dot, 32, 64)) * rden;
 }
@@ -397,9 +275,9 @@ __device__ __forceinline__ float load_g_frags_and_c(const HeadRows<const T>& gr,
 // buffers, then `tail` floats.
 template <int DP, class T, int BN>
 struct Lds {
-  using M = Policy<DP, T>;
-  static constexpr int PR = M::PLANES * DP + M::PAD;   // pitch of row-major tiles (elements)
-  static constexpr int PT = M::PLANES * BN + M::PAD;   // pitch of transposed tiles
+  using M = Mma<T>;
+  static constexpr int PR = DP + M::PAD;   // pitch of row-major tiles (elements)
+  static constexpr int PT = BN + M::PAD;   // pitch of transposed tiles
   static constexpr int RM = BN * PR;       // elements of a row-major tile
   static constexpr int TR = DP * PT;       // elements of a transposed tile
   static constexpr size_t bytes(int na, int nt, int tail_floats) {
@@ -420,21 +298,16 @@ struct Shape {
   // Waves per block.  Staging a stage of streamed rows costs a block the same whatever its size, so the
   // backward kernels, whose stages are the costliest (four staged tiles, one of them rescaled), run eight
   // waves on it where the registers allow two waves per SIMD.
-  // operand fragments read ahead at a time (a split one takes twelve registers)
-  static constexpr int HC = (BF && DP % 64 == 0) ? 4 : (std::is_same<Policy<DP, T>, MmaSplit>::value && DP == 64) ? 1 : 2;
-  static constexpr bool SPLIT = std::is_same<Policy<DP, T>, MmaSplit>::value;
-  static constexpr int NW_FWD = ((BF && DP == 64) || SPLIT) ? 8 : 4;
-  static constexpr int NW_DQ = ((BF && DP == 64) || SPLIT) ? 8 : 4;
-  static constexpr int NW_KV = ((BF && DP == 64) || SPLIT) ? 8 : 4;
-  // the dk / dv kernel keeps the last parts of its own key fragments in LDS (16 registers that 64 channels lack)
-  static constexpr bool KLO = SPLIT && DP == 64;
+  static constexpr int NW_FWD = (BF && DP == 64) ? 8 : 4;
+  static constexpr int NW_DQ = (BF && DP == 64) ? 8 : 4;
+  static constexpr int NW_KV = (BF && DP == 64) ? 8 : 4;
   static constexpr int RT_FWD = 1;
   static constexpr int RT_DQ = 1;
   static constexpr int RT_KV = 1;
   // resident blocks per CU each kernel is built for (fp32 operand fragments take twice the registers)
-  static constexpr int OCC_FWD = SPLIT ? (DP == 32 ? 2 : 1) : (BF && DP == 64) ? 2 : (BF && DP <= 32) ? 3 : (DP <= 32) ? 2 : 1;
-  static constexpr int OCC_DQ = SPLIT ? (DP == 32 ? 2 : 1) : (BF && DP == 64) ? 2 : (DP <= 32) ? 2 : 1;   // (8-wave blocks: one is two waves per SIMD)
-  static constexpr int OCC_KV = SPLIT ? (DP == 32 ? 2 : 1) : (BF && DP == 64) ? 1 : (DP <= 32) ? 2 : 1;
+  static constexpr int OCC_FWD = (BF && DP == 64) ? 2 : (BF && DP <= 32) ? 3 : (DP <= 32) ? 2 : 1;
+  static constexpr int OCC_DQ = (BF && DP == 64) ? 2 : (DP <= 32) ? 2 : 1;   // (8-wave blocks: one is two waves per SIMD)
+  static constexpr int OCC_KV = (BF && DP == 64) ? 1 : (DP <= 32) ? 2 : 1;
 };
 
 // ---------------------------------------------------------------------------------------
@@ -498,15 +371,19 @@ __global__ __launch_bounds__(256) void lin_scan_kernel(float* __restrict__ sa, i
   if (mode == 2) *reinterpret_cast<float4*>(base) = run;
 }
 
-// One block of a state on its way into LDS as a matrix operand: DP rows of DP elements, pitch PLANES DP + PAD.
+__device__ __forceinline__ void lin_store4(float* p, const float4& v) { *reinterpret_cast<float4*>(p) = v; }
+__device__ __forceinline__ void lin_store4(uint16_t* p, const float4& v) {
+  *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf2(v.x, v.y), pack_bf2(v.z, v.w));
+}
+
+// One block of a state on its way into LDS as a matrix operand: DP rows of DP elements, pitch DP + PAD.
 // Up to eight 16-byte loads per thread are in flight before the first is used.
 template <int DP, class T, int NT>
-__device__ __forceinline__ void lin_stage_block(const float* __restrict__ g, typename Policy<DP, T>::Elt* l, int tid) {
-  using M = Policy<DP, T>;
-  constexpr int PS = M::PLANES * DP + M::PAD, LD = LinState<DP>::LD, V4 = DP / 4, TOTAL = DP * V4, NV = (TOTAL + NT - 1) / NT;
+__device__ __forceinline__ void lin_stage_block(const float* __restrict__ g, typename Mma<T>::Elt* l, int tid) {
+  using M = Mma<T>;
+  constexpr int PS = DP + M::PAD, LD = LinState<DP>::LD, V4 = DP / 4, TOTAL = DP * V4, NV = (TOTAL + NT - 1) / NT;
   constexpr int B = NV < 8 ? NV : 8;
-  static_assert(TOTAL % NT == 0 || TOTAL < NT, "every thread moves the same number of pieces, or at most one");
-  if (TOTAL < NT && tid >= TOTAL) return;
+  static_assert(TOTAL % NT == 0, "every thread moves the same number of pieces");
   static_for<(NV + B - 1) / B>([&](auto btag) {
     constexpr int U0 = decltype(btag)::value * B, N = NV - U0 < B ? NV - U0 : B;
     float4 t[N];
@@ -518,7 +395,7 @@ __device__ __forceinline__ void lin_stage_block(const float* __restrict__ g, typ
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const int idx = tid + (U0 + u) * NT;
-      M::put4(l + (idx / V4) * PS + (idx % V4) * 4, DP, t[u]);
+      lin_store4(l + (idx / V4) * PS + (idx % V4) * 4, t[u]);
     }
   });
 }
@@ -526,12 +403,12 @@ __device__ __forceinline__ void lin_stage_block(const float* __restrict__ g, typ
 // t + (own rows x DP, fragments af) . B, where brow is the LDS row that holds output column i's DP
 // contraction elements, already offset by the lane half's EPL hh
 template <int DP, class T>
-__device__ __forceinline__ f16v lin_own_times(const typename Policy<DP, T>::Frag (&af)[DP / Policy<DP, T>::KF],
-                                              const typename Policy<DP, T>::Elt* brow, f16v t) {
-  using M = Policy<DP, T>;
+__device__ __forceinline__ f16v lin_own_times(const typename Mma<T>::Frag (&af)[DP / Mma<T>::KF],
+                                              const typename Mma<T>::Elt* brow, f16v t) {
+  using M = Mma<T>;
 #pragma unroll
   for (int m0 = 0; m0 < DP / M::KF; m0 += 2) {   // (two operand reads in flight, not all of them: register pressure)
-    const typename M::Frag b0 = M::load(brow + M::KF * m0, DP), b1 = M::load(brow + M::KF * (m0 + 1), DP);
+    const typename M::Frag b0 = lds_frag<T>(brow + M::KF * m0), b1 = lds_frag<T>(brow + M::KF * (m0 + 1));
     t = M::mma(af[m0], b0, t);
     t = M::mma(af[m0 + 1], b1, t);
     __builtin_amdgcn_sched_barrier(0);
@@ -594,7 +471,7 @@ __global__ __launch_bounds__(256) void dense_state_kernel(StateSide<T> sa, State
   }
   float esum = 0.f;   // threads < BN: sum of e over the positions tb + tid of every stage
 
-  TileRegs<DP, T, BN, 256, M> xt, yt;
+  TileRegs<DP, T, BN, 256> xt, yt;
   float ev = 1.0f, em = 0.f;   // e of the position this thread stages, as loaded, and whether the position exists
   auto stage_load = [&](int tb) {
     xt.load(Xh, tb, t1, d, tid);
@@ -624,8 +501,8 @@ __global__ __launch_bounds__(256) void dense_state_kernel(StateSide<T> sa, State
         const int rb = tile / CB, cb = (tile % CB + rb) % CB;   // (skewed: every wave gets its share of the summing tiles)
 #pragma unroll
         for (int f = 0; f < BN / KF; ++f) {
-          const Frag a = M::load(Xt + (rb * 32 + i) * PT + KF * f + EPL * hh, BN);
-          const Frag b = M::load(Yt + (cb * 32 + i) * PT + KF * f + EPL * hh, BN);
+          const Frag a = lds_frag<T>(Xt + (rb * 32 + i) * PT + KF * f + EPL * hh);
+          const Frag b = lds_frag<T>(Yt + (cb * 32 + i) * PT + KF * f + EPL * hh);
           acc[t] = M::mma(a, b, acc[t]);
           if (cb == 0) {
             float x[EPL];
@@ -687,15 +564,15 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
     Rows<const T> Q, Rows<const T> K, Rows<const T> V, const float* __restrict__ qscale,
     const float* __restrict__ kscale, Rows<T> O, RowScalarsOut den, int npos, int nk, int d, int masked, float a0,
     float a1, float a2, int ratio, const float* __restrict__ lstate, int lchunk, int lslots) {
-  using M = Policy<DP, T>;
+  using M = Mma<T>;
   using Elt = typename M::Elt;
   using Frag = typename M::Frag;
   using L = Lds<DP, T, BN>;
   constexpr int KF = M::KF, EPL = M::EPL, NF = DP / KF, CB = DP / 32, NFA = 32 / KF, NT = 64 * NW, BM = 32 * RT * NW;
-  constexpr int HC = Shape<DP, T>::HC;   // operand fragments read ahead at a time
+  constexpr int HC = (Shape<DP, T>::BF && NF % 4 == 0) ? 4 : 2;   // operand fragments read ahead at a time
   static_assert(NF % HC == 0, "whole groups of fragments");
   constexpr int PR = L::PR, PT = L::PT;
-  static_assert(L::bytes(1, 1, 0) >= (size_t)DP * (M::PLANES * DP + M::PAD) * sizeof(Elt) + 2 * DP * sizeof(float), "a state fits the stage buffers");
+  static_assert(L::bytes(1, 1, 0) >= (size_t)DP * (DP + M::PAD) * sizeof(Elt) + 2 * DP * sizeof(float), "a state fits the stage buffers");
   extern __shared__ __attribute__((aligned(16))) unsigned char dense_smem[];
   Elt* Kl = reinterpret_cast<Elt*>(dense_smem);   // [2][BN][PR]
   Elt* Vt = Kl + 2 * L::RM;                       // [2][DP][PT]
@@ -713,14 +590,14 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
 
   Frag qf[RT][NF];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) load_own_frags<DP, T, M>(Qh, tok0 + (w * RT + rt) * 32 + i, npos, d, hh, kq, qf[rt]);
+  for (int rt = 0; rt < RT; ++rt) load_own_frags<DP, T>(Qh, tok0 + (w * RT + rt) * 32 + i, npos, d, hh, kq, qf[rt]);
 
   const int kend = masked ? (tok0 + BM < nk ? tok0 + BM : nk) : nk;
   const int nst = (kend + BN - 1) / BN;
   // linear mode: the keys before the block's chunk (unmasked: all keys) come as a state
   const int lc = (lstate && masked) ? tok0 / lchunk : 0;
   const int st0 = lstate ? (masked ? lc * (lchunk / BN) : nst) : 0;
-  TileRegs<DP, T, BN, NT, M> kt, vt;
+  TileRegs<DP, T, BN, NT> kt, vt;
   auto stage_load = [&](int st) {
     kt.load(Kh, st * BN, nk, d, tid);
     vt.load(Vh, st * BN, nk, d, tid);
@@ -744,7 +621,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
   if (st0 < nst) stage_load(st0);   // (requested before the state is: one memory latency, not two)
   if (lstate && (!masked || lc > 0)) {
     // o += a1 qh . S1 + a0 sum v,  den += a1 qh . sum k + a0 count   (S1 = sum k (x) v of the keys in the state)
-    constexpr int PS = M::PLANES * DP + M::PAD;
+    constexpr int PS = DP + M::PAD;
     Elt* St = reinterpret_cast<Elt*>(dense_smem);             // a1 S1 as [value channel][key channel]
     float* sk = reinterpret_cast<float*>(St + DP * PS);       // sum k
     float* sv = sk + DP;                                      // sum v
@@ -767,7 +644,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
 #pragma unroll
       for (int m = 0; m < NF; ++m) {
         float x[EPL];
-        M::values(qf[rt][m], x);
+        M::unpack(__builtin_bit_cast(uint4, qf[rt][m]), x);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) dd += x[e] * sk[KF * m + EPL * hh + e];
       }
@@ -787,14 +664,14 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
 #pragma unroll
     for (int f = 0; f < NFA; ++f)
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) vb[f][cb] = M::load(vl + (cb * 32 + i) * PT + t32 * 32 + KF * f + EPL * hh, BN);
+      for (int cb = 0; cb < CB; ++cb) vb[f][cb] = lds_frag<T>(vl + (cb * 32 + i) * PT + t32 * 32 + KF * f + EPL * hh);
     // scores, transposed: rows = keys trow(r, hh), lanes = own queries
     f16v sc[RT];
 #pragma unroll
     for (int m0 = 0; m0 < NF; m0 += HC) {   // (HC operand fragments are read ahead of the instructions that use them)
       Frag ka[HC];
 #pragma unroll
-      for (int m = 0; m < HC; ++m) ka[m] = M::load(kl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh, DP);
+      for (int m = 0; m < HC; ++m) ka[m] = lds_frag<T>(kl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh);
 #pragma unroll
       for (int m = 0; m < HC; ++m)
 #pragma unroll
@@ -828,7 +705,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_FWD)) void dense_fwd_ke
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         wa[rt] = M::template from_acc<F>(sc[rt]);
-        dn[rt] = M::template fsum<F>(sc[rt], wa[rt], dn[rt]);
+        dn[rt] = M::fsum(wa[rt], dn[rt]);
       }
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb)
@@ -893,15 +770,15 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
     const float* __restrict__ qscale, const float* __restrict__ kscale, Rows<T> DQ, float* __restrict__ rpart,
     int npos, int nk, int d, int masked, int p2, float a1, float a2, int ratio, const float* __restrict__ lstate,
     int lchunk, int lslots, Rows<const T> OUTF, RowScalarsOut cprep) {
-  using M = Policy<DP, T>;
+  using M = Mma<T>;
   using Elt = typename M::Elt;
   using Frag = typename M::Frag;
   using L = Lds<DP, T, BN>;
   constexpr int KF = M::KF, EPL = M::EPL, NF = DP / KF, CB = DP / 32, NFA = 32 / KF, NT = 64 * NW, BM = 32 * RT * NW;
-  constexpr int HC = Shape<DP, T>::HC;   // operand fragments read ahead at a time
+  constexpr int HC = (Shape<DP, T>::BF && NF % 4 == 0) ? 4 : 2;   // operand fragments read ahead at a time
   static_assert(NF % HC == 0, "whole groups of fragments");
   constexpr int PR = L::PR, PT = L::PT;
-  static_assert(L::bytes(2, 1, 0) >= (size_t)DP * (M::PLANES * DP + M::PAD) * sizeof(Elt) + DP * sizeof(float), "a state fits the stage buffers");
+  static_assert(L::bytes(2, 1, 0) >= (size_t)DP * (DP + M::PAD) * sizeof(Elt) + DP * sizeof(float), "a state fits the stage buffers");
   extern __shared__ __attribute__((aligned(16))) unsigned char dense_smem[];
   Elt* Kl = reinterpret_cast<Elt*>(dense_smem);   // [2][BN][PR]
   Elt* Vl = Kl + 2 * L::RM;                       // [2][BN][PR]
@@ -929,15 +806,15 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
     // select uses under that condition, where it gets a wait of its own -- for every load issued before it)
     const float dnv = denh[(int64_t)ps * den.stride], lm = live ? 1.0f : 0.f;
     const float rden = lm / dnv;
-    if (p2) load_own_frags<DP, T, M>(Qh, pos, npos, d, hh, kq * 2.0f * a2, qf[rt]);
+    if (p2) load_own_frags<DP, T>(Qh, pos, npos, d, hh, kq * 2.0f * a2, qf[rt]);
     if (cw) {   // (block-uniform)
       // c_i = grad_out_i . out_i / den_i is formed here from rows the block reads anyway (plus those of out) and left
       // in cvec for the dk / dv kernel: no separate pass over grad_out and out
-      cown[rt] = load_g_frags_and_c<DP, T, M>(Gh, OUTF.head(head), pos, npos, d, hh, rden, gf[rt]);
+      cown[rt] = load_g_frags_and_c<DP, T>(Gh, OUTF.head(head), pos, npos, d, hh, rden, gf[rt]);
       if (live && hh == 0) cw[(int64_t)pos * cprep.stride] = cown[rt];
     } else {
       cown[rt] = lm * ch[(int64_t)ps * cvec.stride];
-      load_own_frags<DP, T, M>(Gh, pos, npos, d, hh, rden, gf[rt]);
+      load_own_frags<DP, T>(Gh, pos, npos, d, hh, rden, gf[rt]);
     }
   }
 
@@ -945,7 +822,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
   const int nst = (kend + BN - 1) / BN;
   const int lc = (lstate && masked) ? tok0 / lchunk : 0;   // (linear mode, as in the forward kernel)
   const int st0 = lstate ? (masked ? lc * (lchunk / BN) : nst) : 0;
-  TileRegs<DP, T, BN, NT, M> kt, vt;
+  TileRegs<DP, T, BN, NT> kt, vt;
   auto stage_load = [&](int st) {
     kt.load(Kh, st * BN, nk, d, tid);
     vt.load(Vh, st * BN, nk, d, tid);
@@ -966,7 +843,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
   if (st0 < nst) stage_load(st0);   // (requested before the state is: one memory latency, not two)
   if (lstate && (!masked || lc > 0)) {
     // sum_j a1 (g . v_j - c) k_j over the keys in the state = a1 (g . S1^T - c sum k)
-    constexpr int PS = M::PLANES * DP + M::PAD;
+    constexpr int PS = DP + M::PAD;
     Elt* Sn = reinterpret_cast<Elt*>(dense_smem);             // a1 S1 as [key channel][value channel]
     float* sk = reinterpret_cast<float*>(Sn + DP * PS);       // sum k
     const float* sp = lstate + ((int64_t)hkv * lslots + lc) * LinState<DP>::floats(1);   // (one block: natural)
@@ -1010,8 +887,8 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
       Frag va[HC], ka[HC];
 #pragma unroll
       for (int m = 0; m < HC; ++m) {
-        va[m] = M::load(vl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh, DP);
-        if (p2) ka[m] = M::load(kl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh, DP);
+        va[m] = lds_frag<T>(vl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh);
+        if (p2) ka[m] = lds_frag<T>(kl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh);
       }
 #pragma unroll
       for (int m = 0; m < HC; ++m)
@@ -1038,7 +915,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_DQ)) void dense_dq_kern
       constexpr int F = decltype(ftag)::value;
       Frag kb_[CB], wa[RT];
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) kb_[cb] = M::load(ktl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh, BN);
+      for (int cb = 0; cb < CB; ++cb) kb_[cb] = lds_frag<T>(ktl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) wa[rt] = M::template from_acc<F>(pt[rt]);
 #pragma unroll
@@ -1122,15 +999,15 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
     const float* __restrict__ qscale, const float* __restrict__ kscale, Rows<T> DK, Rows<T> DV,
     float* __restrict__ rpart, int npos, int nk, int d, int masked, float a0, float a1, float a2, int ratio,
     const float* __restrict__ lstate, int lchunk, int lslots) {
-  using M = Policy<DP, T>;
+  using M = Mma<T>;
   using Elt = typename M::Elt;
   using Frag = typename M::Frag;
   using L = Lds<DP, T, BN>;
   constexpr int KF = M::KF, EPL = M::EPL, NF = DP / KF, CB = DP / 32, NFA = 32 / KF, NT = 64 * NW, BM = 32 * RT * NW;
-  constexpr int HC = Shape<DP, T>::HC;   // operand fragments read ahead at a time
+  constexpr int HC = (Shape<DP, T>::BF && NF % 4 == 0) ? 4 : 2;   // operand fragments read ahead at a time
   static_assert(NF % HC == 0, "whole groups of fragments");
   constexpr int PR = L::PR, PT = L::PT;
-  static_assert(L::bytes(2, 2, 0) >= (size_t)2 * DP * (M::PLANES * DP + M::PAD) * sizeof(Elt) + 2 * DP * sizeof(float), "a state fits the stage buffers");
+  static_assert(L::bytes(2, 2, 0) >= (size_t)2 * DP * (DP + M::PAD) * sizeof(Elt) + 2 * DP * sizeof(float), "a state fits the stage buffers");
   extern __shared__ __attribute__((aligned(16))) unsigned char dense_smem[];
   Elt* Ql = reinterpret_cast<Elt*>(dense_smem);   // [2][BN][PR]
   Elt* Gl = Ql + 2 * L::RM;                       // [2][BN][PR]
@@ -1138,12 +1015,8 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
   Elt* Gt = Qt + 2 * L::TR;                       // [2][DP][PT]
   float* Cl = reinterpret_cast<float*>(Gt + 2 * L::TR);   // [2][BN]: -qs c of the streamed queries
   float* red = Cl + 2 * BN;                       // [NW]
-  fm_u4* kl2 = reinterpret_cast<fm_u4*>(red + (NW + 3) / 4 * 4);   // (KLO) [NW][NF][64]: the last parts of the key fragments
-  constexpr bool KLO = Shape<DP, T>::KLO;
-  static_assert(!KLO || RT == 1, "one own tile per wave");
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, hh = l >> 5;
-  kl2 += w * NF * 64 + l;
   const int nb = gridDim.y, bx = blockIdx.y;   // (key/value heads, key blocks)
   const int hkv = blockIdx.x;
   const int tok0 = bx * BM;   // (under the mask the first key blocks see the most queries: already first)
@@ -1154,18 +1027,9 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int pos = tok0 + (w * RT + rt) * 32 + i;
-    load_own_frags<DP, T, M>(Kh, pos, nk, d, hh, ks, kf[rt]);
-    load_own_frags<DP, T, M>(Vh, pos, nk, d, hh, 1.0f, vf[rt]);
+    load_own_frags<DP, T>(Kh, pos, nk, d, hh, ks, kf[rt]);
+    load_own_frags<DP, T>(Vh, pos, nk, d, hh, 1.0f, vf[rt]);
   }
-  if constexpr (KLO) {   // (read back by the lane that wrote them: no barrier)
-#pragma unroll
-    for (int m = 0; m < NF; ++m) kl2[m * 64] = kf[0][m].p[2];
-  }
-  auto key_frag = [&](int rt, int m) __attribute__((always_inline)) {
-    Frag f = kf[rt][m];
-    if constexpr (KLO) f.p[2] = kl2[m * 64];
-    return f;
-  };
   f16v dk[RT][CB], dv[RT][CB];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
@@ -1177,7 +1041,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
   float dvc[CB], dkc[CB];   // (linear mode) what every own row's dv / dk gets on top, per channel cb * 32 + i
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) dvc[cb] = dkc[cb] = 0.f;
-  TileRegs<DP, T, BN, NT, M> qt, gt;
+  TileRegs<DP, T, BN, NT> qt, gt;
   float creg = 0.f, cmask = 0.f;
   for (int hq = 0; hq < ratio; ++hq) {
     const int head = hkv * ratio + hq;
@@ -1214,7 +1078,7 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
     if (lstate && (!masked || lc + 1 < lslots)) {
       // dv += a0 sum g + a1 qs kh . R1,  dk += a1 qs (v . R1^T - sum c q)   (R1 = sum q (x) g of the queries in the state);
       // the two sums, the same for every own row, wait in dvc / dkc for the epilogue
-      constexpr int PS = M::PLANES * DP + M::PAD;
+      constexpr int PS = DP + M::PAD;
       Elt* Rn = reinterpret_cast<Elt*>(dense_smem);             // a1 qs R1 as [query channel][value channel]
       Elt* Rt = Rn + DP * PS;                                   // and as [value channel][query channel]
       float* rq = reinterpret_cast<float*>(Rt + DP * PS);       // sum c q
@@ -1227,27 +1091,14 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
       __syncthreads();
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) {
-        if constexpr (Shape<DP, T>::SPLIT) {   // (straight into the accumulators: four registers fewer across the walk)
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              dv[rt][cb][r] += a0 * rg[cb * 32 + i];
-              dk[rt][cb][r] -= aq * rq[cb * 32 + i];
-            }
-        } else {
-          dvc[cb] += a0 * rg[cb * 32 + i];
-          dkc[cb] -= aq * rq[cb * 32 + i];
-        }
+        dvc[cb] += a0 * rg[cb * 32 + i];
+        dkc[cb] -= aq * rq[cb * 32 + i];
       }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
-          Frag kx[NF];
-#pragma unroll
-          for (int m = 0; m < NF; ++m) kx[m] = key_frag(rt, m);
-          dv[rt][cb] = lin_own_times<DP, T>(kx, Rt + (cb * 32 + i) * PS + EPL * hh, dv[rt][cb]);
+          dv[rt][cb] = lin_own_times<DP, T>(kf[rt], Rt + (cb * 32 + i) * PS + EPL * hh, dv[rt][cb]);
           dk[rt][cb] = lin_own_times<DP, T>(vf[rt], Rn + (cb * 32 + i) * PS + EPL * hh, dk[rt][cb]);
         }
       __syncthreads();
@@ -1275,17 +1126,16 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
         Frag qa[HC], ga[HC];
 #pragma unroll
         for (int m = 0; m < HC; ++m) {
-          qa[m] = M::load(ql + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh, DP);
-          ga[m] = M::load(gl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh, DP);
+          qa[m] = lds_frag<T>(ql + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh);
+          ga[m] = lds_frag<T>(gl + (t32 * 32 + i) * PR + KF * (m0 + m) + EPL * hh);
         }
 #pragma unroll
         for (int m = 0; m < HC; ++m)
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt) {
-            sc[rt] = M::mma(qa[m], key_frag(rt, m0 + m), m0 + m == 0 ? kZero16 : sc[rt]);
+            sc[rt] = M::mma(qa[m], kf[rt][m0 + m], m0 + m == 0 ? kZero16 : sc[rt]);
             pt[rt] = M::mma(ga[m], vf[rt][m0 + m], pt[rt]);
           }
-        if (Shape<DP, T>::SPLIT && DP == 64) __builtin_amdgcn_sched_barrier(0);   // (register pressure)
       }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
@@ -1306,27 +1156,11 @@ __global__ __launch_bounds__(64 * NW, (Shape<DP, T>::OCC_KV)) void dense_dkdv_ke
       // own keys x channels: dv += f^T (keys x queries) . g,   dk += W^T . q
       static_for<NFA>([&](auto ftag) {
         constexpr int F = decltype(ftag)::value;
-        if constexpr (Shape<DP, T>::SPLIT) {   // (one operand at a time: a split fragment takes twelve registers)
-#pragma unroll
-          for (int rt = 0; rt < RT; ++rt) {
-            const Frag fa = M::template from_acc<F>(sc[rt]);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-              dv[rt][cb] = M::mma(fa, M::load(gtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh, BN), dv[rt][cb]);
-            if (DP == 64) __builtin_amdgcn_sched_barrier(0);
-            const Frag wa = M::template from_acc<F>(pt[rt]);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-              dk[rt][cb] = M::mma(wa, M::load(qtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh, BN), dk[rt][cb]);
-            if (DP == 64) __builtin_amdgcn_sched_barrier(0);
-          }
-          return;
-        }
         Frag bg[CB], bq[CB], fa[RT], wa[RT];
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
-          bg[cb] = M::load(gtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh, BN);
-          bq[cb] = M::load(qtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh, BN);
+          bg[cb] = lds_frag<T>(gtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh);
+          bq[cb] = lds_frag<T>(qtl + (cb * 32 + i) * PT + t32 * 32 + KF * F + EPL * hh);
         }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {

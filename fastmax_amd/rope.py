@@ -116,7 +116,7 @@ class _QKVAttention(torch.autograd.Function):
             q5, k4 = rot[:, :, :, :q_per_kv].permute(0, 2, 3, 1, 4), rot[:, :, :, q_per_kv].permute(0, 2, 1, 3)
         cfg = (bool(mask), bool(normalize), float(temperature), float(a0), float(a1), float(a2), float(lim), int(p))
         save = qkv.requires_grad and _states_fit_bytes(ext, q5, k4, cfg[0], cfg[7])
-        o5, den, scale, arg, saved = ext.forward_strided(q5, k4, v4, *cfg, save)
+        o5, den, scale, arg, saved = ext.forward_strided(q5, k4, v4, *cfg, save, qkv.requires_grad)
         ctx.save_for_backward(q5, k4, v4, o5, den, scale, arg, saved, cos if rope_n else qkv.new_empty(0),
                               sin if rope_n else qkv.new_empty(0))
         ctx.cfg, ctx.geo, ctx.shape = cfg, (groups, q_per_kv, hs, rope_n), qkv.shape

@@ -190,6 +190,10 @@ int fastmax_backward_strided(const fastmax_desc* desc, const fastmax_layout* lay
  * p = 1 past 1024 causal / 512 unmasked positions the chunk states of their linear mode, which both
  * passes rebuild). */
 size_t fastmax_saved_state_bytes(const fastmax_desc* desc);
+/* In the place of saved_bytes, with saved_states == NULL: nothing this forward pass computes will be
+ * handed to a backward pass.  fp32 outputs of up to 64 channels may then come from kernels that round
+ * differently (as close to the exact result; o differs from fastmax_forward's by about 1e-6 of it). */
+#define FASTMAX_NO_BACKWARD ((size_t)-1)
 int fastmax_forward_saving(const fastmax_desc* desc, const void* q, const void* k, const void* v,
                            void* o, int64_t ldo, float* den, int64_t den_stride,
                            float* qk_scale, int32_t* qk_argmax,

@@ -430,9 +430,8 @@ def test_strided_views_with_many_heads_take_the_linear_mode(built, monkeypatch):
 @pytest.mark.parametrize("n", [31, 256, 289])
 @pytest.mark.parametrize("mask", [False, True])
 def test_fp32_contractions_keep_24_bits(ops, d, n, mask):
-    """fp32 contractions run on parts of 3 x 8 bits.  With positive values and weights nothing cancels, so the
-    outputs are as good as their roundings: about sqrt(6 n / 16) of 2^-24 each in the sums (11 at n = 289) on top
-    of a few in the weights.  A product of parts left out would show as 2^-18 or more (64 of these units)."""
+    """With positive values and weights nothing cancels, so the outputs are as good as their roundings: about
+    sqrt(n / 2) of 2^-24 each in the sums (12 at n = 289) on top of a few in the weights."""
     q, k, v, go = (t.abs() for t in O.seeded_inputs((2, n, d), seed=n + d))
     v, go = v + 0.1, go + 0.1
     kw = dict(mask=mask, normalize=True, p=2)
@@ -449,5 +448,5 @@ def test_fp32_contractions_keep_24_bits(ops, d, n, mask):
 @pytest.mark.parametrize("d", [32, 48, 64])
 @pytest.mark.parametrize("mask", [False, True])
 def test_many_heads_fp32(ops, d, mask):
-    # (enough 256-row blocks to fill the chip: the eight-wave form of the kernels; the tests above run the four-wave one)
+    # (enough 256-row blocks to fill the chip)
     run_case(ops, (130, 289, d), seed=d, mask=mask, normalize=True, p=2)

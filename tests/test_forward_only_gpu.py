@@ -1,0 +1,98 @@
+"""fp32 forward passes that nobody differentiates, up to 64 channels on the dense kernels: their contractions run on parts of
+3 x 8 bits (fastmax_amd/csrc/fm_cut.h).  Against the fp64 closed form, and against the training forward pass, which stays on
+the fp32 instruction."""
+import pytest
+import torch
+
+from oracle import fastmax_oracle as O
+
+from helpers import assert_close
+
+KERNEL_PATH = "dense"
+gpu = pytest.mark.gpu
+UNIT = 2.0 ** -24
+
+
+def forwards(q, k, v, mask, normalize=True, a0=1.0, a1=1.0, a2=0.5, p=2):
+    """(o, den) of a pass that no backward pass follows, and of one that may be differentiated"""
+    from fastmax_amd import _ext
+
+    ext = _ext.load()
+    args = [t.cuda() for t in (q, k, v)] + [bool(mask), normalize, 1.0, a0, a1, a2, 1.0, p, False]
+    return ext.forward_ex(*args, False)[:2], ext.forward_ex(*args)[:2]
+
+
+@gpu
+@pytest.mark.parametrize("d", [8, 24, 32, 40, 64])
+@pytest.mark.parametrize("bh,bhkv,nq,nk", [(3, 3, 1, 1), (4, 2, 31, 31), (2, 2, 33, 160), (2, 1, 256, 256), (2, 2, 257, 257), (3, 3, 300, 1000),
+                                           (132, 66, 289, 289), (260, 260, 70, 70)])   # (the last two: blocks of eight waves)
+@pytest.mark.parametrize("mask", [True, False])
+def test_against_the_closed_form(built, d, bh, bhkv, nq, nk, mask):
+    q, _, _, go = O.seeded_inputs((bh, nq, d), seed=nq + d)
+    _, k, v, _ = O.seeded_inputs((bhkv, nk, d), seed=nk + d + 1)
+    print("forward only", d, bh, bhkv, nq, nk, mask, flush=True)
+    (o, den), (ot, dent) = forwards(q, k, v, mask)
+    rep = [t.double().repeat_interleave(bh // bhkv, 0) for t in (k, v)]
+    want = O.dense_truth(q.double(), rep[0], rep[1], go.double(), mask=mask, normalize=True, p=2)[0]
+    # (sums of up to 1000 terms of about equal size: sqrt(1000) roundings of 2^-24 each, and a few in the weights)
+    assert_close("o", o, want, 40 * UNIT)
+    assert_close("den", den, dent, 40 * UNIT)
+    if mask and nq == nk:   # a query with few keys in sight: the bits of the training pass
+        assert torch.equal(o[:, :32], ot[:, :32]) and torch.equal(den[:, :32], dent[:, :32])
+
+
+@gpu
+@pytest.mark.parametrize("mask", [True, False])
+def test_the_module_keeps_the_two_apart(built, mask):
+    """With gradients the module's output has the training pass's bits; without, it comes from the other kernel."""
+    from fastmax_amd import FASTMultiHeadAttention
+
+    q, k, v, _ = (t.cuda() for t in O.seeded_inputs((1, 8, 300, 64), seed=5))
+    att = FASTMultiHeadAttention()
+    args = (None, mask, 0.0, True, 1.0, 1.0, 1.0, 0.5, 1.0, 2)
+    (o, _), (ot, _) = forwards(q[0].cpu(), k[0].cpu(), v[0].cpu(), mask)
+    assert torch.equal(att(q.requires_grad_(True), k, v, *args)[0].detach(), ot)
+    assert torch.equal(att(q.detach(), k, v, *args)[0], o) and not torch.equal(o, ot)
+
+
+# 1 + 2^-8 - 2^-17 and the like: the second and the third part of each are near their largest and of one sign, so that a
+# product of parts left out adds up instead of averaging out
+X, Y = 1.003883361816406, 1.003883242607117
+
+
+def cut_parts(x):
+    out = []
+    x = torch.tensor(x, dtype=torch.float32)
+    for _ in range(3):
+        out.append(x.bfloat16().double())
+        x = (x.double() - out[-1]).float()
+    return out
+
+
+def test_any_lost_product_of_parts_would_show():
+    """Six products of parts give X Y to 2 units of 2^-24; without any one of them it is off by more than 100."""
+    a, b = cut_parts(X), cut_parts(Y)
+    exact = float(torch.tensor(X, dtype=torch.float32).double() * torch.tensor(Y, dtype=torch.float32).double())
+    six = [(0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)]
+    off = lambda pairs: abs(float(sum(a[i] * b[j] for i, j in pairs)) / exact - 1) / UNIT
+    assert off(six) < 2.0
+    for lost in six:
+        assert off([p for p in six if p != lost]) > 100, lost
+
+
+@gpu
+@pytest.mark.parametrize("d", [32, 64])
+@pytest.mark.parametrize("bh", [3, 300])   # (blocks of four and of eight waves)
+def test_fp32_contractions_keep_24_bits(built, d, bh):
+    """The scores show in the denominators (f = s), the weighted sum in the output (f = a constant).  64 keys: 4 steps of 6
+    roundings of at most half a unit each, 2 units left out, a few roundings at the end: 16 units in all."""
+    n = 64
+    q, k = torch.full((bh, n, d), X), torch.full((bh, n, d), Y)
+    v = Y * (2.0 ** (torch.arange(d) % 5 - 2.0)).expand(bh, n, d).contiguous()
+    x, y = torch.tensor(X).double(), torch.tensor(Y).double()
+    (_, den), _ = forwards(q, k, v, False, normalize=False, a0=0.0, a1=1.0, a2=0.0)
+    err = ((den.double().cpu() / (n * d * x * y) - 1).abs().max() / UNIT).item()
+    assert err < 16, f"denominators off by {err:.1f} units"
+    (o, _), _ = forwards(q, k, v, False, normalize=False, a0=X, a1=0.0, a2=0.0)
+    err = ((o.double().cpu() / v.double() - 1).abs().max() / UNIT).item()
+    assert err < 16, f"outputs off by {err:.1f} units"

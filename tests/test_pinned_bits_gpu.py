@@ -40,6 +40,15 @@ DENSE = [
     ("dense", "f32", 8, 8, 300, 300, 128, 1, 2, 4091383673, 2457249628, 1079922644, 362090554),
     ("dense", "f32", 8, 2, 300, 300, 96, 0, 2, 1021814443, 3537306125, 680700910, 1153882343),
     ("dense", "f32", 4, 4, 1300, 1300, 96, 1, 1, 1231972123, 537493458, 1011557046, 1921822793),
+    ("dense", "f32", 64, 64, 333, 333, 32, 1, 2, 175136426, 2041681451, 3894617981, 614471740),
+    ("dense", "f32", 8, 8, 333, 333, 32, 0, 2, 304949949, 1917231796, 1656956889, 4161112970),
+    ("dense", "f32", 130, 130, 289, 289, 64, 1, 2, 897942153, 245571809, 135212676, 4157327010),
+    ("dense", "f32", 16, 4, 300, 700, 64, 1, 2, 3447775792, 1261274757, 412639675, 2531279138),
+    ("dense", "f32", 8, 8, 289, 289, 64, 0, 2, 945933898, 2499552016, 4206485397, 1029954956),
+    ("dense", "f32", 16, 16, 257, 257, 48, 1, 2, 2349627808, 285174191, 2722873527, 2985272880),
+    ("dense", "f32", 8, 8, 61, 61, 24, 1, 2, 2319987192, 2501598304, 4289548840, 4102585435),
+    ("dense", "f32", 8, 8, 1300, 1300, 40, 1, 1, 3340789179, 1775938835, 1233859911, 2943671026),
+    ("dense", "f32", 8, 8, 700, 700, 24, 0, 1, 2212542706, 1038529220, 2833446290, 3868902450),
 ]
 
 
