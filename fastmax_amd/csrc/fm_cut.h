@@ -11,7 +11,8 @@
 // What bounds it: six v_mfma_f32_32x32x16_bf16 take ~200 cycles where eight v_mfma_f32_32x32x2f32 take 512; around them
 // the cutting of the weights (~5.5 VALU instructions a value) and the operand reads, three planes each.  The parts of
 // streamed rows are formed once per block on their way into LDS, those of own rows once per wave, only those of the
-// weights per tile.  Unmasked, 512 heads x 1000 x 64: 1164 us a pass on the fp32 instruction, 798 here.
+// weights per tile.  Unmasked, 512 heads x 1000 x 64: 1164 us a pass on the fp32 instruction, 814 here (798 without
+// the look at the results for values that the parts do not hold).
 //
 // Not for passes that are differentiated.  The gradients of the first rows are differences of nearly equal numbers,
 // g . v - c with c formed from this output, and the row that carries the row-norm maximum takes the rounding of a whole
@@ -95,7 +96,7 @@ template <int DP>
 struct Lds {
   static constexpr int PR = 3 * DP + 8, PT = 3 * BN + 8;   // pitches: odd numbers of 16-byte words
   static constexpr int RM = BN * PR, TR = DP * PT;
-  static constexpr size_t bytes(int own_rows) { return (size_t)2 * (RM + TR) * sizeof(uint16_t) + own_rows * sizeof(float); }
+  static constexpr size_t bytes(int own_rows) { return (size_t)2 * (RM + TR) * sizeof(uint16_t) + (own_rows + 4) * sizeof(float); }
 };
 
 // BN rows x DP channels on their way global -> registers -> LDS by NT threads, as dense::TileRegs
@@ -155,7 +156,7 @@ struct Stage {
 // (which explains the mask): each wave has 32 own rows, the keys are streamed in stages that the waves share.
 // ---------------------------------------------------------------------------------------
 template <int DP, int NW>
-__global__ __launch_bounds__(64 * NW, DP == 32 ? 2 : 1) void cut_fwd_kernel(
+__global__ __launch_bounds__(64 * NW, DP == 32 ? 4 : 2) void cut_fwd_kernel(
     Rows<const float> Q, Rows<const float> K, Rows<const float> V, const float* __restrict__ qscale,
     const float* __restrict__ kscale, Rows<float> O, RowScalarsOut den, int npos, int nk, int d, int masked, float a0,
     float a1, float a2, int ratio) {
@@ -165,6 +166,7 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 2 : 1) void cut_fwd_kernel(
   uint16_t* Kl = reinterpret_cast<uint16_t*>(cut_smem);   // [2][BN][PR]
   uint16_t* Vt = Kl + 2 * L::RM;                          // [2][DP][PT]
   float* denl = reinterpret_cast<float*>(Vt + 2 * L::TR);   // [BM]
+  int* seen = reinterpret_cast<int*>(denl + BM);            // 1: one of the block's sums is zero, 2: one of its values is subnormal
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, hh = l >> 5;
   const int nb = gridDim.y, bx = blockIdx.y;
@@ -176,6 +178,8 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 2 : 1) void cut_fwd_kernel(
   const bool own_live = own >= Qh.lo && own < npos;
   const float* qrow = Qh.base + (unsigned)max(own < npos ? own : npos - 1, Qh.lo) * Qh.pitch;
 
+  bool qodd = false;
+  if (tid == 0) *seen = 0;
   Frag qf[NF];
 #pragma unroll
   for (int m = 0; m < NF; ++m) {
@@ -190,8 +194,12 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 2 : 1) void cut_fwd_kernel(
       x[u + 2] = ok ? t.z * kq : 0.f;
       x[u + 3] = ok ? t.w * kq : 0.f;
     }
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) qodd |= fabsf(x[e]) > 0x1p60f || (fabsf(x[e]) < 0x1p-100f && x[e] != 0.f);
     qf[m] = make(x);
   }
+
+  qodd = __any(qodd);
 
   const int kend = masked ? (tok0 + BM < nk ? tok0 + BM : nk) : nk;
   const int nst = (kend + BN - 1) / BN;
@@ -221,15 +229,19 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 2 : 1) void cut_fwd_kernel(
     }
     if (masked && kb == q00) {   // (wave-uniform) a key may not lie after the query
       FM_KEEP_BRANCH();
+      int lim = i - 4 * hh;
+      asm volatile("" : "+v"(lim));   // (compared here: sixteen comparisons kept across the walk are 32 registers)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        if (trow(r, hh) > i) sc[r] = 0.f;
+        if (trow(r, 0) > lim) sc[r] = 0.f;
     }
     if (!masked && kb + 32 > nk) {   // (wave-uniform) keys past the end
       FM_KEEP_BRANCH();
+      int lim = nk - kb - 4 * hh;
+      asm volatile("" : "+v"(lim));
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        if (kb + trow(r, hh) >= nk) sc[r] = 0.f;
+        if (trow(r, 0) >= lim) sc[r] = 0.f;
     }
   };
   auto tile = [&](int kb, const uint16_t* kl, const uint16_t* vl) __attribute__((always_inline)) {
@@ -271,23 +283,81 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 2 : 1) void cut_fwd_kernel(
     __syncthreads();
   }
 
-  if (first) {
+  // Whether the parts held what the wave's rows are made of.  An infinite first part (of an infinity, or of a finite value
+  // above bf16's largest) makes a result that is not finite.  Values below 2^-102 lose what lies below 2^-133: of the
+  // values that shows in a weighted sum below 2^-100 of the sum of weights (or below 2^-80, where products of parts
+  // begin to underflow; a sum of zero is what it should be unless a value was subnormal), of the weights where their sum is
+  // below 2^-80, of the scores where a query is as small or beyond 2^60.
+  const float sum = dn + __shfl_xor(dn, 32, 64);
+  if (hh == 0) denl[w * 32 + i] = sum;   // (read back by the wave itself)
+  bool odd = own_live && !(fabsf(sum) >= 0x1p-80f && fabsf(sum) < __builtin_inff()), none = false;
+  float top = fabsf(sum);
+#pragma unroll
+  for (int off = 16; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
+  const float least = fmaxf(0x1p-80f, 0x1p-100f * top);
+  // (bits without the sign, doubled: in one comparison of unsigned numbers everything that is not in [least, inf))
+  const uint32_t floor2 = __float_as_uint(least) << 1;
+  uint32_t far = 0;
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) far = max(far, (__float_as_uint(acc[cb][r]) << 1) - floor2);
+  if (!first && __any(far >= 0xff000000u - floor2)) {   // (or a zero, an absent row or column: looked at one by one)
+    FM_KEEP_BRANCH();
+    int li = i, lh = hh;
+    asm volatile("" : "+v"(li), "+v"(lh));
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int pos = q00 + trow(r, lh);
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) {
+        const float mag = fabsf(acc[cb][r]);
+        const bool out = pos >= Qh.lo && pos < npos && cb * 32 + li < d;
+        odd |= out && !(mag < __builtin_inff() && (mag >= least || mag == 0.f));
+        none |= out && mag == 0.f;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (none) atomicOr(seen, 1);
+  __syncthreads();
+  if (*seen) {   // (block-uniform: nothing below writes bit 0)
+    FM_KEEP_BRANCH();
+    bool subnormal = false;
+    for (int idx = tid; idx < kend * (DP / 4); idx += NT) {
+      const int ch = idx % (DP / 4) * 4;
+      const float4 t = *reinterpret_cast<const float4*>(Vh.base + ((unsigned)(idx / (DP / 4)) * Vh.pitch + (unsigned)(ch < d ? ch : 0)));
+      constexpr int CLASS = 0x90;   // negative or positive subnormal
+      subnormal |= __builtin_amdgcn_classf(t.x, CLASS) || __builtin_amdgcn_classf(t.y, CLASS) || __builtin_amdgcn_classf(t.z, CLASS) ||
+                   __builtin_amdgcn_classf(t.w, CLASS);
+    }
+    if (subnormal) atomicOr(seen, 2);
+    __syncthreads();
+    odd |= none && (*seen & 2);
+  }
+  const bool again = first || qodd || __any(odd);
+  if (again) {   // (wave-uniform)
     // The wave's rows on the fp32 instruction, operands straight from memory and in the order of dense_fwd_kernel (the same
     // bits).  No barrier in here: the other waves do not come along.
     FM_KEEP_BRANCH();
+    int li = i, lh = hh;
+    asm volatile("" : "+v"(li), "+v"(lh));   // (addresses are formed here, not kept across the walk)
+    const int lown = q00 + li;
+    const bool llive = lown >= Qh.lo && lown < npos;
+    const float* lq = Qh.base + (unsigned)max(lown < npos ? lown : npos - 1, Qh.lo) * Qh.pitch;
     const int last = masked ? (q00 + 32 < nk ? q00 + 32 : nk) : nk;
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) acc[cb] = dense::kZero16;
     dn = 0.f;
 #pragma unroll 1
     for (int kb = 0; kb < last; kb += 32) {
-      const float* krow = Kh.base + (unsigned)(kb + i < nk ? kb + i : nk - 1) * Kh.pitch;
+      const float* krow = Kh.base + (unsigned)(kb + li < nk ? kb + li : nk - 1) * Kh.pitch;
       f16v sc = dense::kZero16;
 #pragma unroll 1
       for (int g = 0; g < DP / 8; ++g) {
-        const int ch = 8 * g + 4 * hh;
-        const bool on = ch < d, qon = on && own_live, kon = on && kb + i < nk;
-        const float4 k4 = *reinterpret_cast<const float4*>(krow + (on ? ch : 0)), q4 = *reinterpret_cast<const float4*>(qrow + (on ? ch : 0));
+        const int ch = 8 * g + 4 * lh;
+        const bool on = ch < d, qon = on && llive, kon = on && kb + li < nk;
+        const float4 k4 = *reinterpret_cast<const float4*>(krow + (on ? ch : 0)), q4 = *reinterpret_cast<const float4*>(lq + (on ? ch : 0));
         sc = FM_MFMA(kon ? k4.x : 0.f, qon ? q4.x * kq : 0.f, sc);
         sc = FM_MFMA(kon ? k4.y : 0.f, qon ? q4.y * kq : 0.f, sc);
         sc = FM_MFMA(kon ? k4.z : 0.f, qon ? q4.z * kq : 0.f, sc);
@@ -299,22 +369,22 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 2 : 1) void cut_fwd_kernel(
         dn += (sc[F] + sc[F + 1]) + (sc[F + 2] + sc[F + 3]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int key = kb + trow(F + e, hh);
+          const int key = kb + trow(F + e, lh);
           const float* vrow = Vh.base + (unsigned)(key < nk ? key : nk - 1) * Vh.pitch;
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb) {
-            const int c = cb * 32 + i;
+            const int c = cb * 32 + li;
             const float v = vrow[c < d ? c : 0];
             acc[cb] = FM_MFMA(sc[F + e], key < nk && c < d ? v : 0.f, acc[cb]);
           }
+          __builtin_amdgcn_sched_barrier(0);   // (register pressure)
         }
       });
     }
+    const float sum32 = dn + __shfl_xor(dn, 32, 64);
+    if (hh == 0) denl[w * 32 + i] = sum32;   // (read back by the wave itself)
   }
 
-  const float tot = dn + __shfl_xor(dn, 32, 64);
-  if (hh == 0) denl[w * 32 + i] = tot;
-  __syncthreads();
   const HeadRows<float> Oh = O.head(head);
   float* denh = den.head(head);
 #pragma unroll

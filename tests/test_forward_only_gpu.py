@@ -96,3 +96,72 @@ def test_fp32_contractions_keep_24_bits(built, d, bh):
     (o, _), _ = forwards(q, k, v, False, normalize=False, a0=X, a1=0.0, a2=0.0)
     err = ((o.double().cpu() / v.double() - 1).abs().max() / UNIT).item()
     assert err < 16, f"outputs off by {err:.1f} units"
+
+
+def ranged(kind, d, n):
+    """q, k, v with values that three bf16 parts do not hold, and the coefficients"""
+    q, k, v, _ = O.seeded_inputs((2, n, d), seed=n + d)
+    kw = dict(normalize=True, a0=0.5, a1=0.1, a2=0.1)
+    j, c = n // 2, d - 3
+    if kind == "infinite value":
+        v[0, j, c] = float("inf")
+    elif kind == "minus infinity in two rows":
+        v[0, j, c] = v[1, n - 1, 0] = -float("inf")
+    elif kind == "not a number":
+        v[0, j, c] = k[1, j, 1] = float("nan")
+    elif kind == "infinite key":
+        k[0, j, c] = float("inf")
+        kw.update(normalize=False)
+    elif kind == "largest value":   # (rounds to infinity in bf16)
+        v[0, j, c] = torch.finfo(torch.float32).max
+        v[1, 0, 1] = torch.finfo(torch.float32).min
+    elif kind == "tiny values":
+        v *= 2.0 ** -115
+    elif kind == "one tiny channel":
+        v[..., c] *= 2.0 ** -112
+    elif kind == "tiny and zero channels":
+        v[..., c] = 0.0
+        v[..., 1] *= 2.0 ** -112
+    elif kind == "tiny keys and large queries":
+        q, k = q * 2.0 ** 113, k * 2.0 ** -117
+        kw.update(normalize=False)
+    elif kind == "tiny scores":
+        q, k = q.abs() * 2.0 ** -60, k.abs() * 2.0 ** -57
+        kw.update(normalize=False, a0=0.0, a1=1.0, a2=0.0)
+    elif kind == "tiny weights":
+        kw.update(a0=2.0 ** -116, a1=2.0 ** -118, a2=0.0)
+    elif kind == "tiny values under large weights":
+        v *= 2.0 ** -118
+        kw.update(a0=2.0 ** 100, a1=2.0 ** 97, a2=0.0)
+    elif kind == "subnormal values":
+        v *= 2.0 ** -137
+        kw.update(a0=2.0 ** 100, a1=2.0 ** 97, a2=0.0)
+    return q, k, v, kw
+
+
+KINDS = ["infinite value", "minus infinity in two rows", "not a number", "infinite key", "largest value", "tiny values", "one tiny channel",
+         "tiny and zero channels", "tiny keys and large queries", "tiny scores", "tiny weights", "tiny values under large weights",
+         "subnormal values"]
+
+
+@gpu
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("d,n", [(24, 70), (64, 300)])
+@pytest.mark.parametrize("mask", [True, False])
+def test_values_that_the_parts_do_not_hold(built, kind, d, n, mask):
+    """What the training pass's kernel gives for them: not-a-number and infinities in the same places, and each channel as
+    close as elsewhere.  Both are sums of n terms w v over the sum of w, so their rounding goes with the mean of the finite
+    |v| of a channel (not with the result, which may come out near zero): sqrt(300) roundings each, 40 units in all."""
+    q, k, v, kw = ranged(kind, d, n)
+    print("range", kind, d, n, mask, flush=True)
+    (o, den), (ot, dent) = forwards(q, k, v, mask, **kw)
+    o, den, ot, dent = (t.double().cpu() for t in (o, den, ot, dent))
+    size = torch.where(v.isfinite(), v.double().abs(), 0.0).mean(dim=(0, 1))
+    for name, a, b, ref in (("o", o, ot, size), ("den", den[..., None], dent[..., None], None)):
+        assert torch.equal(a.isnan(), b.isnan()), f"{name}: not-a-number in other places"
+        assert torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()]), f"{name}: infinities in other places"
+        fin = b.isfinite()
+        a, b = torch.where(fin, a, 0.0), torch.where(fin, b, 0.0)
+        ref = b.abs().amax(dim=(0, 1)) if ref is None else ref
+        err = ((a - b).abs().amax(dim=(0, 1)) / ref.clamp_min(1e-300)).max().item()
+        assert err < 40 * UNIT, f"{name}: {err / UNIT:.0f} units of 2^-24 of a channel's size"
