@@ -441,14 +441,16 @@ __global__ __launch_bounds__(256, 2) void apply_kernel_bf(
     }
   };
   // streamed tiles travel through registers (they are scaled, and one of them transposed, on the
-  // way), two tiles ahead of their use: two sets of registers that take turns
+  // way), two tiles ahead of their use: two sets of registers that take turns.  In LDS they take turns in Sb2 and Sb3: the
+  // first one is staged by waves that are done with the last step of the state part while others may still read its
+  // slabs from Sb0 and Sb1, and Sb2 and Sb3 were last read a step, i.e. a barrier, before.
   RowTile<D, T, 32> t1a, t2a, t1b, t2b;
   auto tiles_load = [&](int kk, auto& u1, auto& u2) __attribute__((always_inline)) {
     u1.load(A1h, (tile0 + kk) * 32, n, tid);
     u2.load(A2h, (tile0 + kk) * 32, n, tid, a2dh, a2den_stride);
   };
   auto tiles_store = [&](int buf, auto& u1, auto& u2) __attribute__((always_inline)) {
-    uint16_t* tb = buf ? Sb1 : Sb0;
+    uint16_t* tb = buf ? Sb3 : Sb2;
     u1.store_bf(tb, LB, a1s, tid);
     u2.store_t_bf(tb + 32 * LB, TPB, 1.0f, tid);
   };
@@ -463,6 +465,7 @@ __global__ __launch_bounds__(256, 2) void apply_kernel_bf(
   }
   xt.store(Xl, LD, xs, tid);
   if (n_state == 0 && n_tile > 0) tiles_store(0, t1a, t2a);
+  FM_WAIT_VM(0);   // (the wave's own transfers; the barrier covers the other waves')
   __syncthreads();
 
   const int xrow = w * 32 + i;
@@ -628,7 +631,7 @@ __global__ __launch_bounds__(256, 2) void apply_kernel_bf(
       tiles_load(kk + 2 < n_tile ? kk + 2 : n_tile - 1, ld1, ld2);
       const int tl = tile0 + kk;
       if (FWD ? tl <= mine : tl >= mine) {
-        const uint16_t* l1 = buf ? Sb1 : Sb0;
+        const uint16_t* l1 = buf ? Sb3 : Sb2;
         const uint16_t* l2 = l1 + 32 * LB;
         // every LDS operand of the tile is requested first; the scores accumulate in two
         // independent chains
