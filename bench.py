@@ -502,8 +502,7 @@ def measure(name: str, args, full: bool) -> dict:
                     "frac": gbs / PEAK_HBM_GBS, "traffic": None, "bytes_per_step_of_this_kernel_class": bytes_per_step,
                     "ms_per_step_of_this_kernel_class": dom_ms}
     per_th = measured_traffic_bytes_per_token_head(name if not (full and args.batch) else "").get(dom)
-    # (the profiled bytes of the fp32 headline are those of the kernels on the fp32 instruction)
-    if per_th is not None and not dense and not runs_on_cut_operands(cfg, bh, dense):
+    if per_th is not None and not dense:
         n_states = n_builds if dom == "build" else 1
         roofline["traffic"] = per_th * token_heads * n_states / launches  # bytes per launch (profiled, not live)
         roofline["traffic_source"] = TRAFFIC_SOURCE[name]

@@ -103,3 +103,23 @@ def test_traffic_figures_are_read_from_the_committed_profiles():
         assert all(4 * 64 * es <= v < 8 * 64 * es for v in t.values()), (workload, t)
         assert max(t, key=t.get) == "bwd_dq"
     assert bench.measured_traffic_bytes_per_token_head("c2") == {}
+
+
+def test_every_name_a_program_uses_exists():
+    """The GPU half of the benchmark programs is not run here; a name that was removed elsewhere would only fail there."""
+    import builtins
+    import symtable
+
+    def uses(table):
+        for sym in table.get_symbols():
+            if sym.is_global() and sym.is_referenced():
+                yield sym.get_name()
+        for child in table.get_children():
+            yield from uses(child)
+
+    for name in ("bench.py", "bench_gpt.py", "bench_decode.py", "__graft_entry__.py"):
+        with open(os.path.join(ROOT, name)) as f:
+            top = symtable.symtable(f.read(), name, "exec")
+        known = {s.get_name() for s in top.get_symbols() if s.is_assigned() or s.is_imported() or s.is_namespace()}
+        missing = sorted(set(uses(top)) - known - set(dir(builtins)) - {"__file__"})
+        assert not missing, f"{name}: {missing}"

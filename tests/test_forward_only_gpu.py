@@ -56,6 +56,56 @@ def test_the_module_keeps_the_two_apart(built, mask):
 
 
 @gpu
+@pytest.mark.parametrize("d", [24, 64])
+@pytest.mark.parametrize("mask", [True, False])
+def test_strided_views_have_the_same_bits(built, d, mask):
+    """Slices of a fused projection, grouped heads, token-major output: the contiguous call's bits."""
+    from fastmax_amd import _ext
+
+    ext = _ext.load()
+    b, t, groups, r = 2, 290, 2, 3
+    x = torch.randn(b, t, groups, r + 2, d, generator=torch.Generator().manual_seed(d)).cuda()
+    q5, k4, v4 = x[:, :, :, :r].permute(0, 2, 3, 1, 4), x[:, :, :, r].permute(0, 2, 1, 3), x[:, :, :, r + 1].permute(0, 2, 1, 3)
+    tail = (mask, True, 1.0, 1.0, 1.0, 0.5, 1.0, 2, False, False)
+    o5, den = ext.forward_strided(q5, k4, v4, *tail)[:2]
+    o, den3 = ext.forward_ex(q5.reshape(-1, t, d), k4.reshape(-1, t, d), v4.reshape(-1, t, d), *tail)[:2]
+    assert torch.equal(o5.reshape(-1, t, d), o) and torch.equal(den, den3)
+
+
+@gpu
+def test_packed_projection_without_gradients(built):
+    """qkv_attention under no gradients against the same call with them (which has the training pass's bits)."""
+    from fastmax_amd import qkv_attention
+
+    qkv = torch.randn(2, 400, 4 * 3 * 64, generator=torch.Generator().manual_seed(3)).cuda()
+    y = qkv_attention(qkv, None, None, 4, 1, 64, rope_n=0)
+    yt = qkv_attention(qkv.clone().requires_grad_(True), None, None, 4, 1, 64, rope_n=0).detach()
+    assert not torch.equal(y, yt)
+    assert_close("y", y, yt, 40 * UNIT)
+
+
+@gpu
+def test_replays_of_a_captured_call(built):
+    """Inference loops capture the call: every replay has the eager call's bits, with eager work in between."""
+    from fastmax_amd import _ext
+
+    ext = _ext.load()
+    q, k, v = (t.cuda() for t in O.seeded_inputs((6, 300, 64), seed=11)[:3])
+    args = (q, k, v, True, True, 1.0, 1.0, 1.0, 0.5, 1.0, 2, False, False)
+    want = ext.forward_ex(*args)[0]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        o = ext.forward_ex(*args)[0]
+    for _ in range(4):
+        o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want)
+        assert torch.equal(ext.forward_ex(*args)[0], want)
+
+
+@gpu
 @pytest.mark.parametrize("bh,nq,nk,d,mask", [(256, 100, 1000, 32, True), (300, 100, 100, 64, False), (300, 100, 100, 64, True)])
 def test_half_empty_blocks_are_not_slower(built, bh, nq, nk, d, mask):
     """Blocks that hold few queries (a short sequence, or a few queries behind a key prefix) are made small: with eight waves
