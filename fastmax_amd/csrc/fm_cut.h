@@ -11,7 +11,7 @@
 // What bounds it: six v_mfma_f32_32x32x16_bf16 take ~200 cycles where eight v_mfma_f32_32x32x2f32 take 512; around them
 // the cutting of the weights (~5.5 VALU instructions a value) and the operand reads, three planes each.  The parts of
 // streamed rows are formed once per block on their way into LDS, those of own rows once per wave, only those of the
-// weights per tile.  Unmasked, 512 heads x 1000 x 64: 1164 us a pass on the fp32 instruction, 798 here.
+// weights per tile.  Unmasked, 512 heads x 1000 x 64: 1164 us a pass on the fp32 instruction, 800-840 here (by box).
 //
 // Not for passes that are differentiated.  The gradients of the first rows are differences of nearly equal numbers,
 // g . v - c with c formed from this output, and the row that carries the row-norm maximum takes the rounding of a whole
@@ -54,30 +54,6 @@ __device__ __forceinline__ Frag make(const float (&x)[8]) {
     parts(x[2 * e], x[2 * e + 1], w);
 #pragma unroll
     for (int k = 0; k < 3; ++k) f.p[k][e] = w[k];
-  }
-  return f;
-}
-// The same for the weights, which are formed in registers: what a part leaves is one dot product of the packed pair
-// instead of an unpacking and a subtraction (the whole pass 5 % faster).
-__device__ __forceinline__ Frag make_weights(const float (&x)[8]) {
-  // the pairs (-1, 0) and (0, -1), in registers: as a constant the compiler writes the first as the inline -1.0, which
-  // the instruction reads as the fp32 pattern, i.e. as the second
-  uint32_t LO, HI;
-  asm("s_mov_b32 %0, 0xbf80" : "=s"(LO));
-  asm("s_mov_b32 %0, 0xbf800000" : "=s"(HI));
-  Frag f;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float a = x[2 * e], b = x[2 * e + 1];
-    uint32_t w = pack_bf2(a, b);
-    f.p[0][e] = w;
-    a = fm_dot2_bf16(w, LO, a);
-    b = fm_dot2_bf16(w, HI, b);
-    w = pack_bf2(a, b);
-    f.p[1][e] = w;
-    a = fm_dot2_bf16(w, LO, a);
-    b = fm_dot2_bf16(w, HI, b);
-    f.p[2][e] = pack_bf2(a, b);
   }
   return f;
 }
@@ -263,7 +239,7 @@ __global__ __launch_bounds__(64 * NW, DP == 32 ? 4 : 2) void cut_fwd_kernel(
     static_for<NFA>([&](auto ftag) {
       constexpr int F = 8 * decltype(ftag)::value;
       const float x[8] = {sc[F], sc[F + 1], sc[F + 2], sc[F + 3], sc[F + 4], sc[F + 5], sc[F + 6], sc[F + 7]};
-      const Frag wa = make_weights(x);
+      const Frag wa = make(x);
       dn += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) acc[cb] = mma(wa, vb[F / 8][cb], acc[cb]);
