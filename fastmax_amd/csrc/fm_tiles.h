@@ -111,8 +111,8 @@ struct Copy {
   static __device__ __forceinline__ void transfer(const void* base, uint32_t offset, uint32_t dst) {
     // (in asm: behind the builtin the compiler waits for the transfer at the next LDS read of any buffer.  The compiler does not
     // see a memory instruction in it, so the five wait states from a vector instruction that writes a scalar register, as reading
-    // a spilled one back from a lane does, to a memory instruction that reads it are kept here: the move and four of s_nop.)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(offset), "s"(base) : "memory", "m0");
+    // a spilled one back from a lane does, to a memory instruction that reads it are kept here.)
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(dst), "v"(offset), "s"(base) : "memory");
   }
   // the stage's rows pos0 .. pos0 + BN - 1 to the tile at byte address lds
   __device__ __forceinline__ void issue(const HeadRows<const bf16_t>& hr, int pos0, int end, int d, uint32_t lds, int w, int l) const {

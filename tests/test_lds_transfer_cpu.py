@@ -1,7 +1,7 @@
 """The inline assembly that moves 16 bytes a lane from global memory to LDS (fastmax_amd/csrc/fm_tiles.h) hides a memory
 instruction from the compiler, so what the compiler would see to is checked on the listing of a probe: a base address
-that comes out of a lane is followed by five wait states before the instruction that reads it, and a value the compiler
-holds in m0 is not taken to survive the transfer.  hipcc cross-compiles for gfx950 without a GPU."""
+that comes out of a lane is followed by five wait states before the instruction that reads it, and m0 is written by the
+compiler itself, so that a value it holds there is not taken to survive the transfer.  hipcc cross-compiles for gfx950 without a GPU."""
 import os
 import re
 import subprocess
