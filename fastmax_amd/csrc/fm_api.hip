@@ -104,7 +104,6 @@ struct Plan {
   bool plain;          // every tensor is a plain contiguous (heads, tokens, d) array
   bool scan;           // causal p = 1 as one scan per head (fm_linear.h): no states in memory
   bool rowpass;        // unmasked p = 1: states from the build kernel, one pass over the rows per output
-  bool kv64;           // dense bf16 tiles: dk / dv blocks of 64 keys instead of 128
   bool dense;          // dense score tiles, no moment states (fm_dense.h): short sequences, and every head
                        // dimension other than 32 and 64
   bool lin;            // dense kernels in linear mode (p = 1, long sequences): chunk states of (dp + 1) rows in
@@ -215,15 +214,6 @@ Plan make_plan(const fastmax_desc* ds, int pass, bool plain = true, bool allow_d
     pl.scan = pl.rowpass = pl.split = false;
     pl.scratch_bytes = pl.per_head_bytes = 0;
     pl.state_floats = 0;
-    // bf16, p = 2, more than 96 channels: the dk / dv kernel's blocks hold a CU each, so that with few of them the longest walk is
-    // the time.  Half as wide they have half the walk, at 1.3 times the time a tile (its streamed tiles serve half as many keys):
-    // better where blocks of 128 keys leave half the CUs idle (unmasked, 32 heads on 8 of keys x 1024 x 128, 64 blocks: 79 us for
-    // 114; one head a key head, 128 blocks: 31.5 for 42.2, 160: 57.6 for 43.5), and under the mask, where the first keys' walk is
-    // twice the mean, while all are under way at once (272 blocks, 64 heads on 16 of keys x 2049 x 128: 199 us for 232; 256, 32 on
-    // 8 x 4096: 312 for 426; 320, one head a key head: 85.6 for 74.0).  Their partial sums, twice as many a head, have room in
-    // the workspace where key heads are at most half the query heads.
-    const int64_t wide = (int64_t)pl.bhkv * pl.nblk_k;
-    pl.kv64 = pl.p2 && ds->dtype == FASTMAX_BF16 && pl.d > 96 && pl.ratio >= 2 && wide <= (pl.masked && 2 * pl.nq > pl.nk ? 288 : 128);
     size_t fx = align256((size_t)2 * pl.bh * sizeof(float)) + align256((size_t)2 * pl.bh * sizeof(int));
     if (pass == FASTMAX_PASS_BACKWARD) {
       fx += align256((size_t)pl.bh * pl.nq * sizeof(float));
@@ -995,29 +985,27 @@ int cut_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const f
   return launch(std::integral_constant<int, 8>{});
 }
 
-// Score tiles of bf16 tensors at p = 2 (fm_tiles.h), forward.
+// Score tiles of bf16 tensors at p = 2 (fm_tiles.h).  (a2 = 0 is p = 1 without a linear mode: fm_dense.h skips what it would
+// multiply by zero.)
+bool use_tiles(const fastmax_desc* ds, const Plan& pl) { return ds->dtype == FASTMAX_BF16 && pl.p2 && ds->a2 != 0.f; }
+
+// ... forward
 template <int DP>
 int tiles_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const bf16_t* q, const bf16_t* k, const bf16_t* v,
-                  bf16_t* o, float* den, int64_t den_stride, const float* scale, const tiles::Square& sq, hipStream_t stream) {
+                  bf16_t* o, float* den, int64_t den_stride, const float* scale, hipStream_t stream) {
+  constexpr int BM = 128;
+  constexpr size_t smem = (size_t)2 * 2 * tiles::Geo<DP>::TILE;
   const int npos = pl.masked ? pl.nk : pl.nq;
   const int o_words = ((reinterpret_cast<uintptr_t>(o) | (uintptr_t)((L.o.sb | L.o.sg | L.o.sh | L.o.pitch) * 2)) & 7) == 0;   // rows on 8-byte boundaries
-  auto launch = [&](auto rttag, auto nwtag, auto nbuftag, auto occtag) -> int {
-    constexpr int RT = decltype(rttag)::value, NW = decltype(nwtag)::value, NBUF = decltype(nbuftag)::value, BM = 32 * RT * NW;
-    constexpr size_t smem = (size_t)NBUF * 2 * tiles::Geo<DP>::TILE;
-    auto kern = tiles::tiles_fwd_kernel<DP, RT, NW, NBUF, decltype(occtag)::value>;
-    FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
-    const int nb = (npos + BM - 1) / BM - pl.off / BM;
-    ScopedKernel sk(FASTMAX_K_FWD_APPLY, stream);
-    kern<<<dim3(pl.bh, nb), 64 * NW, smem, stream>>>(mk_rows(q, L.q, 0, pl.off), mk_rows(k, L.k), mk_rows(v, L.v), scale,
-                                                     scale + pl.bh, mk_rows(o, L.o, 0, pl.off),
-                                                     mk_scalars(den, pl.nq, den_stride, 0, pl.off), npos, pl.nk, ds->d,
-                                                     pl.masked, sq, pl.ratio, o_words);
-    return launch_status("tiles_fwd_kernel");
-  };
-#define IC(x) std::integral_constant<int, (x)>{}
-  // blocks of four waves, two stages of LDS: as many waves a SIMD as the registers allow.  (Two own tiles a wave: 72 us for
-  // 62 at 96 heads x 2048 x 64, 121 for 79 at 64 x 2049 x 128; eight waves or a third stage: no gain.)
-  return launch(IC(1), IC(4), IC(2), IC(DP <= 64 ? 3 : 2));
+  // blocks of four waves, two stages of LDS: as many waves a SIMD as the registers allow
+  auto kern = tiles::tiles_fwd_kernel<DP, (DP <= 64 ? 3 : 2)>;
+  FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
+  const int nb = (npos + BM - 1) / BM - pl.off / BM;
+  ScopedKernel sk(FASTMAX_K_FWD_APPLY, stream);
+  kern<<<dim3(pl.bh, nb), 256, smem, stream>>>(mk_rows(q, L.q, 0, pl.off), mk_rows(k, L.k), mk_rows(v, L.v), scale, scale + pl.bh,
+                                               mk_rows(o, L.o, 0, pl.off), mk_scalars(den, pl.nq, den_stride, 0, pl.off), npos, pl.nk,
+                                               ds->d, pl.masked, ds->a0, ds->a1, ds->a2, pl.ratio, o_words);
+  return launch_status("tiles_fwd_kernel");
 }
 
 template <class T>
@@ -1036,9 +1024,8 @@ int dense_forward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const
                          : cut_forward<64>(ds, pl, L, q, k, v, o, den, den_stride, scale, stream);
   }
   if constexpr (std::is_same<T, bf16_t>::value) {
-    tiles::Square sq;
-    if (pl.p2 && tiles::square_form(ds->a0, ds->a1, ds->a2, ds->normalize, 1.0f / ds->temperature, sq)) {
-#define FM_TILES_FWD(DP) return tiles_forward<DP>(ds, pl, L, q, k, v, o, den, den_stride, scale, sq, stream)
+    if (use_tiles(ds, pl)) {
+#define FM_TILES_FWD(DP) return tiles_forward<DP>(ds, pl, L, q, k, v, o, den, den_stride, scale, stream)
       if (ds->d <= 32) FM_TILES_FWD(32);
       if (ds->d <= 64) FM_TILES_FWD(64);
       if (ds->d <= 96) FM_TILES_FWD(96);
@@ -1115,53 +1102,48 @@ int dense_backward_dp(const fastmax_desc* ds, const Plan& pl, const Layout& L, c
 template <int DP>
 int tiles_backward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const bf16_t* q, const bf16_t* k, const bf16_t* v,
                    const bf16_t* o, const float* den, int64_t den_stride, const bf16_t* go, bf16_t* dq, bf16_t* dk, bf16_t* dv,
-                   const float* scale, float* cvec, float* rpart, const tiles::Square& sq, int* nbq_out, int* nbk_out,
-                   hipStream_t stream) {
+                   const float* scale, float* cvec, float* rpart, int* nbq_out, int* nbk_out, hipStream_t stream) {
   const int npos = pl.masked ? pl.nk : pl.nq;
   const RowScalars dn = mk_scalars(den, pl.nq, den_stride, 0, pl.off);
   const Rows<const bf16_t> qr = mk_rows(q, L.q, 0, pl.off), gr = mk_rows(go, L.go, 0, pl.off);
   const Rows<const bf16_t> kr = mk_rows(k, L.k), vr = mk_rows(v, L.v);
-  auto launch_dq = [&](auto rttag, auto nwtag, auto nbuftag, auto occtag) -> int {
-    constexpr int RT = decltype(rttag)::value, NW = decltype(nwtag)::value, NBUF = decltype(nbuftag)::value, BM = 32 * RT * NW;
-    constexpr size_t smem = (size_t)NBUF * 2 * tiles::Geo<DP>::TILE + NW * sizeof(float);
-    auto kern = tiles::tiles_dq_kernel<DP, RT, NW, NBUF, decltype(occtag)::value>;
+  constexpr int NWQ = dense::Shape<DP, bf16_t>::NW_DQ, BMQ = 32 * NWQ;   // (the partial sums are those of dense_dq_kernel's blocks)
+  const int nbq = (npos + BMQ - 1) / BMQ - pl.off / BMQ;
+  *nbq_out = nbq;
+  auto launch_dq = [&](auto occtag) -> int {
+    constexpr size_t smem = (size_t)2 * 2 * tiles::Geo<DP>::TILE + NWQ * sizeof(float);
+    auto kern = tiles::tiles_dq_kernel<DP, NWQ, decltype(occtag)::value>;
     FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
-    const int nb = (npos + BM - 1) / BM - pl.off / BM;
-    *nbq_out = nb;
     ScopedKernel sk(FASTMAX_K_BWD_DQ, stream);
-    kern<<<dim3(pl.bh, nb), 64 * NW, smem, stream>>>(qr, gr, dn, kr, vr, mk_rows(o, L.o, 0, pl.off), scale, scale + pl.bh,
-                                                     mk_rows(dq, L.dq, 0, pl.off), ds->normalize ? rpart : nullptr,
-                                                     mk_scalars<float>(cvec, pl.nq, 1, 0, pl.off), npos, pl.nk, ds->d,
-                                                     pl.masked, sq, pl.ratio);
+    kern<<<dim3(pl.bh, nbq), 64 * NWQ, smem, stream>>>(qr, gr, dn, kr, vr, mk_rows(o, L.o, 0, pl.off), scale, scale + pl.bh,
+                                                       mk_rows(dq, L.dq, 0, pl.off), ds->normalize ? rpart : nullptr,
+                                                       mk_scalars<float>(cvec, pl.nq, 1, 0, pl.off), npos, pl.nk, ds->d,
+                                                       pl.masked, ds->a1, ds->a2, pl.ratio);
     return launch_status("tiles_dq_kernel");
   };
-  auto launch_kv = [&](auto kwtag, auto swtag, auto occtag) -> int {
-    constexpr int KW = decltype(kwtag)::value, SW = decltype(swtag)::value, BM = 32 * KW;
-    constexpr size_t smem = tiles::DkDvLds<DP, KW, SW>::BYTES;
-    auto kern = tiles::tiles_dkdv_kernel<DP, KW, SW, decltype(occtag)::value>;
-    FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), smem));
-    const int nb = (pl.nk + BM - 1) / BM;
-    *nbk_out = nb;
-    ScopedKernel sk(FASTMAX_K_BWD_DK, stream);
-    kern<<<dim3(pl.bhkv, nb), 64 * KW * SW, smem, stream>>>(
-        kr, vr, qr, gr, dn, mk_scalars<const float>(cvec, pl.nq, 1, 0, pl.off), scale, scale + pl.bh, mk_rows(dk, L.dk),
-        mk_rows(dv, L.dv), ds->normalize ? rpart + (int64_t)pl.bh * (*nbq_out) : nullptr, npos, pl.nk, ds->d, pl.masked, sq, pl.ratio);
-    return launch_status("tiles_dkdv_kernel");
-  };
-  FM_TRY(launch_dq(IC(1), IC(4), IC(2), IC(DP <= 64 ? 3 : 2)));
-  // A key tile's walk over the queries is shared by two waves where there are too few blocks to fill the chip twice (272
-  // blocks, 64 heads on 16 of keys x 2049 x 64: 151 us for 174), and at 128 channels, where a CU holds one block (by four where
-  // blocks are half as wide); with more blocks one wave a tile is better (1536 blocks, 96 heads x 2048 x 64: 136 us for 184;
-  // all measured while grad_out still passed through registers).
-  if constexpr (DP == 128) {
-    if (pl.kv64) return launch_kv(IC(2), IC(4), IC(2));   // (the plan has the rule)
-    return launch_kv(IC(4), IC(2), IC(2));
+  // At 64 channels a block is eight waves: as two blocks a CU where there are that many, with half the registers and no operand
+  // reads ahead (us, one block a CU -> two: 512 blocks, 256 heads x 512 37.7 -> 28.9; 576, 64 heads x 2049 78.6 -> 71.9; 2048, 128 heads x
+  // 4096 433 -> 389; 64 blocks, 8 heads x 2048 40.8 -> 50.7).
+  if constexpr (DP == 64) {
+    if ((int64_t)pl.bh * nbq >= 512) FM_TRY(launch_dq(std::integral_constant<int, 4>{}));
+    else FM_TRY(launch_dq(std::integral_constant<int, 2>{}));
+  } else {
+    FM_TRY(launch_dq(std::integral_constant<int, (DP <= 32 ? 3 : 2)>{}));
   }
-  if constexpr (DP == 64)
-    if ((int64_t)pl.bhkv * ((pl.nk + 127) / 128) < 512) return launch_kv(IC(4), IC(2), IC(2));
-  if constexpr (DP < 128) return launch_kv(IC(4), IC(1), IC(2));
+  using KV = tiles::DkDv<DP>;
+  constexpr int BM = 32 * KV::KW;
+  static_assert(KV::KW == dense::Shape<DP, bf16_t>::NW_KV, "the partial sums are those of dense_dkdv_kernel's blocks");
+  auto kern = tiles::tiles_dkdv_kernel<DP>;
+  FM_TRY(allow_lds(reinterpret_cast<const void*>(kern), KV::BYTES));
+  const int nb = (pl.nk + BM - 1) / BM;
+  *nbk_out = nb;
+  ScopedKernel sk(FASTMAX_K_BWD_DK, stream);
+  kern<<<dim3(pl.bhkv, nb), 64 * KV::NW, KV::BYTES, stream>>>(
+      kr, vr, qr, gr, dn, mk_scalars<const float>(cvec, pl.nq, 1, 0, pl.off), scale, scale + pl.bh, mk_rows(dk, L.dk),
+      mk_rows(dv, L.dv), ds->normalize ? rpart + (int64_t)pl.bh * (*nbq_out) : nullptr, npos, pl.nk, ds->d, pl.masked, ds->a0,
+      ds->a1, ds->a2, pl.ratio);
+  return launch_status("tiles_dkdv_kernel");
 }
-#undef IC
 
 template <class T>
 int dense_backward(const fastmax_desc* ds, const Plan& pl, const Layout& L, const T* q, const T* k, const T* v,
@@ -1185,12 +1167,11 @@ int dense_backward(const fastmax_desc* ds, const Plan& pl, const Layout& L, cons
   if (pl.lin) qstate = reinterpret_cast<float*>(p + align256((size_t)pl.bhkv * pl.lslots * lin_state_floats(pl.ldp, 1) * sizeof(float)));
   if (!given) FM_TRY(compute_scales<T>(ds, L, q, k, scale_ws, arg_ws, stream));
   int nbq = 0, nbk = 0;
-  tiles::Square sq;
-  const bool square = std::is_same<T, bf16_t>::value && pl.p2 && tiles::square_form(ds->a0, ds->a1, ds->a2, ds->normalize, 1.0f / ds->temperature, sq);
+  const bool tiled = use_tiles(ds, pl);
   if constexpr (std::is_same<T, bf16_t>::value) {
 #define FM_TILES_BWD(DP)                                                                                                   \
-  FM_TRY((tiles_backward<DP>(ds, pl, L, q, k, v, o, den, den_stride, go, dq, dk, dv, scale, cvec, rpart, sq, &nbq, &nbk, stream)))
-    if (square) {
+  FM_TRY((tiles_backward<DP>(ds, pl, L, q, k, v, o, den, den_stride, go, dq, dk, dv, scale, cvec, rpart, &nbq, &nbk, stream)))
+    if (tiled) {
       if (ds->d <= 32) FM_TILES_BWD(32);
       else if (ds->d <= 64) FM_TILES_BWD(64);
       else if (ds->d <= 96) FM_TILES_BWD(96);
@@ -1201,7 +1182,7 @@ int dense_backward(const fastmax_desc* ds, const Plan& pl, const Layout& L, cons
 #define FM_DENSE_BWD(DP)                                                                                              \
   FM_TRY((dense_backward_dp<DP, T>(ds, pl, L, q, k, v, o, den, den_stride, go, dq, dk, dv, scale, cvec, rpart, kstate, \
                                    qstate, &nbq, &nbk, stream)))
-  if (square) {
+  if (tiled) {
   } else if (ds->d <= 32) FM_DENSE_BWD(32);
   else if (ds->d <= 64) FM_DENSE_BWD(64);
   else if (ds->d <= 96) FM_DENSE_BWD(96);

@@ -1,35 +1,28 @@
-// Dense score tiles of bf16 tensors at p = 2: the same sums as fm_dense.h, on a form of the polynomial that costs
-// one multiply-add an element, with operands that reach LDS without passing through registers.
+// Dense score tiles of bf16 tensors at p = 2: the sums of fm_dense.h bit for bit -- the same operands, rounded at the same
+// places, added in the same order -- by kernels whose streamed operands reach LDS without passing through registers.
+// (A kernel that rounds elsewhere can be as good and one multiply-add a score cheaper: f as a shifted square, with 1 / den on the
+// weights.  But its weights lose what a0 holds where a0 is small against a1^2 / a2, and its results are others than those
+// of a version before.)
 //
 // What bounds these kernels is the matrix instruction -- as long as nothing else gets in its way.  Measured on
 // the chip, v_mfma_f32_32x32x16_bf16 occupies the matrix unit for 32 cycles and leaves the SIMD's other ports
 // free: one wave that issues one matrix instruction and five VALU instructions in turn takes 36 cycles a group,
 // and two waves in different phases of their work (eight matrix instructions, then 32 VALU ones) 42 cycles a
 // matrix instruction, not 32 + 20.  (The fp32 instruction is different: it does keep the VALU from issuing.)
-// So the two sides are balanced against each other and against LDS:
 //
-//   * f(s) = a0 + a1 s + a2 s^2 = A [(t s + h)^2 + c]: t rides on an own operand and h is the value the score
-//     accumulator starts from, so u = t s + h is what the matrix instruction delivers, f / A = u^2 + c is ONE
-//     multiply-add of it, f'(s) = 2 A t u is that accumulator itself, and the constants go to the epilogues.
-//     Coefficients it does not suit (a2 zero or small against a1) stay with fm_dense.h: see square_form.
-//   * K, V, Q and grad_out tiles go global -> LDS directly, as stored, row-major only; the second contraction
+//   * K, V and Q tiles go global -> LDS directly, as stored, row-major only; the second contraction
 //     reads them through the transposing LDS load.  The copies take no registers and no VALU work, and
 //     a stage is under way while the stage before it is computed.  Rows are 16-byte chunks whose place in
 //     the row is XORed with a function of the row number, so that row reads and transposing reads both touch every bank once.
-//   * the second contraction is formed transposed (channels x own rows), so that a lane ends up with its own row's
-//     channels: scales and 1 / den are one factor a lane, and rows go out in 8-byte pieces.
 //   * LDS reads run a few steps ahead of the matrix instructions that use them, in an order the compiler is not left to
 //     choose (see steps).
-// What is left: the waits between a wave's phases (scores, polynomial, second contraction), which two or three waves a
-// SIMD hide in part.  LDS delivers 256 bytes a cycle (an operand read takes a CU 4.1 cycles), one operand per matrix
-// instruction is half of that, and the dk / dv kernel needs up to 0.8; two own tiles a wave would halve it, but their
-// registers leave one wave a SIMD, whose VALU work nothing then hides (dq at d = 64: 153 us against 88).  Counters at 128
-// heads x 4096 x 64, forward: matrix unit busy 58 % at 1.8 GHz, to which the chip slows down under this load (2.1 GHz with
-// it 28 % busy).
-// us a launch, fm_dense.h -> these, GPU clock as it comes:            forward        dq            dk, dv
-//   96 heads x 2048 x 64, causal                                      86 -> 61     132 -> 84     187 -> 132
-//   64 heads on 16 of keys x 2049 x 128, causal                      139 -> 79     275 -> 121    554 -> 199
-//   64 heads x 1000 queries behind 3000 keys x 64                    122 -> 77
+//   * rows leave in 8-byte pieces from the forward kernel, whose second contraction is formed transposed (channels x own
+//     rows); in the backward kernels, where the order of a sum over the outputs is that of lanes = channels, through LDS.
+// What is left: the waits between a wave's phases (scores, polynomial, second contraction), which two to four waves a
+// SIMD hide in part, and 4 to 9 VALU instructions a matrix instruction.  LDS delivers 256 bytes a cycle (an operand read takes a CU 4.1
+// cycles) and is a quarter busy.  Without gain: one tile's polynomial placed between the next tile's matrix instructions
+// (d = 64, 128 heads x 4096: dk / dv 710 us for 691, dq 444 for 431), one wave a SIMD with 512 registers in dk / dv at d = 128 (350
+// for 319), blocks of four waves that take two 128-row parts in turn (dk / dv 720).
 #pragma once
 #include "fm_common.h"
 #include "fm_dense.h"
@@ -39,32 +32,6 @@ namespace tiles {
 using dense::kZero16;
 using M = dense::Mma<bf16_t>;
 using Frag = M::Frag;
-
-// The polynomial as a shifted square (see above).  f's sign and any positive factor m^2 may go into A.
-struct Square {
-  float t, h, c, A;
-};
-// Whether the form suits the coefficients, and the form.  Its terms are of size h^2 against max |a|: up to 256 times that,
-// the fp32 rounding of the square (2^-24) stays below 2^-16 of the polynomial's coefficients, where the weights' bf16
-// rounding is 2^-9.  (A NaN or an infinity among the coefficients fails the comparison.)
-// m: with normalised rows the scores are small and the weights near a0, so m^2 = 9/8 |a0| puts them just below 1, where a
-// bf16 step is smallest against the value (half of what it is just above); without normalisation m makes the scale
-// kq t of the own operand a power of two, which rounds nothing.
-inline bool square_form(float a0, float a1, float a2, bool normalize, float kq, Square& sq) {
-  const float top = __builtin_fmaxf(__builtin_fabsf(a0), __builtin_fmaxf(__builtin_fabsf(a1), __builtin_fabsf(a2)));
-  const float sg = a2 < 0.f ? -1.f : 1.f, t = __builtin_sqrtf(__builtin_fabsf(a2)), h = sg * a1 / (2.0f * t);
-  if (!(t > 0.f && top <= 1e18f && h * h <= 256.0f * top)) return false;
-  float m = 1.0f;
-  if (normalize) {
-    if (__builtin_fabsf(a0) >= 0x1p-20f * top) m = __builtin_sqrtf(1.125f * __builtin_fabsf(a0));
-  } else {
-    int e;
-    const float x = __builtin_fabsf(kq) * t;
-    if (x >= 0x1p-60f && x <= 0x1p60f) m = 2.0f * __builtin_frexpf(x, &e);
-  }
-  sq = Square{t / m, h / m, (sg * a0 - h * h) / (m * m), sg * m * m};
-  return true;
-}
 
 template <int DP>
 struct Geo {
@@ -83,21 +50,26 @@ struct Geo {
   static constexpr int KEYS = CPR == 16 ? 16 : CPR == 8 ? 8 : 4;   // chunks a key can move a chunk among
 };
 
-// waits until at most N transfers to LDS of this wave are under way and its LDS reads are done, then for the
-// block: behind it every wave sees what all have staged, and buffers read before it may be overwritten
-template <int N>
-__device__ __forceinline__ void stage_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+// waits for this wave's transfers to LDS and its LDS reads, then for the block: behind it every wave sees what all have
+// staged, and buffers read before it may be overwritten
+__device__ __forceinline__ void stage_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// the lane number, made anew where it is called: what an epilogue derives from it is not prepared before the loops and kept through them
+__device__ __forceinline__ int fresh_lane() {
+  int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  asm volatile("" : "+v"(l));
+  return l;
 }
 
 // One streamed tensor's share of a stage for this wave: chunk (u NW + wave) 64 + lane of the tile, u = 0..NI-1.
 // Rows outside [lo, end) are fetched from the nearest row inside and channels past d from the row's last chunk:
 // valid addresses whose products the kernels' masks, zero operands and stores leave out.
-template <int DP, int NW>
+template <int DP, int NW, bool LEAN = false>
 struct Copy {
   using G = Geo<DP>;
-  static constexpr int NI = G::BN * G::CPR / 64 / NW;
-  static_assert(NI * 64 * NW == G::BN * G::CPR, "every lane moves whole chunks");
+  static constexpr int ALL = G::BN * G::CPR / 64, NI = (ALL + NW - 1) / NW;
+  static constexpr bool EVEN = ALL % NW == 0;   // (12 instructions of 96 channels on eight waves: four waves have a second one)
+  static __device__ __forceinline__ bool has(int u, int w) { return EVEN || u * NW + w < ALL; }
   uint32_t off[NI];   // bytes from the tile's first row to this lane's chunk in instruction u
   static __device__ __forceinline__ int row(int u, int w, int l) { return ((u * NW + w) * 64 + l) / G::CPR; }
   static __device__ __forceinline__ int channel(int u, int w, int l, int d) {
@@ -120,14 +92,22 @@ struct Copy {
     if (pos0 >= hr.lo && pos0 + G::BN <= end) {   // (uniform) nothing to clamp: the lane's offsets stand
       const bf16_t* base = hr.base + (uint64_t)((unsigned)pos0 * hr.pitch);
 #pragma unroll
-      for (int u = 0; u < NI; ++u) transfer(base, off[u], dst + u * NW * 1024);
+      for (int u = 0; u < NI; ++u)
+        if (has(u, w)) {
+          uint32_t o = off[u];
+          if constexpr (LEAN) {   // (no register to keep it in)
+            const int k = fresh_lane();
+            o = ((unsigned)row(u, w, k) * hr.pitch + (unsigned)channel(u, w, k, d)) * 2u;
+          }
+          transfer(base, o, dst + u * NW * 1024);
+        }
     } else {
-      asm volatile("" : "+v"(l));   // (rare: nothing of it is kept in registers)
+      l = fresh_lane();   // (rare: nothing of it is kept in registers)
 #pragma unroll
       for (int u = 0; u < NI; ++u) {
         const int p = pos0 + row(u, w, l);
         const int ps = max(p < end ? p : end - 1, hr.lo);
-        transfer(hr.base, ((unsigned)ps * hr.pitch + (unsigned)channel(u, w, l, d)) * 2u, dst + u * NW * 1024);
+        if (has(u, w)) transfer(hr.base, ((unsigned)ps * hr.pitch + (unsigned)channel(u, w, l, d)) * 2u, dst + u * NW * 1024);
       }
     }
   }
@@ -193,6 +173,68 @@ __device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
 }
 
+// 32 rows of a sum in accumulators (registers = rows r0 + trow, lanes = channels), times `scale`, to the rows inside
+// [lo, end); `dot`: also this lane's part of their inner product with the rows of x, over rows and then channels as the
+// fm_dense.h kernels take them.  Rows pass through LDS (32 rows of this wave's own): the accumulators' layout has a lane hold two
+// bytes of a row, and loads and stores of two bytes keep the address unit busy 16 cycles each (a block of eight waves x 64 channels: 2 us
+// for x and 4 to 6 for dk and dv, with nothing beside them).
+template <int DP>
+__device__ __forceinline__ float store_rows(const f16v (&acc)[DP / 32], float scale, const HeadRows<bf16_t>& out, const HeadRows<const bf16_t>& x,
+                                            bool dot, int r0, int lo, int end, int d, unsigned char* lds) {
+  using G = Geo<DP>;
+  constexpr int CB = DP / 32, CPR = G::CPR, N = CPR / 2, SH = CPR % 8 == 0 ? 2 : 1;
+  const int lane = fresh_lane(), c0 = lane & 31, hh = lane >> 5;
+  // chunk c of row r is kept at chunk c ^ (r / 4 % 2 << SH): the two halves of a wave, four rows apart, use different banks
+  auto at = [&](int row, int chunk) { return lds + row * G::PITCH + ((chunk ^ ((row >> 2 & 1) << SH)) << 4); };
+  // channel cb * 32 + c0 of row trow(r, hh): one address a lane for even cb, one for odd, constants on top
+  unsigned char* const even = lds + 4 * hh * G::PITCH + (((c0 >> 3) ^ (hh << SH)) << 4) + (c0 & 7) * 2;
+  unsigned char* const odd = SH == 2 ? lds + 4 * hh * G::PITCH + (((4 + (c0 >> 3)) ^ (hh << SH)) << 4) + (c0 & 7) * 2 : even + 64;
+  auto elt = [&](int r, int cb) { return reinterpret_cast<uint16_t*>((cb & 1 ? odd : even) + (cb >> 1) * 128 + (8 * (r >> 2) + (r & 3)) * G::PITCH); };
+  const bool whole = r0 >= lo && r0 + 32 <= end && d == DP;   // (uniform)
+  float rs = 0.f;
+  if (dot) {
+    uint4 t[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int row = (u * 64 + lane) / CPR, ch = (u * 64 + lane) % CPR * 8, pos = r0 + row;
+      t[u] = *reinterpret_cast<const uint4*>(x.base + ((unsigned)max(pos < end ? pos : end - 1, lo) * x.pitch + (unsigned)(ch < d ? ch : 0)));
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) *reinterpret_cast<uint4*>(at((u * 64 + lane) / CPR, (u * 64 + lane) % CPR)) = t[u];
+    asm volatile("" ::: "memory");   // (a wave's LDS accesses are carried out in their order)
+    auto term = [&](int r, int cb) { return __builtin_fmaf(acc[cb][r] * scale, dense::to_f32_elt(*elt(r, cb)), rs); };
+    if (whole) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) rs = term(r, cb);
+    } else {
+      FM_KEEP_BRANCH();
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+          const int pos = r0 + trow(r, hh);
+          const float t1 = term(r, cb);
+          rs = pos >= lo && pos < end && cb * 32 + c0 < d ? t1 : rs;
+        }
+    }
+    asm volatile("" ::: "memory");
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) *elt(r, cb) = M::to_elt(acc[cb][r] * scale);
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int row = (u * 64 + lane) / CPR, chunk = (u * 64 + lane) % CPR, pos = r0 + row;
+    if (pos >= lo && pos < end && chunk * 8 < d)
+      *reinterpret_cast<uint4*>(out.base + ((unsigned)pos * out.pitch + (unsigned)(chunk * 8))) = *reinterpret_cast<const uint4*>(at(row, chunk));
+  }
+  return rs;
+}
+
 // The fragments of one own row (position pos of the head), times `scale`: fragment m holds channels 16 m + 8 hh .. + 7.  A
 // row outside [lo, end) gives zeros, and so do channels past d.  Uniform base, 32-bit lane offset, and the offset is made
 // anew on every call: hoisted out of a loop, one 64-bit address per fragment would stay in registers.
@@ -210,16 +252,16 @@ __device__ __forceinline__ void own_row(const HeadRows<const bf16_t>& hr, int po
     float x[8];
     M::unpack(t, x);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = live && ok ? x[e] * scale : 0.f;
-    f[m] = __builtin_bit_cast(Frag, M::pack(x));
+    for (int e = 0; e < 8; ++e) x[e] *= scale;
+    const Frag y = __builtin_bit_cast(Frag, M::pack(x));
+    f[m] = live && ok ? y : M::zero();
   }
 }
 
 // N steps of a contraction whose operands come from LDS: step I reads the operands of step I + AHEAD (load) before it
 // uses its own (use).  A read takes as long as four or more matrix instructions, and the compiler's own order -- read, wait, one
-// matrix instruction -- leaves the matrix unit idle most of that time; the fence keeps LDS reads and matrix instructions
-// in the order written here and lets everything else move across.  The first AHEAD reads are issued by `prime`, so that they can
-// be placed under the work before the contraction.
+// matrix instruction -- leaves the matrix unit idle most of that time; the fences keep what a step holds in that step.  The
+// first AHEAD reads are issued by `prime`, so that they can be placed under the work before the contraction.
 __device__ __forceinline__ void order_fence() { __builtin_amdgcn_sched_barrier(0); }
 template <int N, int AHEAD, class Load>
 __device__ __forceinline__ void prime(Load&& load) {
@@ -240,20 +282,19 @@ __device__ __forceinline__ void steps(Load&& load, Use&& use) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Forward.  grid = (heads, query blocks of 32 RT NW positions from the one that holds position Q.lo); npos: positions of
-// the queries end here (nk under the mask: query i sits at position i + nk - nq).  NBUF stages of LDS.
+// Forward.  grid = (heads, query blocks of 128 positions from the one that holds position Q.lo); npos: positions of
+// the queries end here (nk under the mask: query i sits at position i + nk - nq).  Two stages of LDS.  (Eight waves, a third stage: no
+// gain; two own tiles a wave, half the LDS reads: 72 us for 62 at 96 heads x 2048 x 64, 121 for 79 at 64 x 2049 x 128.)
 // ---------------------------------------------------------------------------------------
-// RT own tiles a wave; OCC waves a SIMD.
-template <int DP, int RT, int NW, int NBUF, int OCC>
-__global__ __launch_bounds__(64 * NW, OCC) void tiles_fwd_kernel(
+template <int DP, int OCC>   // OCC: waves a SIMD
+__global__ __launch_bounds__(256, OCC) void tiles_fwd_kernel(
     Rows<const bf16_t> Q, Rows<const bf16_t> K, Rows<const bf16_t> V, const float* __restrict__ qscale,
-    const float* __restrict__ kscale, Rows<bf16_t> O, RowScalarsOut den, int npos, int nk, int d, int masked, Square sq, int ratio,
-    int o_words) {
+    const float* __restrict__ kscale, Rows<bf16_t> O, RowScalarsOut den, int npos, int nk, int d, int masked, float a0, float a1, float a2,
+    int ratio, int o_words) {
   using G = Geo<DP>;
+  constexpr int NW = 4, NF = DP / 16, CB = DP / 32, BM = 32 * NW, BN = G::BN, STAGE = 2 * G::TILE;
   using C = Copy<DP, NW>;
-  constexpr int NF = DP / 16, CB = DP / 32, BM = 32 * RT * NW, BN = G::BN, PD = NBUF - 1;
-  constexpr int STAGE = 2 * G::TILE;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_smem[];   // [NBUF][K tile, V tile]
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_smem[];   // [2][K tile, V tile]
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, hh = l >> 5;
   const int nb = gridDim.y, bx = blockIdx.y;
@@ -273,31 +314,21 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_fwd_kernel(
     cv.issue(Vh, st * BN, nk, d, lds0 + buf * STAGE + G::TILE, w, l);
   };
   issue(0, 0);
-  if (PD > 1 && nst > 1) issue(1, 1);
 
-  const float kq = qscale[head] * kscale[hkv] * sq.t;
-  Frag qf[RT][NF];
-  const int q00 = tok0 + w * RT * 32;   // first position of the wave's own tile 0
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) own_row<DP>(Qh, q00 + rt * 32 + i, npos, d, hh, kq, qf[rt]);
+  const float kq = qscale[head] * kscale[hkv];
+  Frag qf[NF];
+  const int q0 = tok0 + w * 32;   // first position of the wave's own tile
+  own_row<DP>(Qh, q0 + i, npos, d, hh, kq, qf);
   Reads<DP> rd;
   rd.init(l);
-  const f16v start = splat16(sq.h);
 
-  f16v acc[RT][CB];
-  float dn[RT];
+  f16v acc[CB];
+  float dn = 0.f;
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    dn[rt] = 0.f;
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) acc[rt][cb] = kZero16;
-  }
+  for (int cb = 0; cb < CB; ++cb) acc[cb] = kZero16;
 
-  // One 32-key tile against the wave's own tiles.  EDGE: rel = key tile base - first position of own tile 0: own
-  // tile rt has the key tile on its diagonal when rel == 32 rt and wholly after its queries when rel > 32 rt;
-  // keys left of the sequence's end: `left`.  Only these tiles pay for per-element tests.
   constexpr int RA = 3, CA = 2;   // operand steps read ahead
-  auto scores = [&](const unsigned char* kl, int t32, f16v (&sc)[RT]) __attribute__((always_inline)) {
+  auto scores = [&](const unsigned char* kl, int t32, f16v& sc) __attribute__((always_inline)) {
     Frag ka[RA + 1];
     auto rows = [&](auto m) __attribute__((always_inline)) {
       constexpr int I = decltype(m)::value;
@@ -306,27 +337,26 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_fwd_kernel(
     prime<NF, RA>(rows);
     steps<NF, RA>(rows, [&](auto m) __attribute__((always_inline)) {
       constexpr int I = decltype(m)::value;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) sc[rt] = M::mma(ka[I % (RA + 1)], qf[rt][I], I == 0 ? start : sc[rt]);
+      sc = M::mma(ka[I % (RA + 1)], qf[I], I == 0 ? kZero16 : sc);
     });
   };
-  auto weights = [&](f16v (&sc)[RT]) __attribute__((always_inline)) {
+  auto weights = [&](f16v& sc) __attribute__((always_inline)) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sc[rt][r] = sc[rt][r] * sc[rt][r] + sq.c;
-  };
-  auto edge = [&](f16v (&sc)[RT], int rel, int left) __attribute__((always_inline)) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int lim = masked ? (rel > 32 * rt ? -1 : rel == 32 * rt ? i : 31) : 31;
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (trow(r, hh) > lim || trow(r, hh) >= left) sc[rt][r] = 0.f;
+    for (int r = 0; r < 16; ++r) {
+      const float s = sc[r];
+      sc[r] = a0 + s * (a1 + a2 * s);
     }
   };
-  auto values = [&](const unsigned char* vl, int t32, const f16v (&sc)[RT]) __attribute__((always_inline)) {
-    Frag vc[CA + 1], wa[RT];
+  // a key tile on the own tile's diagonal, or with no more than `left` keys before the sequence's end: only these pay for
+  // per-element tests
+  auto edge = [&](f16v& sc, bool diagonal, int left) __attribute__((always_inline)) {
+    const int lim = diagonal ? i : 31;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (trow(r, hh) > lim || trow(r, hh) >= left) sc[r] = 0.f;
+  };
+  auto values = [&](const unsigned char* vl, int t32, const f16v& sc) __attribute__((always_inline)) {
+    Frag vc[CA + 1], wa;
     auto cols = [&](auto n) __attribute__((always_inline)) {
       constexpr int I = decltype(n)::value;
       vc[I % (CA + 1)] = rd.col(vl, t32, I / CB, I % CB);
@@ -334,35 +364,31 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_fwd_kernel(
     prime<2 * CB, CA>(cols);
     steps<2 * CB, CA>(cols, [&](auto n) __attribute__((always_inline)) {
       constexpr int I = decltype(n)::value, F = I / CB, cb = I % CB;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        if constexpr (cb == 0) {
-          wa[rt] = M::template from_acc<F>(sc[rt]);
-          dn[rt] = M::fsum(wa[rt], dn[rt]);
-        }
-        acc[rt][cb] = M::mma(vc[I % (CA + 1)], wa[rt], acc[rt][cb]);
+      if constexpr (cb == 0) {
+        wa = M::template from_acc<F>(sc);
+        dn = M::fsum(wa, dn);
       }
+      acc[cb] = M::mma(vc[I % (CA + 1)], wa, acc[cb]);
     });
   };
 
   int buf = 0;
-  // the stage is in LDS, the one PD further on its way
+  // the stage is in LDS, the one after it on its way
   auto next_stage = [&](int st) __attribute__((always_inline)) -> const unsigned char* {
-    if (PD > 1 && st + 1 < nst) stage_barrier<2 * C::NI>();
-    else stage_barrier<0>();
-    if (st + PD < nst) issue(st + PD, buf == 0 ? NBUF - 1 : buf - 1);
+    stage_barrier();
+    if (st + 1 < nst) issue(st + 1, buf ^ 1);
     const unsigned char* kl = tiles_smem + buf * STAGE;
-    buf = buf + 1 == NBUF ? 0 : buf + 1;
+    buf ^= 1;
     return kl;
   };
   // stages whose keys all exist and lie before every own query; then the rest (none of this diverges within a wave,
   // and every wave of the block passes nst barriers)
-  const int n_in = (masked && q00 < nk ? q00 : nk) / BN < nst ? (masked && q00 < nk ? q00 : nk) / BN : nst;
+  const int n_in = (masked && q0 < nk ? q0 : nk) / BN < nst ? (masked && q0 < nk ? q0 : nk) / BN : nst;
   int st = 0;
   for (; st < n_in; ++st) {
     const unsigned char* kl = next_stage(st);
     const unsigned char* vl = kl + G::TILE;
-    f16v s0[RT], s1[RT];
+    f16v s0, s1;
     scores(kl, 0, s0);
     weights(s0);
     scores(kl, 1, s1);
@@ -376,11 +402,11 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_fwd_kernel(
 #pragma unroll 1
     for (int t32 = 0; t32 < 2; ++t32) {
       const int kt = st * BN + t32 * 32;
-      if (kt >= nk || (masked && kt > q00 + 32 * (RT - 1))) continue;   // past the end, or after every own query
-      f16v s[RT];
+      if (kt >= nk || (masked && kt > q0)) continue;   // past the end, or after every own query
+      f16v s;
       scores(kl + t32 * 32 * G::PITCH, 0, s);
       weights(s);
-      edge(s, kt - q00, nk - kt);
+      edge(s, masked && kt == q0, nk - kt);
       values(vl + t32 * 32 * G::PITCH, 0, s);
     }
   }
@@ -388,53 +414,48 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_fwd_kernel(
   // lanes = own queries, registers 4 j .. 4 j + 3 of a column block = channels 8 j + 4 hh ..
   const HeadRows<bf16_t> Oh = O.head(head);
   float* denh = den.head(head);
+  const float tot = dn + other_half(dn, hh);
+  const int pos = q0 + i;
+  if (pos < npos && pos >= Qh.lo) {
+    const float inv = 1.0f / tot;
+    bf16_t* row = Oh.base + (unsigned)pos * Oh.pitch + 4 * hh;
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const float tot = dn[rt] + other_half(dn[rt], hh);
-    const int pos = q00 + rt * 32 + i;
-    if (pos < npos && pos >= Qh.lo) {
-      const float inv = 1.0f / tot;
-      bf16_t* row = Oh.base + (unsigned)pos * Oh.pitch + 4 * hh;
+    for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (cb * 32 + 8 * j < d) {
-            const uint2 x = pack_bf4u(acc[rt][cb][4 * j] * inv, acc[rt][cb][4 * j + 1] * inv, acc[rt][cb][4 * j + 2] * inv,
-                                      acc[rt][cb][4 * j + 3] * inv);
-            bf16_t* to = row + cb * 32 + 8 * j;
-            if (o_words) {
-              *reinterpret_cast<uint2*>(to) = x;
-            } else {   // (rows of o that do not start on 8-byte boundaries, e.g. d + 1 elements apart)
-              to[0].x = (uint16_t)x.x;
-              to[1].x = (uint16_t)(x.x >> 16);
-              to[2].x = (uint16_t)x.y;
-              to[3].x = (uint16_t)(x.y >> 16);
-            }
+      for (int j = 0; j < 4; ++j)
+        if (cb * 32 + 8 * j < d) {
+          const uint2 x = pack_bf4u(acc[cb][4 * j] * inv, acc[cb][4 * j + 1] * inv, acc[cb][4 * j + 2] * inv, acc[cb][4 * j + 3] * inv);
+          bf16_t* to = row + cb * 32 + 8 * j;
+          if (o_words) {
+            *reinterpret_cast<uint2*>(to) = x;
+          } else {   // (rows of o that do not start on 8-byte boundaries, e.g. d + 1 elements apart)
+            to[0].x = (uint16_t)x.x;
+            to[1].x = (uint16_t)(x.x >> 16);
+            to[2].x = (uint16_t)x.y;
+            to[3].x = (uint16_t)(x.y >> 16);
           }
-      if (hh == 0) denh[(int64_t)pos * den.stride] = sq.A * tot;
-    }
+        }
+    if (hh == 0) denh[(int64_t)pos * den.stride] = tot;
   }
 }
 
 // ---------------------------------------------------------------------------------------
-// dq.  The forward kernel's walk with two score tiles a step: u as there, and P = grad_out . v - grad_out . o,
-// whose start value is the own row's -grad_out . o.  W = u P goes straight back as the operand of W . K; what is
-// constant in a row -- scales, 1 / den, f' = 2 A t u -- waits for the epilogue.  c_i = grad_out_i . o_i / den_i
-// is left in cprep for the dk / dv kernel.  rpart[head * gridDim.y + block] receives the block's sum of dq . q for
-// the normalisation chain rule (when rpart is given).
+// dq.  The forward kernel's walk with two score tiles a step: the own rows carry q times 2 a2, so that the score
+// accumulator, started at a1, is f'(s), and g = grad_out / den, whose accumulator starts at -c.  W = f'(s) (g . v - c) goes
+// straight back as the operand of W . K.  c_i = grad_out_i . o_i / den_i is left in cprep for the dk / dv kernel.
+// rpart[head * gridDim.y + block] receives the block's sum of dq . q for the normalisation chain rule (when rpart is
+// given), a sum whose order is part of the result: that of the lanes and rows of dense_dq_kernel, blocks as wide as there.
 // ---------------------------------------------------------------------------------------
-template <int DP, int RT, int NW, int NBUF, int OCC>
+template <int DP, int NW, int OCC>
 __global__ __launch_bounds__(64 * NW, OCC) void tiles_dq_kernel(
     Rows<const bf16_t> Q, Rows<const bf16_t> GO, RowScalars den, Rows<const bf16_t> K, Rows<const bf16_t> V,
     Rows<const bf16_t> OUTF, const float* __restrict__ qscale, const float* __restrict__ kscale, Rows<bf16_t> DQ,
-    float* __restrict__ rpart, RowScalarsOut cprep, int npos, int nk, int d, int masked, Square sq, int ratio) {
+    float* __restrict__ rpart, RowScalarsOut cprep, int npos, int nk, int d, int masked, float a1, float a2, int ratio) {
   using G = Geo<DP>;
-  using C = Copy<DP, NW>;
-  constexpr int NF = DP / 16, CB = DP / 32, BM = 32 * RT * NW, BN = G::BN, PD = NBUF - 1;
-  constexpr int STAGE = 2 * G::TILE;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_smem[];   // [NBUF][K tile, V tile], [NW]
-  float* red = reinterpret_cast<float*>(tiles_smem + NBUF * STAGE);
+  using C = Copy<DP, NW, (OCC == 4)>;
+  constexpr int NF = DP / 16, CB = DP / 32, BM = 32 * NW, BN = G::BN, STAGE = 2 * G::TILE;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_smem[];   // [2][K tile, V tile], [NW]
+  float* red = reinterpret_cast<float*>(tiles_smem + 2 * STAGE);
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, hh = l >> 5;
   const int nb = gridDim.y, bx = blockIdx.y;
@@ -453,61 +474,66 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_dq_kernel(
     cv.issue(Vh, st * BN, nk, d, lds0 + buf * STAGE + G::TILE, w, l);
   };
   issue(0, 0);
-  if (PD > 1 && nst > 1) issue(1, 1);
 
-  const float kq = qscale[head] * kscale[hkv];
-  const int q00 = tok0 + w * RT * 32;
-  Frag qf[RT][NF], gf[RT][NF];
-  float rden[RT], craw[RT];
+  const float kq = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, qscale[head] * kscale[hkv])));   // (uniform, in a scalar register)
+  const int q0 = tok0 + w * 32;
+  Frag qf[NF], gf[NF];
+  float c;
   {
     const HeadRows<const bf16_t> Gh = GO.head(head), OFh = OUTF.head(head);
-    const float* denh = den.head(head);
-    float* cw = cprep.head(head);
+    const int pos = q0 + i;
+    const bool live = pos >= Qh.lo && pos < npos;
+    const int ps = max(pos < npos ? pos : npos - 1, Qh.lo);
+    const float rden = (live ? 1.0f : 0.f) / den.head(head)[(int64_t)ps * den.stride];
+    own_row<DP>(Qh, pos, npos, d, hh, kq * 2.0f * a2, qf);
+    const bf16_t* grow = Gh.base + (unsigned)ps * Gh.pitch;
+    const bf16_t* orow = OFh.base + (unsigned)ps * OFh.pitch;
+    float dot = 0.f;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int pos = q00 + rt * 32 + i;
-      const bool live = pos >= Qh.lo && pos < npos;
-      const int ps = max(pos < npos ? pos : npos - 1, Qh.lo);
-      rden[rt] = 1.0f / denh[(int64_t)ps * den.stride];
-      own_row<DP>(Qh, pos, npos, d, hh, kq * sq.t, qf[rt]);
-      const bf16_t* grow = Gh.base + (unsigned)ps * Gh.pitch;
-      const bf16_t* orow = OFh.base + (unsigned)ps * OFh.pitch;
-      float dot = 0.f;
+    for (int m = 0; m < NF; ++m) {
+      const int ch = 16 * m + 8 * hh;
+      const bool ok = live && ch < d;
+      const uint4 tg = *reinterpret_cast<const uint4*>(grow + (ok ? ch : 0));
+      const uint4 to = *reinterpret_cast<const uint4*>(orow + (ok ? ch : 0));
+      float x[8], y[8];
+      M::unpack(ok ? tg : make_uint4(0u, 0u, 0u, 0u), x);
+      M::unpack(ok ? to : make_uint4(0u, 0u, 0u, 0u), y);
 #pragma unroll
-      for (int m = 0; m < NF; ++m) {
-        const int ch = 16 * m + 8 * hh;
-        const bool ok = live && ch < d;
-        uint4 tg = *reinterpret_cast<const uint4*>(grow + (ok ? ch : 0));
-        const uint4 to = *reinterpret_cast<const uint4*>(orow + (ok ? ch : 0));
-        if (!ok) tg = make_uint4(0u, 0u, 0u, 0u);
-        float x[8], y[8];
-        M::unpack(tg, x);
-        M::unpack(to, y);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) dot += ok ? x[e] * y[e] : 0.f;
-        gf[rt][m] = __builtin_bit_cast(Frag, tg);
+      for (int e = 0; e < 8; ++e) {
+        dot = __builtin_fmaf(x[e], y[e], dot);   // (a product of two bf16 numbers is exact)
+        x[e] *= rden;
       }
-      craw[rt] = dot + other_half(dot, hh);
-      if (live && hh == 0) cw[(int64_t)pos * cprep.stride] = craw[rt] * rden[rt];
+      gf[m] = __builtin_bit_cast(Frag, M::pack(x));
     }
+    c = (dot + other_half(dot, hh)) * rden;
+    if (live && hh == 0) cprep.head(head)[(int64_t)pos * cprep.stride] = c;
   }
   Reads<DP> rd;
   rd.init(l);
-  constexpr bool TIGHT = DP > 96;   // no registers for the start values: they are added afterwards
-  const f16v start = splat16(sq.h);
-  f16v gstart[RT];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) gstart[rt] = splat16(-craw[rt]);
+  // no registers for tiles of the start values: they are moved into the accumulators each time
+  constexpr bool TIGHT = DP > 96 || OCC == 4;
+  f16v start, gstart;
+  if constexpr (!TIGHT) {
+    start = splat16(a1);
+    gstart = splat16(-c);
+  }
 
-  f16v acc[RT][CB];
+  f16v acc[CB];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) acc[rt][cb] = kZero16;
+  for (int cb = 0; cb < CB; ++cb) acc[cb] = kZero16;
 
   constexpr int RA = OCC > 2 ? 0 : 2, CA = OCC > 2 ? 0 : 2;   // operand steps read ahead
-  auto weights = [&](const unsigned char* kl, const unsigned char* vl, int t32, f16v (&wt)[RT]) __attribute__((always_inline)) {
-    f16v sc[RT];
+  auto weights = [&](const unsigned char* kl, const unsigned char* vl, int t32, f16v& wt) __attribute__((always_inline)) {
+    f16v sc;
+    if constexpr (TIGHT) {
+      float a = a1, b = -c;
+      asm volatile("" : "+v"(a), "+v"(b));   // (or both tiles would be prepared before the loop and kept)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        sc[r] = a;
+        wt[r] = b;
+      }
+    }
     Frag ka[RA + 1], va[RA + 1];
     auto rows = [&](auto m) __attribute__((always_inline)) {
       constexpr int I = decltype(m)::value, X = I % (RA + 1);
@@ -517,29 +543,21 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_dq_kernel(
     prime<NF, RA>(rows);
     steps<NF, RA>(rows, [&](auto m) __attribute__((always_inline)) {
       constexpr int I = decltype(m)::value, X = I % (RA + 1);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        sc[rt] = M::mma(ka[X], qf[rt][I], I == 0 ? (TIGHT ? kZero16 : start) : sc[rt]);
-        wt[rt] = M::mma(va[X], gf[rt][I], I == 0 ? (TIGHT ? kZero16 : gstart[rt]) : wt[rt]);
-      }
+      sc = M::mma(ka[X], qf[I], I == 0 && !TIGHT ? start : sc);
+      wt = M::mma(va[X], gf[I], I == 0 && !TIGHT ? gstart : wt);
     });
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) wt[rt][r] = TIGHT ? (sc[rt][r] + sq.h) * (wt[rt][r] - craw[rt]) : sc[rt][r] * wt[rt][r];
+    for (int r = 0; r < 16; ++r) wt[r] = sc[r] * wt[r];
   };
   // (as in the forward kernel)
-  auto edge = [&](f16v (&wt)[RT], int rel, int left) __attribute__((always_inline)) {
+  auto edge = [&](f16v& wt, bool diagonal, int left) __attribute__((always_inline)) {
+    const int lane = fresh_lane(), lim = diagonal ? lane & 31 : 31;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int lim = masked ? (rel > 32 * rt ? -1 : rel == 32 * rt ? i : 31) : 31;
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (trow(r, hh) > lim || trow(r, hh) >= left) wt[rt][r] = 0.f;
-    }
+    for (int r = 0; r < 16; ++r)
+      if (trow(r, lane >> 5) > lim || trow(r, lane >> 5) >= left) wt[r] = 0.f;
   };
-  auto keys = [&](const unsigned char* kl, int t32, const f16v (&wt)[RT]) __attribute__((always_inline)) {
-    Frag kc[CA + 1], wa[RT];
+  auto keys = [&](const unsigned char* kl, int t32, const f16v& wt) __attribute__((always_inline)) {
+    Frag kc[CA + 1], wa;
     auto cols = [&](auto n) __attribute__((always_inline)) {
       constexpr int I = decltype(n)::value;
       kc[I % (CA + 1)] = rd.col(kl, t32, I / CB, I % CB);
@@ -547,31 +565,27 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_dq_kernel(
     prime<2 * CB, CA>(cols);
     steps<2 * CB, CA>(cols, [&](auto n) __attribute__((always_inline)) {
       constexpr int I = decltype(n)::value, F = I / CB, cb = I % CB;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        if constexpr (cb == 0) wa[rt] = M::template from_acc<F>(wt[rt]);
-        acc[rt][cb] = M::mma(kc[I % (CA + 1)], wa[rt], acc[rt][cb]);
-      }
+      if constexpr (cb == 0) wa = M::template from_acc<F>(wt);
+      acc[cb] = M::mma(wa, kc[I % (CA + 1)], acc[cb]);
     });
   };
 
   int buf = 0;
   auto next_stage = [&](int st) __attribute__((always_inline)) -> const unsigned char* {
-    if (PD > 1 && st + 1 < nst) stage_barrier<2 * C::NI>();
-    else stage_barrier<0>();
-    if (st + PD < nst) issue(st + PD, buf == 0 ? NBUF - 1 : buf - 1);
+    stage_barrier();
+    if (st + 1 < nst) issue(st + 1, buf ^ 1);
     const unsigned char* kl = tiles_smem + buf * STAGE;
-    buf = buf + 1 == NBUF ? 0 : buf + 1;
+    buf ^= 1;
     return kl;
   };
-  const int n_in = (masked && q00 < nk ? q00 : nk) / BN < nst ? (masked && q00 < nk ? q00 : nk) / BN : nst;
+  const int n_in = (masked && q0 < nk ? q0 : nk) / BN < nst ? (masked && q0 < nk ? q0 : nk) / BN : nst;
   int st = 0;
   for (; st < n_in; ++st) {
     const unsigned char* kl = next_stage(st);
     const unsigned char* vl = kl + G::TILE;
 #pragma unroll
     for (int t32 = 0; t32 < 2; ++t32) {
-      f16v wt[RT];
+      f16v wt;
       weights(kl, vl, t32, wt);
       keys(kl, t32, wt);
     }
@@ -582,98 +596,115 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_dq_kernel(
 #pragma unroll 1
     for (int t32 = 0; t32 < 2; ++t32) {
       const int kt = st * BN + t32 * 32;
-      if (kt >= nk || (masked && kt > q00 + 32 * (RT - 1))) continue;
+      if (kt >= nk || (masked && kt > q0)) continue;
       const int off = t32 * 32 * G::PITCH;
-      f16v wt[RT];
+      f16v wt;
       weights(kl + off, vl + off, 0, wt);
-      edge(wt, kt - q00, nk - kt);
+      edge(wt, masked && kt == q0, nk - kt);
       keys(kl + off, 0, wt);
     }
   }
 
-  // lanes = own queries, registers 4 j .. 4 j + 3 of a column block = channels 8 j + 4 hh ..
-  const HeadRows<bf16_t> Dh = DQ.head(head);
-  float rs = 0.f;
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int pos = q00 + rt * 32 + i;
-    if (pos < npos && pos >= Qh.lo) {
-      const float fac = 2.0f * sq.A * sq.t * kq * rden[rt];
-      const bf16_t* qrow = Qh.base + (unsigned)pos * Qh.pitch + 4 * hh;
-      bf16_t* row = Dh.base + (unsigned)pos * Dh.pitch + 4 * hh;
-      float qv[CB][4][4];
-      if (rpart) {   // (requested before the first store: no load waits behind one)
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) load4(qrow + (cb * 32 + 8 * j < d ? cb * 32 + 8 * j : 0), qv[cb][j]);
-      }
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (cb * 32 + 8 * j < d) {
-            float x[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              x[e] = acc[rt][cb][4 * j + e] * fac;
-              if (rpart) rs += x[e] * qv[cb][j][e];
-            }
-            *reinterpret_cast<uint2*>(row + cb * 32 + 8 * j) = pack_bf4u(x[0], x[1], x[2], x[3]);
-          }
-    }
-  }
+  // dq = qs ks acc (the keys went in unscaled); sum of dqh . qh = qs ks sum acc . q
+  __syncthreads();   // (the stages have been read)
+  static_assert(NW * 32 * G::PITCH <= 2 * STAGE, "a tile of rows for every wave");
+  float rs = store_rows<DP>(acc, kq, DQ.head(head), Qh, rpart != nullptr, q0, Qh.lo, npos, d, tiles_smem + w * 32 * G::PITCH);
   if (rpart) {
-    rs = dense::block_sum<NW>(rs, red, tid);
-    if (tid == 0) rpart[(int64_t)head * nb + bx] = rs;
+    const int t = w * 64 + fresh_lane();
+    rs = dense::block_sum<NW>(rs, red, t);
+    if (t == 0) rpart[(int64_t)head * nb + bx] = rs;
   }
 }
 
 // ---------------------------------------------------------------------------------------
 // dk and dv.  grid = (key/value heads, key blocks of 32 KW positions); the streamed rows are the queries at or after the
-// block's first key (all of them when unmasked) of every query head of the group in turn.  A block is KW x SW
-// waves: wave (x, y) owns key tile x and takes the query tiles y, y + SW, .. of every stage, so that the longest walk
-// -- the first keys of a long causal sequence, every query of every head -- is shared; at the end the SW parts are
-// added through LDS.  Four share stages of 128 rows, which with the own rows of two key tiles are all of a CU's LDS.
-// q and grad_out rows go to LDS as they are, 1 / den is a factor of the weights in fp32: one rounding less than grad_out / den
-// in bf16 (dk and dv 2.4e-3 of 64 bits, before 2.9e-3), and a stage's 32 more multiplications a wave replace about 50
-// instructions that divided and stored it (96 heads x 2048 x 64: 136 -> 132 us; 64 on 16 x 2049 x 128, SW = 2: 263 -> 232).
-// (1 / den and c both read behind the first contraction, P = g.v / den - c: 141 us instead of 132.)  A head's query scale is a factor of everything its walk adds to dk, so the accumulator is kept over the
-// scale of the head at hand.  rpart[kvhead * gridDim.y + block] = sum of dk . k.
+// block's first key (all of them when unmasked) of every query head of the group in turn.  q rows go to LDS as they are;
+// grad_out rows pass through registers and go there twice, times qs / den for the score side (so that W comes out times qs, the
+// factor of qh in dkh = sum W qh) and times 1 / den for dv, the operands that dense_dkdv_kernel forms.
+// Up to 64 channels a wave owns a key tile and both its sums.  Beyond, where one wave's accumulators and own rows take
+// all the registers a lone wave of a SIMD has and nothing hides its VALU work, two waves share a key tile: the one sums dk, the other
+// dv; of a stage's two query tiles each forms the weights of one, keeps those of its own sum and hands the others over through LDS.
+// rpart[kvhead * gridDim.y + block] = sum of dkh . kh, added up in dense_dkdv_kernel's order over blocks as wide.
 // ---------------------------------------------------------------------------------------
-template <int DP, int KW, int SW>
-struct DkDvLds {   // two buffers of a q and a g tile, their rows' scalars, the own rows; the parts of SW waves lie over all of it
-  static constexpr int ROWS = SW == 4 ? 128 : 64;   // streamed rows of a stage
-  static constexpr int TILE = ROWS * Geo<DP>::PITCH, SCALARS = 4 * TILE, OWN = SCALARS + 4 * ROWS * 4;
-  // (with 128 rows the first fragment of the own k rows has no place: it stays in registers)
-  static constexpr int KREG = SW == 4 ? 1 : 0, PARTS = SW == 4 ? 4 * KW * DP * 32 * 4 : SW == 2 ? 2 * KW * DP * 32 * 4 : 0;
-  static constexpr int END = OWN + (DP > 64 ? (2 * DP / 16 - KREG) * KW * 1024 : 0);
-  static constexpr size_t BYTES = END > PARTS ? END : PARTS;
+template <int DP>
+struct DkDv {
+  static constexpr bool PAIR = DP > 64;
+  static constexpr int KW = DP == 64 ? 8 : 4, NW = PAIR ? 2 * KW : KW;   // key tiles and waves of a block
+  static constexpr int BN = Geo<DP>::BN, TILE = Geo<DP>::TILE;
+  // two buffers each of q, qs g, g; then -qs c of the streamed rows, the weights handed over, the block sum
+  static constexpr int QG = 2 * TILE, GV = 4 * TILE, SCALARS = 6 * TILE, GIVE = SCALARS + 2 * BN * 4, RED = GIVE + (PAIR ? NW * 2048 : 0);
+  static constexpr size_t BYTES = RED + NW * 4;
   static_assert(BYTES <= 160 * 1024, "a CU's LDS");
 };
-template <int DP, int KW, int SW, int OCC>
-__global__ __launch_bounds__(64 * KW * SW, OCC) void tiles_dkdv_kernel(
+
+// One wave's share of a stage of grad_out rows on their way through registers (chunks as in Copy).
+template <int DP, int NW>
+struct Scaled {
+  using G = Geo<DP>;
+  using C = Copy<DP, NW>;
+  uint4 raw[C::NI];
+  float div[C::NI];
+  static __device__ __forceinline__ int chunk(int u, int w, int l) {   // (a wave without a u-th share loads what its first one does)
+    return (((C::has(u, w) ? u * NW + w : w) * 64 + l) % G::CPR ^ G::key(row(u, w, l))) * 8;
+  }
+  static __device__ __forceinline__ int row(int u, int w, int l) { return ((C::has(u, w) ? u * NW + w : w) * 64 + l) / G::CPR; }
+  __device__ __forceinline__ void load(const HeadRows<const bf16_t>& hr, int pos0, int end, int d, const float* den, unsigned stride, int w, int l) {
+#pragma unroll
+    for (int u = 0; u < C::NI; ++u) {
+      const int p = pos0 + row(u, w, l), c = chunk(u, w, l);
+      const unsigned ps = (unsigned)max(p < end ? p : end - 1, hr.lo);
+      raw[u] = *reinterpret_cast<const uint4*>(hr.base + (ps * hr.pitch + (unsigned)(c < d ? c : 0)));
+      div[u] = den[ps * stride];
+    }
+  }
+  // over den, times qs to the tile at qg, as it is to the tile at gv; zeros for rows outside [lo, end) and channels past d
+  __device__ __forceinline__ void store(unsigned char* qg, unsigned char* gv, float qs, int pos0, int lo, int end, int d, int w, int l) const {
+#pragma unroll
+    for (int u = 0; u < C::NI; ++u) {
+      if (!C::has(u, w)) continue;
+      const int p = pos0 + row(u, w, l);
+      // (as bits: a choice between the loaded registers and zero would become a branch)
+      const uint32_t keep = p >= lo && p < end && chunk(u, w, l) < d ? ~0u : 0u;
+      float x[8], y[8];
+      M::unpack(make_uint4(raw[u].x & keep, raw[u].y & keep, raw[u].z & keep, raw[u].w & keep), x);
+      const float inv = 1.0f / div[u], f = inv * qs;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        y[e] = x[e] * inv;
+        x[e] *= f;
+      }
+      const int at = ((u * NW + w) * 64 + l) * 16;
+      *reinterpret_cast<uint4*>(qg + at) = M::pack(x);
+      *reinterpret_cast<uint4*>(gv + at) = M::pack(y);
+    }
+  }
+};
+
+// waits for this wave's LDS accesses, then for the block; what is under way to registers or LDS from memory stays so
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int DP>
+__global__ __launch_bounds__(64 * DkDv<DP>::NW, 2) void tiles_dkdv_kernel(
     Rows<const bf16_t> K, Rows<const bf16_t> V, Rows<const bf16_t> Q, Rows<const bf16_t> GO, RowScalars den, RowScalars cvec,
     const float* __restrict__ qscale, const float* __restrict__ kscale, Rows<bf16_t> DK, Rows<bf16_t> DV,
-    float* __restrict__ rpart, int npos, int nk, int d, int masked, Square sq, int ratio) {
+    float* __restrict__ rpart, int npos, int nk, int d, int masked, float a0, float a1, float a2, int ratio) {
   using G = Geo<DP>;
-  using LD = DkDvLds<DP, KW, SW>;
-  constexpr int NW = KW * SW, NF = DP / 16, CB = DP / 32, BM = 32 * KW, BN = LD::ROWS, TILE = LD::TILE, KREG = LD::KREG;
-  static_assert(SW == 1 || SW == 2 || (SW == 4 && DP > 64), "a stage holds two or four query tiles");
+  using LD = DkDv<DP>;
+  constexpr bool PAIR = LD::PAIR;
+  constexpr int KW = LD::KW, NW = LD::NW, NF = DP / 16, CB = DP / 32, BM = 32 * KW, BN = LD::BN, TILE = LD::TILE, NS = PAIR ? 1 : 2;
+  static_assert(BN == 64, "a stage is two query tiles");
   using C = Copy<DP, NW>;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_smem[];   // [2][q tile, g tile], [2][-go.o, 1 / den][BN], own rows
-  unsigned char* Ql = tiles_smem;
-  unsigned char* Gl = tiles_smem + TILE;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tiles_smem[];
   float* Cl = reinterpret_cast<float*>(tiles_smem + LD::SCALARS);
+  float* red = reinterpret_cast<float*>(tiles_smem + LD::RED);
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, i = l & 31, hh = l >> 5;
-  const int kw = w % KW, sw = w / KW;
+  const int kw = w % KW, side = w / KW;   // side (of a pair): 0 sums dk, 1 sums dv
   const int nb = gridDim.y, bx = blockIdx.y;
   const int hkv = blockIdx.x;
   const int tok0 = bx * BM;   // (under the mask the first key blocks see the most queries: already first)
   const int k00 = tok0 + kw * 32;
   const HeadRows<const bf16_t> Kh = K.head(hkv), Vh = V.head(hkv);
-  const HeadRows<bf16_t> DKh = DK.head(hkv), DVh = DV.head(hkv);   // (here: the strides need not be kept)
   const float ks = kscale[hkv];
   const int lo = Q.lo;
   const int nst = (npos + BN - 1) / BN;
@@ -681,95 +712,55 @@ __global__ __launch_bounds__(64 * KW * SW, OCC) void tiles_dkdv_kernel(
   const uint32_t lds0 = lds_address(tiles_smem);
 
   // the loading side runs one stage ahead of the computing one, across heads
-  HeadRows<const bf16_t> Qh, Gh;
-  const float *denh, *ch;
-  C cq, cg;
-  float dreg = 1.0f, creg = 0.f, lon = qscale[hkv * ratio] == 0.f ? 0.f : 1.0f;
-  Qh = Q.head(hkv * ratio);
-  Gh = GO.head(hkv * ratio);
-  denh = den.head(hkv * ratio);
-  ch = cvec.head(hkv * ratio);
+  HeadRows<const bf16_t> Qh = Q.head(hkv * ratio), Gh = GO.head(hkv * ratio);
+  const float *denh = den.head(hkv * ratio), *ch = cvec.head(hkv * ratio);
   const int64_t qstep = Q.step(), gstep = GO.step();   // (the heads of a group are equally far apart)
+  float lqs = qscale[hkv * ratio];
+  C cq;
+  cq.init(w, l, d, Qh.pitch);
+  Scaled<DP, NW> sg;
+  float creg = 0.f;
   auto stage_load = [&](int st, int buf) __attribute__((always_inline)) {
-    if (w < BN / 64) {
-      const int pos = st * BN + tid, ps = max(pos < npos ? pos : npos - 1, lo);
-      dreg = denh[(unsigned)ps * (unsigned)den.stride];
-      creg = ch[(unsigned)ps * (unsigned)cvec.stride];
+    sg.load(Gh, st * BN, npos, d, denh, (unsigned)den.stride, w, l);
+    if (w == 0) {
+      const int pos = st * BN + l;
+      creg = ch[(unsigned)max(pos < npos ? pos : npos - 1, lo) * (unsigned)cvec.stride];
     }
-#pragma unroll
-    for (int g = 0; g < BN / G::BN; ++g) {
-      cq.issue(Qh, st * BN + g * G::BN, npos, d, lds0 + buf * 2 * TILE + g * G::TILE, w, l);
-      cg.issue(Gh, st * BN + g * G::BN, npos, d, lds0 + (buf * 2 + 1) * TILE + g * G::TILE, w, l);
-    }
+    cq.issue(Qh, st * BN, npos, d, lds0 + buf * TILE, w, l);
   };
-  // (rows outside the range count for nothing: both scalars zero)
   auto stage_store = [&](int st, int buf) __attribute__((always_inline)) {
-    if (w < BN / 64) {
-      const int pos = st * BN + tid;
-      const bool in = pos >= lo && pos < npos;
-      float* s = Cl + buf * 2 * BN + tid;
-      s[0] = in && creg != 0.f ? -creg * dreg * lon : 0.f;   // (c = go.o / den, which is 0 where den has overflowed)
-      s[BN] = in ? __builtin_amdgcn_rcpf(dreg) : 0.f;   // (one unit in the last place of 24 bits, on its way to 8)
+    sg.store(tiles_smem + LD::QG + buf * TILE, tiles_smem + LD::GV + buf * TILE, lqs, st * BN, lo, npos, d, w, l);
+    if (w == 0) {
+      const int pos = st * BN + l;
+      Cl[buf * BN + l] = -creg * lqs * ((pos >= lo && pos < npos) ? 1.0f : 0.f);   // (-qs c: the tile's start value)
     }
   };
 
   Reads<DP> rd;   // (at the buffer being read)
   rd.init(l);
-  if (SW > 1) rd.shift(sw * 32 * G::PITCH);
   rd.pin();
-  // own rows: in registers up to 64 channels; beyond, where the accumulators take half of them, in LDS
-  constexpr bool VLDS = DP > 64;
-  Frag* Vl = reinterpret_cast<Frag*>(tiles_smem + LD::OWN) + kw * NF * 64 + l;
-  Frag* Kl = Vl + (KW * NF - kw * KREG - KREG) * 64;   // (at fragment 0, held or not)
   Frag kf[NF], vf[NF];
-  auto own_to_lds = [&](const HeadRows<const bf16_t>& hr, float scale, Frag* dst, auto from) __attribute__((always_inline)) {
-    uint32_t off = (unsigned)(k00 + i < nk ? k00 + i : nk - 1) * hr.pitch;
-    asm volatile("" : "+v"(off));
-#pragma unroll 2
-    for (int m = decltype(from)::value; m < NF; ++m) {
-      const int ch = 16 * m + 8 * hh;
-      const uint4 t = *reinterpret_cast<const uint4*>(hr.base + (off + (unsigned)(ch < d ? ch : 0)));
-      float x[8];
-      M::unpack(t, x);
-      const bool ok = k00 + i < nk && ch < d;
+  f16v acc[NS][CB];   // dk and dv, or the one this wave sums
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = ok ? x[e] * scale : 0.f;
-      dst[m * 64] = __builtin_bit_cast(Frag, M::pack(x));
-    }
-  };
-  auto own_first = [&]() __attribute__((always_inline)) {
-    const bool ok = k00 + i < nk;
-    const uint4 t = *reinterpret_cast<const uint4*>(Kh.base + ((unsigned)(ok ? k00 + i : nk - 1) * Kh.pitch + 8u * hh));
-    return __builtin_bit_cast(Frag, ok ? t : make_uint4(0u, 0u, 0u, 0u));
-  };
-  f16v dk[CB], dv[CB];
+  for (int s = 0; s < NS; ++s)
 #pragma unroll
-  for (int cb = 0; cb < CB; ++cb) dk[cb] = dv[cb] = kZero16;
-  const f16v start = splat16(sq.h);
-  float T = 0.f;   // this head's scale
+    for (int cb = 0; cb < CB; ++cb) acc[s][cb] = kZero16;
+  if (st0 < nst) stage_load(st0, 0);
+  own_row<DP>(Vh, k00 + i, nk, d, hh, 1.0f, vf);
+  __builtin_amdgcn_sched_barrier(0);   // (one row after the other: registers)
+  own_row<DP>(Kh, k00 + i, nk, d, hh, ks, kf);
+  if (st0 < nst) stage_store(st0, 0);
 
-  cq.init(w, l, d, Qh.pitch);
-  cg.init(w, l, d, Gh.pitch);
-  if constexpr (KREG) kf[0] = own_first();
-  if (st0 < nst) {
-    stage_load(st0, 0);
-    stage_store(st0, 0);
-  }
-  // One 32-query tile against the wave's own keys.  diag: the tile's queries before row `first` (the lane's own key when
-  // they are the same positions) lie before the key and do not see it.
-  auto tile = [&](int t, const float* cl, auto diag, int first) __attribute__((always_inline)) {
-    const unsigned char* qt = Ql + t * 32 * G::PITCH;
-    const unsigned char* gt = Gl + t * 32 * G::PITCH;
-    // rows = queries, lanes = own keys: u and den P = g . v - g . o
-    f16v sc, pt;
-    constexpr int RA = VLDS ? 1 : 2, CA = VLDS ? 1 : 2;   // operand steps read ahead
-    Frag qa[RA + 1], ga[RA + 1], ka[RA + 1], va[RA + 1];
+  float c2, c1, b2;   // f and f' of s = qs sr, where sr = q . kh is what the score tile holds
+  // The weights of query tile t: f(s) in sc, qs f'(s) (g . v - c) in pt; rows = queries, lanes = own keys.
+  auto scores = [&](int t, const float* cl, f16v& sc, f16v& pt) __attribute__((always_inline)) {
+    constexpr int RA = PAIR ? 1 : 2;   // operand steps read ahead
+    const unsigned char *qt = tiles_smem, *gt = tiles_smem + LD::QG;
+    Frag qa[RA + 1], ga[RA + 1];
     auto rows = [&](auto m) __attribute__((always_inline)) {
       constexpr int I = decltype(m)::value, X = I % (RA + 1);
-      qa[X] = rd.row(qt, 0, I);
-      if constexpr (VLDS && I >= KREG) ka[X] = Kl[I * 64];
-      ga[X] = rd.row(gt, 0, I);
-      if constexpr (VLDS) va[X] = Vl[I * 64];
+      qa[X] = rd.row(qt + t * 32 * G::PITCH, 0, I);
+      ga[X] = rd.row(gt + t * 32 * G::PITCH, 0, I);
     };
     prime<NF, RA>(rows);
 #pragma unroll
@@ -779,79 +770,32 @@ __global__ __launch_bounds__(64 * KW * SW, OCC) void tiles_dkdv_kernel(
     }
     steps<NF, RA>(rows, [&](auto m) __attribute__((always_inline)) {
       constexpr int I = decltype(m)::value, X = I % (RA + 1);
-      sc = M::mma(qa[X], VLDS && I >= KREG ? ka[X] : kf[I], I == 0 ? (VLDS ? kZero16 : start) : sc);
-      pt = M::mma(ga[X], VLDS ? va[X] : vf[I], pt);
+      sc = M::mma(qa[X], kf[I], I == 0 ? kZero16 : sc);
+      pt = M::mma(ga[X], vf[I], pt);
     });
-    Frag gc[CA + 1], qc[CA + 1];
-    auto cols = [&](auto n) __attribute__((always_inline)) {
-      constexpr int I = decltype(n)::value, X = I % (CA + 1);
-      gc[X] = rd.col(gt, 0, I / CB, I % CB);
-      qc[X] = rd.col(qt, 0, I / CB, I % CB);
-    };
-    prime<2 * CB, CA>(cols);
+  };
+  // diag: the tile's queries before row `first` (the lane's own key when they are the same positions) do not see the key
+  auto polynomial = [&](f16v& sc, f16v& pt, auto diag, int first) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float4 r4 = *reinterpret_cast<const float4*>(cl + BN + 8 * j + 4 * hh);
-      const float rden[4] = {r4.x, r4.y, r4.z, r4.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = 4 * j + e;
-        const float u = VLDS ? sc[r] * T + sq.h : sc[r];   // (own k rows in LDS are not scaled: no registers for a start value either)
-        sc[r] = (u * u + sq.c) * rden[e];
-        pt[r] = u * (pt[r] * rden[e]);
-      }
+    for (int r = 0; r < 16; ++r) {
+      const float s = sc[r];
+      sc[r] = a0 + s * (c1 + c2 * s);
+      pt[r] = (a1 + b2 * s) * pt[r];
     }
     if constexpr (decltype(diag)::value) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (trow(r, hh) < first) sc[r] = pt[r] = 0.f;
     }
-    Frag fa, wa;
-    steps<2 * CB, CA>(cols, [&](auto n) __attribute__((always_inline)) {
-      constexpr int I = decltype(n)::value, X = I % (CA + 1), F = I / CB, cb = I % CB;
-      if constexpr (cb == 0) {
-        fa = M::template from_acc<F>(sc);
-        wa = M::template from_acc<F>(pt);
-      }
-      dv[cb] = M::mma(gc[X], fa, dv[cb]);
-      dk[cb] = M::mma(qc[X], wa, dk[cb]);
-    });
   };
 
-  float qs_at = 1.0f, was_on = 1.0f;   // dk holds its sum over qs_at
   int buf = 0;
   for (int hq = 0; hq < ratio; ++hq) {
     const float qs = qscale[hkv * ratio + hq];
-    // (a scale of zero: nothing of this head reaches dk, whose sum stays over the scale before)
-    const float on = qs == 0.f ? 0.f : 1.0f;
-    if constexpr (!VLDS) {
-      if (hq == 0 || on != was_on) own_row<DP>(Vh, k00 + i, nk, d, hh, on, vf);
-      __builtin_amdgcn_sched_barrier(0);   // (one row after the other: registers)
-      own_row<DP>(Kh, k00 + i, nk, d, hh, ks * qs * sq.t, kf);
-    } else {
-      T = ks * qs * sq.t;
-      if (hq == 0 || on != was_on) {
-        if (hq > 0) __syncthreads();   // (the other waves of this key tile are through with the head before)
-        if (sw == 0) {
-          if (hq == 0) own_to_lds(Kh, 1.0f, Kl, std::integral_constant<int, KREG>{});
-          own_to_lds(Vh, on, Vl, std::integral_constant<int, 0>{});
-        }
-      }
-    }
-    was_on = on;
-    if (on != 0.f) {
-      if (hq > 0) {
-        const float fac = qs_at / qs;
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) dk[cb][r] *= fac;
-      }
-      qs_at = qs;
-    }
+    c2 = a2 * qs * qs; c1 = a1 * qs; b2 = 2.0f * a2 * qs;
     // one stage, from buffer buf, while the next one (of this head or the next) is on its way to the other
     auto stage = [&](auto edge, int st) __attribute__((always_inline)) {
-      stage_barrier<0>();
+      stage_barrier();
       const bool more = st + 1 < nst || hq + 1 < ratio;
       const int next = st + 1 < nst ? st + 1 : st0;
       if (more) {
@@ -860,19 +804,82 @@ __global__ __launch_bounds__(64 * KW * SW, OCC) void tiles_dkdv_kernel(
           Gh.base += gstep;
           denh += den.hs;
           ch += cvec.hs;
-          lon = qscale[hkv * ratio + hq + 1] == 0.f ? 0.f : 1.0f;
+          lqs = qscale[hkv * ratio + hq + 1];
         }
         stage_load(next, buf ^ 1);
       }
+      const float* cl = Cl + buf * BN;
+      // (tiles past the end, or before every own key, count for nothing)
+      auto live = [&](int t) { const int qb = st * BN + t * 32; return qb < npos && !(decltype(edge)::value && qb < k00); };
+      auto first = [&](int t) { return st * BN + t * 32 == k00 ? i : 0; };
+      constexpr int CA = 2;   // operand steps read ahead
+      if constexpr (!PAIR) {
 #pragma unroll
-      for (int t = 0; t < BN / 32 / SW; ++t) {
-        const int t32 = SW > 1 ? sw : t, qb = st * BN + t32 * 32;
-        if (qb >= npos || (decltype(edge)::value && qb < k00)) continue;   // past the end, or before every own key
+        for (int t = 0; t < 2; ++t) {
+          if (!live(t)) continue;
+          __builtin_amdgcn_sched_barrier(0);
+          f16v sc, pt;
+          scores(t, cl + t * 32, sc, pt);
+          Frag gc[CA + 1], qc[CA + 1];
+          auto cols = [&](auto n) __attribute__((always_inline)) {
+            constexpr int I = decltype(n)::value, X = I % (CA + 1);
+            gc[X] = rd.col(tiles_smem + LD::GV, t, I / CB, I % CB);
+            qc[X] = rd.col(tiles_smem, t, I / CB, I % CB);
+          };
+          prime<2 * CB, CA>(cols);
+          polynomial(sc, pt, edge, first(t));
+          Frag fa, wa;
+          steps<2 * CB, CA>(cols, [&](auto n) __attribute__((always_inline)) {
+            constexpr int I = decltype(n)::value, X = I % (CA + 1), F = I / CB, cb = I % CB;
+            if constexpr (cb == 0) {
+              fa = M::template from_acc<F>(sc);
+              wa = M::template from_acc<F>(pt);
+            }
+            acc[1][cb] = M::mma(fa, gc[X], acc[1][cb]);
+            acc[0][cb] = M::mma(wa, qc[X], acc[0][cb]);
+          });
+        }
+      } else {
+        Frag* give = reinterpret_cast<Frag*>(tiles_smem + LD::GIVE);
+        const unsigned char* mine = tiles_smem + (side ? LD::GV : 0);   // the streamed rows of this wave's sum
+        Frag keep[2] = {M::zero(), M::zero()};
         __builtin_amdgcn_sched_barrier(0);
-        tile(t, Cl + buf * 2 * BN + t32 * 32, edge, qb == k00 ? i : 0);
+        if (live(side)) {
+          f16v sc, pt;
+          scores(side, cl + side * 32, sc, pt);
+          polynomial(sc, pt, edge, first(side));
+          const Frag f0 = M::template from_acc<0>(sc), f1 = M::template from_acc<1>(sc);
+          const Frag w0 = M::template from_acc<0>(pt), w1 = M::template from_acc<1>(pt);
+          keep[0] = side ? f0 : w0;
+          keep[1] = side ? f1 : w1;
+          give[w * 128 + l] = side ? w0 : f0;
+          give[w * 128 + 64 + l] = side ? w1 : f1;
+        }
+        lds_barrier();
+        const Frag* got = give + ((1 - side) * KW + kw) * 128 + l;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          if (!live(t)) continue;
+          Frag a[2], xc[CA + 1];
+          a[0] = got[0];
+          a[1] = got[64];
+          auto cols = [&](auto n) __attribute__((always_inline)) {
+            constexpr int I = decltype(n)::value;
+            xc[I % (CA + 1)] = rd.col(mine, t, I / CB, I % CB);
+          };
+          prime<2 * CB, CA>(cols);
+          if (t == side) {
+            a[0] = keep[0];
+            a[1] = keep[1];
+          }
+          steps<2 * CB, CA>(cols, [&](auto n) __attribute__((always_inline)) {
+            constexpr int I = decltype(n)::value, F = I / CB, cb = I % CB;
+            acc[0][cb] = M::mma(a[F], xc[I % (CA + 1)], acc[0][cb]);
+          });
+        }
       }
       if (more) stage_store(next, buf ^ 1);
-      rd.shift(buf ? -2 * TILE : 2 * TILE);
+      rd.shift(buf ? -TILE : TILE);
       buf ^= 1;
     };
     // stages with queries that lie before an own key or at the same position; then those wholly after (every wave passes
@@ -882,87 +889,15 @@ __global__ __launch_bounds__(64 * KW * SW, OCC) void tiles_dkdv_kernel(
     for (; st < nst; ++st) stage(std::false_type{}, st);
   }
 
-  // the parts of the SW waves: the last two give theirs to the first two; of these the first finish dk, the second dv
-  if constexpr (SW > 1) {
-    float4* part = reinterpret_cast<float4*>(tiles_smem) + (size_t)kw * (CB * 4 * 64) + l;
-    float4* part2 = part + (size_t)KW * (CB * 4 * 64);
-    auto leave = [&](float4* p, const f16v (&a)[CB]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) p[(cb * 4 + j) * 64] = make_float4(a[cb][4 * j], a[cb][4 * j + 1], a[cb][4 * j + 2], a[cb][4 * j + 3]);
-    };
-    auto take = [&](const float4* p, f16v (&a)[CB]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float4 t = p[(cb * 4 + j) * 64];
-          a[cb][4 * j] += t.x; a[cb][4 * j + 1] += t.y; a[cb][4 * j + 2] += t.z; a[cb][4 * j + 3] += t.w;
-        }
-    };
-    __syncthreads();
-    if constexpr (SW == 4) {
-      constexpr size_t HALF = (size_t)2 * KW * (CB * 4 * 64);   // (sw = 0 and 2, sw = 1 and 3)
-      if (sw >= 2) {
-        leave(part + (sw - 2) * HALF, dk);
-        leave(part2 + (sw - 2) * HALF, dv);
-      }
-      __syncthreads();
-      if (sw < 2) {
-        take(part + sw * HALF, dk);
-        take(part2 + sw * HALF, dv);
-      }
-      __syncthreads();
-    }
-    if (sw == 1) leave(part, dk);
-    else if (sw == 0) leave(part2, dv);
-    __syncthreads();
-    if (sw == 1) take(part2, dv);
-    else if (sw == 0) take(part, dk);
-  }
-  // lanes = own keys, registers 4 j .. 4 j + 3 of a column block = channels 8 j + 4 hh ..
-  int lane = tid;
-  asm volatile("" : "+v"(lane));   // (nothing below is prepared before the loops and kept through them)
-  const int pos = k00 + (lane & 31);
+  // dk = ks dkh (dkh = the accumulated sum); sum of dkh . kh = ks sum acc . k
+  __syncthreads();   // (the stages have been read)
+  static_assert(NW * 32 * G::PITCH <= LD::SCALARS, "a tile of rows for every wave");
   float rs = 0.f;
-  if (pos < nk && sw == 0) {
-    const float fac = 2.0f * sq.A * sq.t * ks * qs_at;
-    const bf16_t* krow = Kh.base + (unsigned)pos * Kh.pitch + 4 * hh;
-    bf16_t* row = DKh.base + (unsigned)pos * DKh.pitch + 4 * hh;
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      float kv[4][4];
-      if (rpart) {   // (requested before the block's first store)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) load4(krow + (cb * 32 + 8 * j < d ? cb * 32 + 8 * j : 0), kv[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (cb * 32 + 8 * j < d) {
-          float x[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            x[e] = dk[cb][4 * j + e] * fac;
-            if (rpart) rs += x[e] * kv[j][e];
-          }
-          *reinterpret_cast<uint2*>(row + cb * 32 + 8 * j) = pack_bf4u(x[0], x[1], x[2], x[3]);
-        }
-    }
-  }
-  if (pos < nk && sw == (SW > 1 ? 1 : 0)) {
-    bf16_t* row = DVh.base + (unsigned)pos * DVh.pitch + 4 * hh;
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (cb * 32 + 8 * j < d)
-          *reinterpret_cast<uint2*>(row + cb * 32 + 8 * j) =
-              pack_bf4u(dv[cb][4 * j] * sq.A, dv[cb][4 * j + 1] * sq.A, dv[cb][4 * j + 2] * sq.A, dv[cb][4 * j + 3] * sq.A);
-  }
+  unsigned char* own = tiles_smem + w * 32 * G::PITCH;
+  if (side == 0) rs = store_rows<DP>(acc[0], ks, DK.head(hkv), Kh, rpart != nullptr, k00, 0, nk, d, own);
+  if (!PAIR || side == 1) store_rows<DP>(acc[NS - 1], 1.0f, DV.head(hkv), Kh, false, k00, 0, nk, d, own);
   if (rpart) {
-    __syncthreads();   // (the parts were just read)
-    rs = dense::block_sum<NW>(rs, Cl, tid);
+    rs = dense::block_sum<NW>(rs, red, tid);
     if (tid == 0) rpart[(int64_t)hkv * nb + bx] = rs;
   }
 }
