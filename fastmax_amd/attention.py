@@ -31,17 +31,12 @@ from . import _cabi, _ext
 
 # fraction of the free device memory the saved prefix states of one call may take
 SAVE_STATES_MEMORY_FRACTION = 0.25
-# States up to this size are kept without asking how much is free (the question costs a call of 6 us, a tenth of what the
-# kernels of a small call take): less than one of the 20 MB pieces the allocator takes device memory in.
-SAVE_STATES_SMALL = 8 << 20
 
 
 def _states_fit(q3: torch.Tensor, k3: torch.Tensor, mask: bool, p: int) -> bool:
     """True when the prefix states of this call (the library's own figure: one state per key/value
     head per chunk or token split) take less than SAVE_STATES_MEMORY_FRACTION of the free memory."""
     need = _ext.load().saved_state_bytes(q3, k3, bool(mask), int(p))
-    if need <= SAVE_STATES_SMALL and SAVE_STATES_MEMORY_FRACTION > 0:
-        return True
     free, _ = torch.cuda.mem_get_info(k3.device)
     return need <= SAVE_STATES_MEMORY_FRACTION * free
 
@@ -49,8 +44,6 @@ def _states_fit(q3: torch.Tensor, k3: torch.Tensor, mask: bool, p: int) -> bool:
 def _states_fit_bytes(ext, q5: torch.Tensor, k4: torch.Tensor, mask: bool, p: int) -> bool:
     """The same test for strided (B, G, R, T, D) / (B, G, T, D) views."""
     need = ext.saved_state_bytes_strided(q5, k4, bool(mask), int(p))
-    if need <= SAVE_STATES_SMALL and SAVE_STATES_MEMORY_FRACTION > 0:
-        return True
     free, _ = torch.cuda.mem_get_info(k4.device)
     return need <= SAVE_STATES_MEMORY_FRACTION * free
 
