@@ -16,8 +16,8 @@
 //     the row is XORed with a function of the row number, so that row reads and transposing reads both touch every bank once.
 //   * LDS reads run a few steps ahead of the matrix instructions that use them, in an order the compiler is not left to
 //     choose (see steps).
-//   * rows leave in 8-byte pieces from the forward kernel, whose second contraction is formed transposed (channels x own
-//     rows); in the backward kernels, where the order of a sum over the outputs is that of lanes = channels, through LDS.
+//   * the forward kernel forms its second contraction transposed (channels x own rows), so that rows leave in 8-byte pieces; the
+//     backward kernels do not: the order of a sum over their outputs is that of lanes = channels.
 // What is left: the waits between a wave's phases (scores, polynomial, second contraction), which two to four waves a
 // SIMD hide in part, and 4 to 9 VALU instructions a matrix instruction.  LDS delivers 256 bytes a cycle (an operand read takes a CU 4.1
 // cycles) and is a quarter busy.  Without gain: one tile's polynomial placed between the next tile's matrix instructions
@@ -173,64 +173,56 @@ __device__ __forceinline__ uint32_t lds_address(const unsigned char* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
 }
 
+// Element c of row pos: uniform base, 32-bit lane offset in bytes (a head spans less than 4 GiB).
+template <class T>
+__device__ __forceinline__ T* element(const HeadRows<T>& hr, int pos, int c) {
+  using Byte = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+  return reinterpret_cast<T*>(reinterpret_cast<Byte*>(hr.base) + ((unsigned)pos * hr.pitch + (unsigned)c) * 2u);
+}
+
 // 32 rows of a sum in accumulators (registers = rows r0 + trow, lanes = channels), times `scale`, to the rows inside
 // [lo, end); `dot`: also this lane's part of their inner product with the rows of x, over rows and then channels as the
-// fm_dense.h kernels take them.  Rows pass through LDS (32 rows of this wave's own): the accumulators' layout has a lane hold two
-// bytes of a row, and loads and stores of two bytes keep the address unit busy 16 cycles each (a block of eight waves x 64 channels: 2 us
-// for x and 4 to 6 for dk and dv, with nothing beside them).
+// fm_dense.h kernels take them.  All of x is requested at once and used before the first store: no load waits behind a store or on
+// its own.  A block's epilogue is a tenth of a causal pass at 2048 tokens and bound by its instructions, so whole tiles go
+// without tests (dk and dv of 256 rows x 64 channels with one stage of queries: 14.6 us a block with a test an element here and a
+// select an element in own_row, 11.5 without; rows passed through LDS for 16-byte accesses: 12.4).
 template <int DP>
 __device__ __forceinline__ float store_rows(const f16v (&acc)[DP / 32], float scale, const HeadRows<bf16_t>& out, const HeadRows<const bf16_t>& x,
-                                            bool dot, int r0, int lo, int end, int d, unsigned char* lds) {
-  using G = Geo<DP>;
-  constexpr int CB = DP / 32, CPR = G::CPR, N = CPR / 2, SH = CPR % 8 == 0 ? 2 : 1;
+                                            bool dot, int r0, int lo, int end, int d) {
+  constexpr int CB = DP / 32;
   const int lane = fresh_lane(), c0 = lane & 31, hh = lane >> 5;
-  // chunk c of row r is kept at chunk c ^ (r / 4 % 2 << SH): the two halves of a wave, four rows apart, use different banks
-  auto at = [&](int row, int chunk) { return lds + row * G::PITCH + ((chunk ^ ((row >> 2 & 1) << SH)) << 4); };
-  // channel cb * 32 + c0 of row trow(r, hh): one address a lane for even cb, one for odd, constants on top
-  unsigned char* const even = lds + 4 * hh * G::PITCH + (((c0 >> 3) ^ (hh << SH)) << 4) + (c0 & 7) * 2;
-  unsigned char* const odd = SH == 2 ? lds + 4 * hh * G::PITCH + (((4 + (c0 >> 3)) ^ (hh << SH)) << 4) + (c0 & 7) * 2 : even + 64;
-  auto elt = [&](int r, int cb) { return reinterpret_cast<uint16_t*>((cb & 1 ? odd : even) + (cb >> 1) * 128 + (8 * (r >> 2) + (r & 3)) * G::PITCH); };
-  const bool whole = r0 >= lo && r0 + 32 <= end && d == DP;   // (uniform)
   float rs = 0.f;
-  if (dot) {
-    uint4 t[N];
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-      const int row = (u * 64 + lane) / CPR, ch = (u * 64 + lane) % CPR * 8, pos = r0 + row;
-      t[u] = *reinterpret_cast<const uint4*>(x.base + ((unsigned)max(pos < end ? pos : end - 1, lo) * x.pitch + (unsigned)(ch < d ? ch : 0)));
-    }
-#pragma unroll
-    for (int u = 0; u < N; ++u) *reinterpret_cast<uint4*>(at((u * 64 + lane) / CPR, (u * 64 + lane) % CPR)) = t[u];
-    asm volatile("" ::: "memory");   // (a wave's LDS accesses are carried out in their order)
-    auto term = [&](int r, int cb) { return __builtin_fmaf(acc[cb][r] * scale, dense::to_f32_elt(*elt(r, cb)), rs); };
-    if (whole) {
+  auto run = [&](auto whole) __attribute__((always_inline)) {
+    constexpr bool W = decltype(whole)::value;   // every row and channel exists
+    auto in = [&](int r, int cb) { return W || (r0 + trow(r, hh) >= lo && r0 + trow(r, hh) < end && cb * 32 + c0 < d); };
+    if (dot) {
+      float xv[16][CB];
 #pragma unroll
       for (int r = 0; r < 16; ++r)
 #pragma unroll
-        for (int cb = 0; cb < CB; ++cb) rs = term(r, cb);
-    } else {
-      FM_KEEP_BRANCH();
+        for (int cb = 0; cb < CB; ++cb) {   // (clamped, not predicated)
+          const int pos = r0 + trow(r, hh), c = cb * 32 + c0;
+          xv[r][cb] = to_f32(*element(x, W ? pos : max(pos < end ? pos : end - 1, lo), W || c < d ? c : 0));
+        }
 #pragma unroll
       for (int r = 0; r < 16; ++r)
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
-          const int pos = r0 + trow(r, hh);
-          const float t1 = term(r, cb);
-          rs = pos >= lo && pos < end && cb * 32 + c0 < d ? t1 : rs;
+          const float t = __builtin_fmaf(acc[cb][r] * scale, xv[r][cb], rs);
+          rs = in(r, cb) ? t : rs;
         }
     }
-    asm volatile("" ::: "memory");
-  }
 #pragma unroll
-  for (int r = 0; r < 16; ++r)
+    for (int r = 0; r < 16; ++r)
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) *elt(r, cb) = M::to_elt(acc[cb][r] * scale);
-  asm volatile("" ::: "memory");
-#pragma unroll
-  for (int u = 0; u < N; ++u) {
-    const int row = (u * 64 + lane) / CPR, chunk = (u * 64 + lane) % CPR, pos = r0 + row;
-    if (pos >= lo && pos < end && chunk * 8 < d)
-      *reinterpret_cast<uint4*>(out.base + ((unsigned)pos * out.pitch + (unsigned)(chunk * 8))) = *reinterpret_cast<const uint4*>(at(row, chunk));
+      for (int cb = 0; cb < CB; ++cb)
+        if (in(r, cb)) *element(out, r0 + trow(r, hh), cb * 32 + c0) = bf16_t{M::to_elt(acc[cb][r] * scale)};
+  };
+  if (r0 >= lo && r0 + 32 <= end && d == DP) {   // (uniform)
+    run(std::true_type{});
+  } else {
+    FM_KEEP_BRANCH();
+    run(std::false_type{});
   }
   return rs;
 }
@@ -606,9 +598,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_dq_kernel(
   }
 
   // dq = qs ks acc (the keys went in unscaled); sum of dqh . qh = qs ks sum acc . q
-  __syncthreads();   // (the stages have been read)
-  static_assert(NW * 32 * G::PITCH <= 2 * STAGE, "a tile of rows for every wave");
-  float rs = store_rows<DP>(acc, kq, DQ.head(head), Qh, rpart != nullptr, q0, Qh.lo, npos, d, tiles_smem + w * 32 * G::PITCH);
+  float rs = store_rows<DP>(acc, kq, DQ.head(head), Qh, rpart != nullptr, q0, Qh.lo, npos, d);
   if (rpart) {
     const int t = w * 64 + fresh_lane();
     rs = dense::block_sum<NW>(rs, red, t);
@@ -890,12 +880,9 @@ __global__ __launch_bounds__(64 * DkDv<DP>::NW, 2) void tiles_dkdv_kernel(
   }
 
   // dk = ks dkh (dkh = the accumulated sum); sum of dkh . kh = ks sum acc . k
-  __syncthreads();   // (the stages have been read)
-  static_assert(NW * 32 * G::PITCH <= LD::SCALARS, "a tile of rows for every wave");
   float rs = 0.f;
-  unsigned char* own = tiles_smem + w * 32 * G::PITCH;
-  if (side == 0) rs = store_rows<DP>(acc[0], ks, DK.head(hkv), Kh, rpart != nullptr, k00, 0, nk, d, own);
-  if (!PAIR || side == 1) store_rows<DP>(acc[NS - 1], 1.0f, DV.head(hkv), Kh, false, k00, 0, nk, d, own);
+  if (side == 0) rs = store_rows<DP>(acc[0], ks, DK.head(hkv), Kh, rpart != nullptr, k00, 0, nk, d);
+  if (!PAIR || side == 1) store_rows<DP>(acc[NS - 1], 1.0f, DV.head(hkv), Kh, false, k00, 0, nk, d);
   if (rpart) {
     rs = dense::block_sum<NW>(rs, red, tid);
     if (tid == 0) rpart[(int64_t)hkv * nb + bx] = rs;

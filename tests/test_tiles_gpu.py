@@ -1,6 +1,6 @@
 """The bf16 score-tile kernels at p = 2 (fastmax_amd/csrc/fm_tiles.h) where they can go wrong -- edges of tiles, stages
-and blocks, padded head dimensions, key prefixes, groups of heads, rows that start on odd addresses, coefficients either
-side of the shifted-square form -- against the fp64 closed form.  Tolerance: bf16 rounds weights and outputs by at most 2^-9
+and blocks, padded head dimensions, key prefixes, groups of heads, rows that start on odd addresses, coefficients small and
+large against each other -- against the fp64 closed form.  Tolerance: bf16 rounds weights and outputs by at most 2^-9
 each (3.9e-3 together); measured 2e-3 to 4e-3 normwise.  The largest difference is measured against the largest value, where
 the first rows' sums of few terms round by up to 1e-2: the package's 2e-2 for bf16 inputs holds for both."""
 import ctypes as C
