@@ -156,7 +156,8 @@ bool use_linear_scan(const fastmax_desc* ds, const Plan& pl);
 // Dense score tiles cost 2 n d flop per token under the mask (4 n d without it), the moment form about
 // 2.1 d^3 (p = 2) whatever n is: below these key counts the dense kernels are the faster ones (measured,
 // forward + backward, 96 and 768 heads; with few heads the sequential state build of the moment form
-// fills the chip badly and the dense kernels stay ahead for longer).  A causal sequence of a single chunk
+// fills the chip badly and the dense kernels stay ahead for longer.  bf16: measured with fm_dense.h; fm_tiles.h is 1.2 to 1.8
+// times as fast, so that its crossovers, not measured, lie higher).  A causal sequence of a single chunk
 // has no states to build either way and stays with the moment kernels' own intra-chunk tiles.  Head
 // dimensions without moment kernels always take the dense ones (p = 1 at d = 32 / 64: see below).
 bool use_dense(const fastmax_desc* ds, bool plain = true) {
