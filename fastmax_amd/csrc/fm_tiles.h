@@ -61,9 +61,13 @@ __device__ __forceinline__ int fresh_lane() {
   return l;
 }
 
+// what rows that do not exist are copied from
+static __device__ const uint4 zero_chunk = {0u, 0u, 0u, 0u};
+
 // One streamed tensor's share of a stage for this wave: chunk (u NW + wave) 64 + lane of the tile, u = 0..NI-1.
-// Rows outside [lo, end) are fetched from the nearest row inside and channels past d from the row's last chunk:
-// valid addresses whose products the kernels' masks, zero operands and stores leave out.
+// Rows outside [lo, end) and channels past d are zeros.  (Copies of the nearest row or chunk would do for finite values, which the
+// kernels' masks and zero operands leave out; but an infinity times zero is a NaN.)  Chunks past d are cleared once, and their lanes
+// move nothing; a lane's place in LDS does not depend on the others'.
 template <int DP, int NW, bool LEAN = false>
 struct Copy {
   using G = Geo<DP>;
@@ -72,13 +76,13 @@ struct Copy {
   static __device__ __forceinline__ bool has(int u, int w) { return EVEN || u * NW + w < ALL; }
   uint32_t off[NI];   // bytes from the tile's first row to this lane's chunk in instruction u
   static __device__ __forceinline__ int row(int u, int w, int l) { return ((u * NW + w) * 64 + l) / G::CPR; }
-  static __device__ __forceinline__ int channel(int u, int w, int l, int d) {
-    const int c = (((u * NW + w) * 64 + l) % G::CPR ^ G::key(row(u, w, l))) * 8;
-    return c < d ? c : d - 8;
+  static __device__ __forceinline__ int channel(int u, int w, int l) { return (((u * NW + w) * 64 + l) % G::CPR ^ G::key(row(u, w, l))) * 8; }
+  static __device__ __forceinline__ uint32_t offset(int u, int w, int l, unsigned pitch) {
+    return ((unsigned)row(u, w, l) * pitch + (unsigned)channel(u, w, l)) * 2u;
   }
-  __device__ __forceinline__ void init(int w, int l, int d, unsigned pitch) {
+  __device__ __forceinline__ void init(int w, int l, unsigned pitch) {
 #pragma unroll
-    for (int u = 0; u < NI; ++u) off[u] = ((unsigned)row(u, w, l) * pitch + (unsigned)channel(u, w, l, d)) * 2u;
+    for (int u = 0; u < NI; ++u) off[u] = offset(u, w, l, pitch);
   }
   static __device__ __forceinline__ void transfer(const void* base, uint32_t offset, uint32_t dst) {
     // (in asm: behind the builtin the compiler waits for the transfer at the next LDS read of any buffer.  The compiler does not
@@ -86,28 +90,38 @@ struct Copy {
     // a spilled one back from a lane does, to a memory instruction that reads it are kept here.)
     asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(dst), "v"(offset), "s"(base) : "memory");
   }
+  // this wave's chunks past d of the tile at `tile`
+  static __device__ __forceinline__ void clear(unsigned char* tile, int d, int w) {
+    const int l = fresh_lane();
+#pragma unroll
+    for (int u = 0; u < NI; ++u)
+      if (has(u, w) && channel(u, w, l) >= d) *reinterpret_cast<uint4*>(tile + ((u * NW + w) * 64 + l) * 16) = make_uint4(0u, 0u, 0u, 0u);
+  }
+  static __device__ __forceinline__ void transfer_from(uint64_t address, uint32_t dst) {   // (an address of its own for every lane)
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(dst), "v"(address) : "memory");
+  }
   // the stage's rows pos0 .. pos0 + BN - 1 to the tile at byte address lds
   __device__ __forceinline__ void issue(const HeadRows<const bf16_t>& hr, int pos0, int end, int d, uint32_t lds, int w, int l) const {
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds + (uint32_t)(w * 1024));
-    if (pos0 >= hr.lo && pos0 + G::BN <= end) {   // (uniform) nothing to clamp: the lane's offsets stand
-      const bf16_t* base = hr.base + (uint64_t)((unsigned)pos0 * hr.pitch);
+    uint64_t zeros = (uint64_t)reinterpret_cast<uintptr_t>(&zero_chunk);
+    const bool inside = pos0 >= hr.lo && pos0 + G::BN <= end;   // (uniform)
+    const bf16_t* base = hr.base + (int64_t)pos0 * hr.pitch;
+    if (inside) {
 #pragma unroll
       for (int u = 0; u < NI; ++u)
         if (has(u, w)) {
-          uint32_t o = off[u];
-          if constexpr (LEAN) {   // (no register to keep it in)
-            const int k = fresh_lane();
-            o = ((unsigned)row(u, w, k) * hr.pitch + (unsigned)channel(u, w, k, d)) * 2u;
-          }
-          transfer(base, o, dst + u * NW * 1024);
+          const int k = LEAN ? fresh_lane() : l;   // (LEAN: no registers to keep what follows in)
+          const uint32_t o = LEAN ? offset(u, w, k, hr.pitch) : off[u];
+          if (d == DP || channel(u, w, k) < d) transfer(base, o, dst + u * NW * 1024);
         }
     } else {
       l = fresh_lane();   // (rare: nothing of it is kept in registers)
+      asm volatile("" : "+s"(zeros));
 #pragma unroll
       for (int u = 0; u < NI; ++u) {
-        const int p = pos0 + row(u, w, l);
-        const int ps = max(p < end ? p : end - 1, hr.lo);
-        if (has(u, w)) transfer(hr.base, ((unsigned)ps * hr.pitch + (unsigned)channel(u, w, l, d)) * 2u, dst + u * NW * 1024);
+        const int p = pos0 + row(u, w, l), c = channel(u, w, l);
+        const uint64_t from = (uint64_t)reinterpret_cast<uintptr_t>(hr.base) + (uint64_t)(((unsigned)p * hr.pitch + (unsigned)c) * 2u);
+        if (has(u, w)) transfer_from(p >= hr.lo && p < end && c < d ? from : zeros, dst + u * NW * 1024);
       }
     }
   }
@@ -299,13 +313,16 @@ __global__ __launch_bounds__(256, OCC) void tiles_fwd_kernel(
   const uint32_t lds0 = lds_address(tiles_smem);
 
   C ck, cv;
-  ck.init(w, l, d, Kh.pitch);
-  cv.init(w, l, d, Vh.pitch);
+  ck.init(w, l, Kh.pitch);
+  cv.init(w, l, Vh.pitch);
   auto issue = [&](int st, int buf) {
     ck.issue(Kh, st * BN, nk, d, lds0 + buf * STAGE, w, l);
     cv.issue(Vh, st * BN, nk, d, lds0 + buf * STAGE + G::TILE, w, l);
   };
   issue(0, 0);
+  if (d < DP)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) C::clear(tiles_smem + t * G::TILE, d, w);
 
   const float kq = qscale[head] * kscale[hkv];
   Frag qf[NF];
@@ -459,13 +476,16 @@ __global__ __launch_bounds__(64 * NW, OCC) void tiles_dq_kernel(
   const uint32_t lds0 = lds_address(tiles_smem);
 
   C ck, cv;
-  ck.init(w, l, d, Kh.pitch);
-  cv.init(w, l, d, Vh.pitch);
+  ck.init(w, l, Kh.pitch);
+  cv.init(w, l, Vh.pitch);
   auto issue = [&](int st, int buf) {
     ck.issue(Kh, st * BN, nk, d, lds0 + buf * STAGE, w, l);
     cv.issue(Vh, st * BN, nk, d, lds0 + buf * STAGE + G::TILE, w, l);
   };
   issue(0, 0);
+  if (d < DP)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) C::clear(tiles_smem + t * G::TILE, d, w);
 
   const float kq = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, qscale[head] * kscale[hkv])));   // (uniform, in a scalar register)
   const int q0 = tok0 + w * 32;
@@ -707,7 +727,7 @@ __global__ __launch_bounds__(64 * DkDv<DP>::NW, 2) void tiles_dkdv_kernel(
   const int64_t qstep = Q.step(), gstep = GO.step();   // (the heads of a group are equally far apart)
   float lqs = qscale[hkv * ratio];
   C cq;
-  cq.init(w, l, d, Qh.pitch);
+  cq.init(w, l, Qh.pitch);
   Scaled<DP, NW> sg;
   float creg = 0.f;
   auto stage_load = [&](int st, int buf) __attribute__((always_inline)) {
@@ -736,6 +756,10 @@ __global__ __launch_bounds__(64 * DkDv<DP>::NW, 2) void tiles_dkdv_kernel(
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) acc[s][cb] = kZero16;
   if (st0 < nst) stage_load(st0, 0);
+  if (d < DP) {
+    C::clear(tiles_smem, d, w);
+    C::clear(tiles_smem + TILE, d, w);
+  }
   own_row<DP>(Vh, k00 + i, nk, d, hh, 1.0f, vf);
   __builtin_amdgcn_sched_barrier(0);   // (one row after the other: registers)
   own_row<DP>(Kh, k00 + i, nk, d, hh, ks, kf);

@@ -152,3 +152,39 @@ def test_small_constant_term(built, mask, a0, a1, a2, lim, d):
 def test_small_constant_term_and_small_rows(built, a0, scale, d):
     errors = normwise(2, 2, 512, 512, d, True, seed=3, scale=scale, normalize=False, a0=a0, a1=1.0, a2=1e-3)
     assert max(errors.values()) <= NORMWISE, errors
+
+
+@pytest.mark.parametrize("mask", [True, False])
+@pytest.mark.parametrize("d", [24, 64, 104, 128])
+def test_an_infinity_in_the_last_row_stays_one(built, d, mask):
+    """150 keys end within a stage: rows behind the last one count for nothing, also where the last one holds an infinity (times a
+    weight of zero, a copy of it would make a NaN of the infinite sum)."""
+    from fastmax_amd import ops
+
+    print("tiles infinity in v", d, mask, flush=True)
+    q, k, v, go = (t.cuda() for t in O.seeded_inputs((2, 150, d), seed=d, dtype=torch.bfloat16))
+    v[0, -1, d - 1] = float("inf")
+    o, den, *_ = ops.forward(q, k, v, mask=mask, normalize=True, p=2)
+    sees = o[0, -1:] if mask else o[0]
+    assert torch.all(sees[:, d - 1] == float("inf")) and torch.isfinite(sees[:, :d - 1]).all()
+    assert torch.isfinite(o[1]).all() and torch.isfinite(den).all()
+
+
+@pytest.mark.parametrize("mask", [True, False])
+@pytest.mark.parametrize("d", [24, 40, 104])
+def test_an_infinity_in_the_last_channel_stays_with_its_key(built, d, mask):
+    """Head dimensions that are padded to a multiple of 32: an infinite key has infinite scores, and its queries an infinite
+    denominator and no weight left for other keys, whose dv is finite."""
+    from fastmax_amd import ops
+
+    print("tiles infinity in k", d, mask, flush=True)
+    q, k, v, go = (t.cuda() for t in O.seeded_inputs((2, 150, d), seed=d, dtype=torch.bfloat16))
+    q, k = q * 0.2, k * 0.2
+    k[0, 70, d - 1] = float("inf")
+    kw = dict(mask=mask, normalize=False, p=2)
+    o, den, sc, arg = ops.forward(q, k, v, **kw)
+    first = 70 if mask else 0
+    assert torch.all(den[0, first:] == float("inf")) and torch.isfinite(den[0, :first]).all() and torch.isfinite(den[1]).all()
+    _, _, dv = ops.backward(q, k, v, o, den, go, qk_scale=sc, qk_argmax=arg, **kw)
+    others = [j for j in range(150) if j != 70]
+    assert torch.isfinite(dv[0, others]).all() and torch.isfinite(dv[1]).all()
