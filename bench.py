@@ -29,7 +29,7 @@ PEAK_TFLOPS = {"f32": 157.3, "bf16": 2500.0}
 PEAK_HBM_GBS = 8000.0
 
 WORKLOADS = {
-    # the shape the metric is quoted on (causal, p=2, fp32)
+    # the shape the metric is quoted on: causal, p=2, fp32, B 64, H 16, N 10000, D 64
     "headline": dict(B=64, H=16, N=10000, D=64, mask=True, p=2, dtype="f32"),
     "headline-unmasked": dict(B=64, H=16, N=10000, D=64, mask=False, p=2, dtype="f32"),
     "headline-p1": dict(B=64, H=16, N=10000, D=64, mask=True, p=1, dtype="f32"),

@@ -1,7 +1,7 @@
 """CPU oracle for Fastmax polynomial-kernel attention.  TEST INFRASTRUCTURE ONLY.
 
 Nothing in the shipped package imports this file: only tests/, the smoke check and
-the cpu_baseline leg of bench.py may use it, and only as the checker.
+the cpu_baseline leg of bench.py may use it, and only to compare against.
 
 It restates, in plain torch on the CPU, what the reference's pure-PyTorch path
 computes (reference: example.py:83-197, identical copies at model.py:78-205 and
